@@ -235,7 +235,6 @@ __global__ __launch_bounds__(kBinBlock) void accumulate_kernel(RankArgs A, Binne
   constexpr bool kDeadBit = B <= 8192;
   __shared__ double sum[B];
   __shared__ uint8_t ext[EXT ? B : 1];
-  __shared__ double lds_max[kBinWaves];
   __shared__ double lds_cost[2 * kBinWaves];
   const uint4 it = P.ac_item[blockIdx.x];  // bin, first slot, end slot, partial row (kWholeBin: none)
   for (uint32_t i = threadIdx.x; i < uint32_t(B); i += kBinBlock) {
@@ -313,8 +312,7 @@ __global__ __launch_bounds__(kBinBlock) void accumulate_kernel(RankArgs A, Binne
     for (uint32_t i = threadIdx.x; i < nb; i += kBinBlock) p[i] = EXT && ext[EXT ? i : 0] ? -sum[i] : sum[i];
   }
   wg_store_costs<VARIANT, kBinWaves>(A, cost, blockIdx.x, lds_cost);
-  emax = wg_max<kBinWaves>(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // Split bins, one workgroup per unit (bin, first partial row, rows, first vertex | mode << 31):
@@ -325,7 +323,6 @@ template <int VARIANT>
 __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, BinnedPlan P, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
   __shared__ double part[kBinWaves][kWave];
-  __shared__ double lds_max[kBinWaves];
   __shared__ double lds_cost[2 * kBinWaves];
   CostAcc cost;
   const uint4 m = P.multi[blockIdx.x];
@@ -379,8 +376,7 @@ __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, Binn
     }
   }
   wg_store_costs<VARIANT, kBinWaves>(A, cost, P.n_ac + blockIdx.x, lds_cost);
-  emax = wg_max<kBinWaves>(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // The overlay's values for this iteration: entry i takes its source's contribution, negated when the source was in

@@ -83,7 +83,7 @@ __device__ __forceinline__ void ppr_reduce_err(const PprArgs &A, int l, double e
   __syncthreads();
   if (threadIdx.x < kCols) {
     const double m = fmax(fmax(lds[j], lds[kCols + j]), fmax(lds[2 * kCols + j], lds[3 * kCols + j]));
-    if (j < A.k) atomic_max_nonneg(&A.err[size_t(l) * kCols + j], m);
+    if (j < A.k && m >= A.tol) A.err[size_t(l) * kCols + j] = kChanged;
   }
 }
 

@@ -1,4 +1,4 @@
-// rank.hip -- the pull-based, atomic-free rank update with the fused L-inf reduction, plus small map kernels.
+// rank.hip -- the pull-based, atomic-free rank update with the fused convergence test, plus small map kernels.
 //
 // Row plan (every variant). One launch per iteration covers all vertices of the degree-ordered layout (rows
 // sorted by in-degree, descending; layout.hip) through a table of sections, heaviest first so that long rows
@@ -16,8 +16,7 @@
 //                                            the same FP64 value the reference divides per edge
 //   a[v] = C0 + P*cv                      -- or the DF-P closed form (C0 + P*(cv - r[v]/d))/(1 - P/d)
 //   prune / frontier flags                 -- vaff[v] = 0 if |a-r|/max(r,a) <= C; naff[v] = (|a-r|/max > D)
-// Each vertex has exactly one writer, so the update needs no atomics on ranks; the only atomic is one 64-bit max
-// per workgroup for the L-inf change. Every sum is taken in a fixed order, so results repeat bit for bit.
+// Each vertex has exactly one writer, so the update needs no atomics. Every sum is taken in a fixed order, so results repeat bit for bit.
 #include <algorithm>
 #include <type_traits>
 
@@ -179,7 +178,6 @@ template <int VARIANT>
 __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPlan P, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
   __shared__ double lds_sum[kWavesPerBlock];
-  __shared__ double lds_max[kWavesPerBlock];
   int s = 0;
   while (s + 1 < P.nsec && blockIdx.x >= P.sec[s + 1].block_begin) ++s;
   const RankSection &S = P.sec[s];
@@ -202,8 +200,7 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
   }
   __shared__ double lds_cost[2 * kWavesPerBlock];
   store_costs<VARIANT>(A, cost, blockIdx.x, lds_cost);
-  emax = block_max(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // Chunked rows, after the rank kernel of the same iteration: one wave per row adds the row's chunk partials (in a
@@ -211,7 +208,6 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
 template <int VARIANT>
 __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, RankPlan P, uint32_t n_rows, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;  // same outcome as the rank kernel's entry test of this iteration
-  __shared__ double lds_max[kWavesPerBlock];
   __shared__ double lds_cost[2 * kWavesPerBlock];
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   double emax = 0.0;
@@ -236,8 +232,7 @@ __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, Rank
     }
   }
   store_costs<VARIANT>(A, cost, P.blocks + blockIdx.x, lds_cost);
-  emax = block_max(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 template <int VARIANT>
@@ -313,7 +308,6 @@ template <int S>
 __global__ __launch_bounds__(kBlock) void sliced_finish_kernel(RankArgs A, SlicedPlan P, uint32_t huge_blocks,
                                                                LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
-  __shared__ double lds_max[kWavesPerBlock];
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   double emax = 0.0;
   if (blockIdx.x < huge_blocks) {
@@ -358,8 +352,7 @@ __global__ __launch_bounds__(kBlock) void sliced_finish_kernel(RankArgs A, Slice
       if (valid) emax = fmax(emax, finish_vertex<kPlain>(A, v, cv, d, rv, 0.0));
     }
   }
-  emax = block_max(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // r = a = 1/N (or keep r as loaded and copy it to a); contributions cr = ca = r/deg.

@@ -95,19 +95,6 @@ __device__ __forceinline__ void wg_store_costs(const RankArgs &A, const CostAcc 
   }
 }
 
-// Workgroup-wide max over WAVES waves, valid in thread 0. Every thread must call it.
-template <int WAVES>
-__device__ __forceinline__ double wg_max(double x, double *lds) {
-  x = group_max<kWave>(x);
-  const int w = threadIdx.x / kWave;
-  if ((threadIdx.x & (kWave - 1)) == 0) lds[w] = x;
-  __syncthreads();
-  double m = 0.0;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < WAVES; ++i) m = fmax(m, lds[i]);
-  return m;
-}
-
 template <int VARIANT>
 __device__ __forceinline__ double finish_vertex(const RankArgs &A, uint32_t v, double cv) {
   return finish_vertex<VARIANT>(A, v, cv, A.deg[v], A.r[v], Traits<VARIANT>::prune ? A.cr[v] : 0.0);

@@ -103,15 +103,13 @@ __global__ __launch_bounds__(kBlock) void weighted_step_kernel(WeightedArgs A, u
       default: band_rows<ADJOINT, 1>(A, rb, re, emax); break;
     }
   }
-  emax = block_max(emax, lds);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // Heavy rows, after the step of the same iteration: a wave per row adds its chunk sums in chunk order.
 template <bool ADJOINT>
 __global__ __launch_bounds__(kBlock) void weighted_heavy_kernel(WeightedArgs A, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
-  __shared__ double lds[kWavesPerBlock];
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   const uint32_t *order = A.sched.order + A.sched.n_low + A.sched.n_high;
   double emax = 0.0;
@@ -121,8 +119,7 @@ __global__ __launch_bounds__(kBlock) void weighted_heavy_kernel(WeightedArgs A, 
     s = group_sum<kWave>(s);
     if (lane == 0) emax = fmax(emax, wfinish<ADJOINT>(A, order[h], s));
   }
-  emax = block_max(emax, lds);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 // W_u = sum of u's out-weights (FP64), one wave per row.

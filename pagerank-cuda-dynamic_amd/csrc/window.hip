@@ -68,7 +68,6 @@ __global__ __launch_bounds__(kBinBlock) void window_update_kernel(RankArgs A, Wi
   static_assert(S >= int(kWinRows) + 2, "ring smaller than a chunk");
   constexpr uint32_t R = kWinRows;
   __shared__ double ring[S];
-  __shared__ double lds_max[kWinWaves];
   __shared__ double lds_cost[2 * kWinWaves];
   const uint32_t N = W.N, H = W.H, t = threadIdx.x;
   const uint32_t a = uint32_t(uint64_t(blockIdx.x) * N / gridDim.x);
@@ -144,8 +143,7 @@ __global__ __launch_bounds__(kBinBlock) void window_update_kernel(RankArgs A, Wi
     }
   }
   wg_store_costs<VARIANT, kWinWaves>(A, cost, blockIdx.x, lds_cost);
-  emax = wg_max<kWinWaves>(emax, lds_max);
-  if (threadIdx.x == 0) atomic_max_nonneg(&ctl.err[iter_index(ctl)], emax);
+  report_change(ctl, emax);
 }
 
 template <int S>
