@@ -80,7 +80,8 @@ typedef struct prh_stats {
 /* Launch tuning (no counterpart in the reference, whose values are fixed: switch degree 64, 256-thread blocks).
  * Results do not depend on these beyond floating-point summation order. */
 typedef struct prh_tuning {
-  uint32_t switch_degree; /* in-degree <= this: several vertices per wave; above: one wave per vertex [64] */
+  uint32_t switch_degree; /* in-degree <= this: several vertices per wave; above: one wave (long rows: one workgroup)
+                             per vertex [64] */
   uint32_t huge_degree;   /* in-degree > this: split into chunks of this many edges, one workgroup per chunk,
                              summed by a second launch [16384] */
   int low_width;          /* lanes per vertex of in-degree <= switch_degree: 1, 2, 4, 8, 16 or 32; 0 = by degree
@@ -89,7 +90,7 @@ typedef struct prh_tuning {
   int source_slices;      /* Static / Naive-dynamic: 0 = row kernel; 1, 2, 4 or 8 = sum each row slice by slice,
                              source u in slice (u / 16) mod source_slices, slice x on the workgroups b with
                              b mod source_slices = x (8: one slice per XCD and its L2) [0] */
-  uint32_t block_edges;   /* edges per workgroup of the rank kernels (>= 256) [2048] */
+  uint32_t block_edges;   /* edges per workgroup of the rank kernels, fewer on small graphs (>= 256) [2048] */
   int extension_direction; /* DF / DF-P extension: 0 push along out-edges of frontier vertices; 1 push or pull
                               (unaffected rows look for a frontier in-neighbour), whichever the last rank launch
                               found cheaper; 2 pull. The flags, hence the results, are the same for all [1] */

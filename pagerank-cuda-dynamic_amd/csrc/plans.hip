@@ -479,7 +479,7 @@ int build_binned_plan_t(prh_context *c, prh_graph *g) {
 
 // Rank-kernel plan over the degree-ordered layout for the context's tuning (cached in the graph):
 //   rows with in-degree > huge_degree: chunks of huge_degree edges, one workgroup each;
-//   switch_degree < in-degree <= huge_degree: one wave per row;
+//   switch_degree < in-degree <= huge_degree: one wave per row, or one workgroup (kBlockRowDegree);
 //   in-degree <= switch_degree: bands of equal lanes-per-row W, W = pow2ceil(d)/2 in 1..32 (or the fixed
 //   low_width), each band a contiguous row range.
 int build_rank_plan(prh_context *c, prh_graph *g) {
@@ -489,7 +489,11 @@ int build_rank_plan(prh_context *c, prh_graph *g) {
   PrepTimer timer(g->plan_prep);
   const uint32_t N = g->N;
   const std::vector<uint32_t> &deg = g->sorted_deg;
-  const uint64_t kEdgesPerBlock = t.block_edges;
+  // Edges per workgroup: block_edges, and on graphs of fewer than 8192 such workgroups (the chip holds 2048 at a time)
+  // as many fewer as it takes to have 8192: a workgroup goes through its rows in rounds of dependent loads, and with few
+  // workgroups the rounds are the launch's time (300K vertices, 6M edges: 2.93 ms per solve at 2048 edges each, 2.27
+  // at 730).
+  const uint64_t kEdgesPerBlock = std::min<uint64_t>(t.block_edges, std::max<uint64_t>(256, g->M / 8192));
   PRH_HIP(c, hipStreamSynchronize(c->stream));  // the old tables may still be in use
   auto above = [&](uint32_t x) { return layout_rows_above(g, x); };
   auto edges = [&](uint32_t b, uint32_t e) {
@@ -546,8 +550,9 @@ int build_rank_plan(prh_context *c, prh_graph *g) {
   p.partial = g->chunk_partial;
   p.n_chunked = n_chunked;
   add(prh::kChunkedRows, 0, 0, n_items, 1, n_items);
-  // Wave rows.
+  // Block rows, then wave rows.
   const uint32_t w_end = above(t.switch_degree);
+  const uint32_t b_end = std::min(w_end, std::max(n_chunked, above(uint32_t(std::max<uint64_t>(prh::kBlockRowDegree, g->M / 4096)))));
   auto row_section = [&](int kind, int width, uint32_t b, uint32_t e) {
     if (e <= b) return;
     const uint32_t unit = kind == prh::kWaveRows ? prh::kWavesPerBlock : prh::kWavesPerBlock * (prh::kWave / width);
@@ -556,7 +561,8 @@ int build_rank_plan(prh_context *c, prh_graph *g) {
     per = std::max<uint64_t>(unit, (per + unit - 1) / unit * unit);
     add(kind, width, b, e, uint32_t(per), uint32_t((uint64_t(e - b) + per - 1) / per));
   };
-  row_section(prh::kWaveRows, 64, n_chunked, std::max(n_chunked, w_end));
+  if (b_end > n_chunked) add(prh::kBlockRows, 0, n_chunked, b_end, 1, b_end - n_chunked);
+  row_section(prh::kWaveRows, 64, std::max(n_chunked, b_end), std::max(n_chunked, w_end));
   // Group-row bands.
   const uint32_t lb = std::max(n_chunked, w_end);
   if (t.low_width) {

@@ -43,17 +43,26 @@ enum SectionKind : int {
   kGroupRows = 0,    // `width` lanes per row (1..32), rows split into contiguous per-block ranges
   kWaveRows = 1,     // one wave per row
   kChunkedRows = 2,  // one workgroup per fixed-size edge chunk of a row; a second launch finishes the rows
+  kBlockRows = 3,    // one workgroup per row
 };
+
+// In-degree above which a row takes a workgroup of the rank kernel instead of a wave: this, or 1/4096 of the edges on
+// larger graphs. A wave's row of d edges is a chain of d / 512 batches, and the launch cannot end before it; a launch
+// of M edges lasts about as long as a chain of M / 300K batches, so longer rows than M / 600 would set its time, and a
+// workgroup costs more than a wave per row. Measured per solve, one row class per in-degree above 64 -> with this
+// rule: RMAT-16 1038 -> 814 us, 300K vertices (6M edges) 3357 -> 2286 us, 1M (17M) 11.8 -> 6.64 ms, 3M (51M) 16.83
+// -> 16.82 ms; a fixed 1024 takes 17.6 ms at 3M and 6.86 ms at 1M, and 256 takes 3.75 ms at 300K.
+constexpr uint32_t kBlockRowDegree = 1024;
 
 struct RankSection {
   int kind;
   int width;                 // lanes per row for kGroupRows
-  uint32_t begin, end;       // rows (kGroupRows, kWaveRows) or items (kChunkedRows)
+  uint32_t begin, end;       // rows (kGroupRows, kWaveRows, kBlockRows) or items (kChunkedRows)
   uint32_t block_begin;      // first block of the section
   uint32_t per_block;        // rows or items per block
 };
 
-constexpr int kMaxSections = 8;
+constexpr int kMaxSections = 9;  // chunked, block and wave rows, six bands of group rows
 
 struct RankPlan {
   RankSection sec[kMaxSections];

@@ -5,6 +5,7 @@
 // start early:
 //   chunked rows  (in-degree above the chunk threshold): one workgroup per fixed-size edge chunk, each writing its
 //                 partial sum; finish_chunked_kernel (the next launch) adds a row's partials in chunk order;
+//   block rows    one workgroup per row;
 //   wave rows     one wave per row, DPP/swizzle wave sum;
 //   group rows    W lanes per row (W = 1..32), one band per W over a contiguous row range, DPP group sum.
 //
@@ -72,32 +73,80 @@ __device__ __forceinline__ void store_costs(const RankArgs &A, CostAcc c, uint32
   }
 }
 
-// Sum of cr[src[e]] for e = first, first + STEP, ... < end, four gathers in flight per lane.
-template <int STEP>
-__device__ __forceinline__ double gather_sum(const uint32_t *src, const double *cr, uint32_t e, uint32_t end) {
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  for (; e + 3 * STEP < end; e += 4 * STEP) {
-    const uint32_t u0 = stream_u32(src + e), u1 = stream_u32(src + e + STEP);
-    const uint32_t u2 = stream_u32(src + e + 2 * STEP), u3 = stream_u32(src + e + 3 * STEP);
-    s0 += cr[u0];
-    s1 += cr[u1];
-    s2 += cr[u2];
-    s3 += cr[u3];
-  }
-  for (; e < end; e += STEP) s0 += cr[stream_u32(src + e)];
-  return (s0 + s1) + (s2 + s3);
+// On graphs whose contributions fit the L2s a launch is bound by its longest chain of dependent loads, not by bytes
+// (RMAT-16: 29 us per iteration for 1 M gathers that the L2s serve in 5). One batch of U strided edges e, e + STEP,
+// ...: all U source ids are loaded before the first gather and all gathers are in flight together, so a batch costs
+// two round trips whatever U is. Only the last edge may lie past `end`
+// (a lane without it sits these two loads out: repeating a load instead costs the address unit as much as a new one).
+template <int STEP, int U>
+__device__ __forceinline__ void gather_batch(const uint32_t *src, const double *cr, uint32_t e, uint32_t end,
+                                             double (&s)[4]) {
+  const bool last = e + (U - 1) * STEP < end;
+  uint32_t u[U];
+  double x[U];
+#pragma unroll
+  for (int k = 0; k + 1 < U; ++k) u[k] = stream_u32(src + e + k * STEP);
+  u[U - 1] = last ? stream_u32(src + e + (U - 1) * STEP) : 0u;
+#pragma unroll
+  for (int k = 0; k + 1 < U; ++k) x[k] = cr[u[k]];
+  x[U - 1] = last ? cr[u[U - 1]] : 0.0;
+#pragma unroll
+  for (int k = 0; k < U; ++k) s[k & 3] += x[k];
 }
 
+// Sum of cr[src[e]] for e = b + i, b + i + STEP, ... < end, where i < STEP is the thread's place among the STEP threads
+// of the row (a wave or a workgroup) and b, end are the same for all of them: batches of eight gathers a thread, the
+// last batch of exactly as many as are left.
 template <int STEP>
-__device__ __forceinline__ double gather_sum(const RankArgs &A, uint32_t e, uint32_t end) {
-  return gather_sum<STEP>(A.src, A.cr, e, end);
+__device__ __forceinline__ double gather_sum(const uint32_t *src, const double *cr, uint32_t b, uint32_t end,
+                                             uint32_t i) {
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  uint32_t n = __builtin_amdgcn_readfirstlane((end - b + STEP - 1) / STEP);
+  uint32_t e = b + i;
+  for (; n > 8; n -= 8, e += 8 * STEP) gather_batch<STEP, 8>(src, cr, e, end, s);
+  // A thread of the last batch may have no edge in a one-edge batch; in longer ones its first edge always exists.
+  switch (n) {
+    case 1:
+      if (e < end) s[0] += cr[stream_u32(src + e)];
+      break;
+    case 2: gather_batch<STEP, 2>(src, cr, e, end, s); break;
+    case 3: gather_batch<STEP, 3>(src, cr, e, end, s); break;
+    case 4: gather_batch<STEP, 4>(src, cr, e, end, s); break;
+    case 5: gather_batch<STEP, 5>(src, cr, e, end, s); break;
+    case 6: gather_batch<STEP, 6>(src, cr, e, end, s); break;
+    case 7: gather_batch<STEP, 7>(src, cr, e, end, s); break;
+    case 8: gather_batch<STEP, 8>(src, cr, e, end, s); break;
+    default: break;
+  }
+  return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// The same for a group of W lanes, whose rows differ within the wave: lane j takes edges b + j, b + j + W, ... A band's
+// rows have W < in-degree <= 2 W, so the first two edges go together (two round trips; one by one they took four), and
+// what rows of other degrees have left goes by fours.
+template <int W>
+__device__ __forceinline__ double group_gather_sum(const uint32_t *src, const double *cr, uint32_t e, uint32_t end) {
+  if (e >= end) return 0.0;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  gather_batch<W, 2>(src, cr, e, end, s);
+  for (e += 2 * W; e < end; e += 4 * W) {
+    uint32_t u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = stream_u32(src + (e + k * W < end ? e + k * W : e));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double x = cr[u[k]];
+      s[k] += e + k * W < end ? x : 0.0;
+    }
+  }
+  return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 // Sum of a workgroup-strided gather, valid in thread 0. Every thread must call it.
 __device__ __forceinline__ double block_gather_sum(const uint32_t *src, const double *cr, uint32_t b, uint32_t e,
                                                    double *lds) {
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  double acc = group_sum<kWave>(gather_sum<kBlock>(src, cr, b + threadIdx.x, e));
+  const double acc = group_sum<kWave>(gather_sum<kBlock>(src, cr, b, e, threadIdx.x));
   if (lane == 0) lds[w] = acc;
   __syncthreads();
   const double t = (lds[0] + lds[1]) + (lds[2] + lds[3]);
@@ -119,6 +168,27 @@ __device__ __forceinline__ void chunked_rows(const RankArgs &A, const RankPlan &
   }
 }
 
+// One workgroup per row of `per_block` rows: the rows too long for one wave's chain of batches (kBlockRowDegree).
+template <int VARIANT>
+__device__ __forceinline__ void block_rows(const RankArgs &A, const RankSection &S, uint32_t blk, double *lds,
+                                           double &emax, CostAcc &cost) {
+  const uint32_t rb = S.begin + blk * S.per_block, re = min(S.end, rb + S.per_block);
+  for (uint32_t v = rb; v < re; ++v) {  // block-uniform
+    const RowOperands o = row_operands<VARIANT>(A, v);
+    RowFlags f;
+    const double t = o.upd ? block_gather_sum(A.src, A.cr, o.b, o.e, lds) : 0.0;
+    if (threadIdx.x == 0) {
+      if (o.upd) {
+        emax = fmax(emax, finish_vertex<VARIANT>(A, v, t, o.d, o.rv, o.crv, f));
+      } else {
+        copy_vertex<VARIANT>(A, v, o.rv, o.crv);
+        f.affected = false;
+      }
+      cost.add(f, o.e - o.b, o.d);
+    }
+  }
+}
+
 template <int VARIANT>
 __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &S, uint32_t blk, double &emax,
                                           CostAcc &cost) {
@@ -135,8 +205,7 @@ __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &
       }
       continue;
     }
-    double acc = gather_sum<kWave>(A, o.b + lane, o.e);
-    acc = group_sum<kWave>(acc);
+    const double acc = group_sum<kWave>(gather_sum<kWave>(A.src, A.cr, o.b, o.e, lane));
     if (lane == 0) {
       emax = fmax(emax, finish_vertex<VARIANT>(A, v, acc, o.d, o.rv, o.crv, f));
       cost.add(f, o.e - o.b, o.d);
@@ -158,7 +227,7 @@ __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection 
     double acc = 0.0;
     if (valid) {
       o = row_operands<VARIANT>(A, v);
-      if (o.upd) acc = gather_sum<W>(A, o.b + j, o.e);
+      if (o.upd) acc = group_gather_sum<W>(A.src, A.cr, o.b + j, o.e);
     }
     acc = group_sum<W>(acc);  // all lanes active again here
     if (valid && j == 0) {
@@ -186,6 +255,8 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
   CostAcc cost;
   if (S.kind == kChunkedRows) {
     chunked_rows<VARIANT>(A, P, S, blk, lds_sum);
+  } else if (S.kind == kBlockRows) {
+    block_rows<VARIANT>(A, S, blk, lds_sum, emax, cost);
   } else if (S.kind == kWaveRows) {
     wave_rows<VARIANT>(A, S, blk, emax, cost);
   } else {
@@ -273,7 +344,7 @@ __global__ __launch_bounds__(kBlock) void sliced_gather_kernel(SlicedPlan P, con
   } else if (S.kind == kWaveRows) {
     for (uint32_t k = ib + w; k < ie; k += kWavesPerBlock) {  // wave-uniform
       const double t = group_sum<kWave>(
-          gather_sum<kWave>(P.src, cr, stream_u32(P.item_off + k) + lane, stream_u32(P.item_off + k + 1)));
+          gather_sum<kWave>(P.src, cr, stream_u32(P.item_off + k), stream_u32(P.item_off + k + 1), lane));
       if (lane == 0) P.partial[k] = t;
     }
   } else {
@@ -283,7 +354,7 @@ __global__ __launch_bounds__(kBlock) void sliced_gather_kernel(SlicedPlan P, con
       for (uint32_t k0 = ib + w * G; k0 < ie; k0 += kWavesPerBlock * G) {  // wave-uniform
         const uint32_t k = k0 + g;
         double acc = 0.0;
-        if (k < ie) acc = gather_sum<W>(P.src, cr, stream_u32(P.item_off + k) + q, stream_u32(P.item_off + k + 1));
+        if (k < ie) acc = group_gather_sum<W>(P.src, cr, stream_u32(P.item_off + k) + q, stream_u32(P.item_off + k + 1));
         acc = group_sum<W>(acc);
         if (k < ie && q == 0) P.partial[k] = acc;
       }
