@@ -189,7 +189,6 @@ void prh_context_destroy(prh_context *c) {
   release(c, c->loop);
   release(c, c->flags);
   for (int i = 0; i < 2; ++i) {
-    release(c, c->ppr_rank[i]);
     release(c, c->ppr_contrib[i]);
   }
   release(c, c->ppr_partial);

@@ -83,7 +83,7 @@ struct prh_context {
   prhc::DevBuf<uint8_t> arena;
   size_t arena_top = 0, arena_want = 0;
   // batched personalized PageRank
-  prhc::DevBuf<double> ppr_rank[2], ppr_contrib[2], ppr_partial, ppr_mass, ppr_out;
+  prhc::DevBuf<double> ppr_contrib[2], ppr_partial, ppr_mass, ppr_out;
   prhc::DevBuf<int32_t> ppr_row;
   prhc::DevBuf<uint32_t> ppr_tables;
   prhc::DevBuf<unsigned long long> ppr_err;

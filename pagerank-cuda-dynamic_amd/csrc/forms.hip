@@ -16,9 +16,6 @@
 namespace prhc {
 namespace {
 
-// Edge chunk of a heavy vertex for the batched solver.
-constexpr uint32_t kPprChunk = 1024;
-
 int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, const uint32_t *seeds,
              const prh_options *o, double *ranks, int *iterations, prh_stats *st) {
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
@@ -31,111 +28,101 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
     return fail(c, PRH_ERROR_INVALID_ARGUMENT, "bad options");
   const uint32_t N = g->N;
   const int L = o->max_iterations;
-  // Seed table: one row per distinct seed vertex, s_j[v] = (occurrences of v in seed set j) / |seed set j|.
-  std::vector<int32_t> row(N, -1);
-  std::vector<double> mass;
-  int32_t rows = 0;
   for (int j = 0; j < k; ++j) {
     if (so[j + 1] <= so[j]) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "seed set %d is empty", j);
-    const double share = 1.0 / double(so[j + 1] - so[j]);
-    for (uint32_t i = so[j]; i < so[j + 1]; ++i) {
-      const uint32_t v = seeds[i];
-      if (v >= N) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "seed %u >= N", v);
-      if (row[v] < 0) {
-        row[v] = rows++;
-        mass.resize(size_t(rows) * prh::kPprCols, 0.0);
-      }
-      mass[size_t(row[v]) * prh::kPprCols + j] += share;
-    }
+    for (uint32_t i = so[j]; i < so[j + 1]; ++i)
+      if (seeds[i] >= N) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "seed %u >= N", seeds[i]);
   }
+  const uint32_t n_seeds = so[k] - so[0];
+  std::vector<uint32_t> first(size_t(k) + 1);
+  for (int j = 0; j <= k; ++j) first[j] = so[j] - so[0];
   hipStream_t s = c->stream;
   PRH_HIP(c, hipSetDevice(c->device));
-  // Light / heavy split of the in-degree at the chunk size, and the heavy chunks (built on the host: few).
+  const int tile = prh::ppr_tile(k), cols = (k + tile - 1) / tile * tile;
+  // Rows by in-degree, and the heavy rows' chunks (built on the host: few).
+  const uint32_t chunk_edges = prh::ppr_chunk(tile);
   const uint32_t nt = prh::partition_tiles(N);
   PRH_CHECK(ensure(c, c->sched_in, N));
   PRH_CHECK(ensure(c, c->tiles, size_t(3) * nt));
   PRH_CHECK(ensure(c, c->counts, 8));
-  PRH_HIP(c, prh::launch_partition(g->in_off, N, kPprChunk, 0xFFFFFFFFu, c->sched_in.p, c->tiles.p, c->counts.p, s));
-  PRH_HIP(c, hipMemcpyAsync(c->pinned, c->counts.p, 8, hipMemcpyDeviceToHost, s));
+  PRH_HIP(c, prh::launch_partition(g->l_in_off, N, prh::kPprGroup, chunk_edges, c->sched_in.p, c->tiles.p, c->counts.p,
+                                   s));
+  PRH_HIP(c, hipMemcpyAsync(c->pinned, c->counts.p, 12, hipMemcpyDeviceToHost, s));
   PRH_HIP(c, hipStreamSynchronize(s));
-  const uint32_t n_light = reinterpret_cast<uint32_t *>(c->pinned)[0];
-  const uint32_t n_heavy = reinterpret_cast<uint32_t *>(c->pinned)[1];
-  std::vector<uint32_t> hv(n_heavy), hb(n_heavy), he(n_heavy);
+  const uint32_t n_low = reinterpret_cast<uint32_t *>(c->pinned)[0];
+  const uint32_t n_high = reinterpret_cast<uint32_t *>(c->pinned)[1];
+  const uint32_t n_heavy = reinterpret_cast<uint32_t *>(c->pinned)[2];
+  std::vector<uint32_t> range(size_t(2) * n_heavy);
   PRH_CHECK(ensure(c, c->scratch_u32, size_t(2) * n_heavy + 1));
   if (n_heavy) {
-    PRH_HIP(c, prh::launch_gather_ranges(g->in_off, c->sched_in.p + n_light, n_heavy, c->scratch_u32.p,
+    PRH_HIP(c, prh::launch_gather_ranges(g->l_in_off, c->sched_in.p + n_low + n_high, n_heavy, c->scratch_u32.p,
                                          c->scratch_u32.p + n_heavy, s));
-    PRH_HIP(c, hipMemcpyAsync(hv.data(), c->sched_in.p + n_light, size_t(n_heavy) * 4, hipMemcpyDeviceToHost, s));
-    PRH_HIP(c, hipMemcpyAsync(hb.data(), c->scratch_u32.p, size_t(n_heavy) * 4, hipMemcpyDeviceToHost, s));
-    PRH_HIP(c, hipMemcpyAsync(he.data(), c->scratch_u32.p + n_heavy, size_t(n_heavy) * 4, hipMemcpyDeviceToHost, s));
+    PRH_HIP(c, hipMemcpyAsync(range.data(), c->scratch_u32.p, range.size() * 4, hipMemcpyDeviceToHost, s));
     PRH_HIP(c, hipStreamSynchronize(s));
   }
   std::vector<uint32_t> cb, ce, hf(size_t(n_heavy) + 1);
   for (uint32_t h = 0; h < n_heavy; ++h) {
     hf[h] = uint32_t(cb.size());
-    for (uint32_t e = hb[h]; e < he[h]; e += kPprChunk) {
-      cb.push_back(e);
-      ce.push_back(std::min(he[h], e + kPprChunk));
+    const uint64_t end = range[n_heavy + h];
+    for (uint64_t e = range[h]; e < end; e += chunk_edges) {
+      cb.push_back(uint32_t(e));
+      ce.push_back(uint32_t(std::min<uint64_t>(end, e + chunk_edges)));
     }
   }
   hf[n_heavy] = uint32_t(cb.size());
   const uint32_t n_chunks = uint32_t(cb.size());
   // Device buffers.
-  const size_t NC = size_t(N) * prh::kPprCols;
-  for (int i = 0; i < 2; ++i) {
-    PRH_CHECK(ensure(c, c->ppr_rank[i], NC));
-    PRH_CHECK(ensure(c, c->ppr_contrib[i], NC));
-  }
+  for (int i = 0; i < 2; ++i) PRH_CHECK(ensure(c, c->ppr_contrib[i], size_t(N) * cols));
   PRH_CHECK(ensure(c, c->ppr_out, size_t(N) * k));
-  PRH_CHECK(ensure(c, c->ppr_partial, std::max<size_t>(1, size_t(n_chunks) * prh::kPprCols)));
-  PRH_CHECK(ensure(c, c->ppr_mass, std::max<size_t>(1, mass.size())));
+  PRH_CHECK(ensure(c, c->ppr_partial, std::max<size_t>(1, size_t(n_chunks) * cols)));
+  PRH_CHECK(ensure(c, c->ppr_mass, size_t(std::min(n_seeds, N)) * cols));
   PRH_CHECK(ensure(c, c->ppr_row, N));
-  PRH_CHECK(ensure(c, c->ppr_tables, size_t(2) * n_chunks + size_t(2) * n_heavy + 1));
+  PRH_CHECK(ensure(c, c->ppr_tables, size_t(2) * n_chunks + n_heavy + 1 + n_seeds + k + 1));
   PRH_CHECK(ensure(c, c->ppr_err, std::max<size_t>(1, size_t(L) * prh::kPprCols)));
   PRH_CHECK(ensure(c, c->ppr_state, 1));
   uint32_t *t = c->ppr_tables.p;
-  PRH_HIP(c, hipMemcpyAsync(c->ppr_row.p, row.data(), size_t(N) * 4, hipMemcpyHostToDevice, s));
-  if (!mass.empty()) PRH_HIP(c, hipMemcpyAsync(c->ppr_mass.p, mass.data(), mass.size() * 8, hipMemcpyHostToDevice, s));
+  uint32_t *d_seeds = t + 2 * size_t(n_chunks) + n_heavy + 1, *d_first = d_seeds + n_seeds;
+  PRH_HIP(c, hipMemcpyAsync(d_seeds, seeds + so[0], size_t(n_seeds) * 4, hipMemcpyHostToDevice, s));
+  PRH_HIP(c, hipMemcpyAsync(d_first, first.data(), first.size() * 4, hipMemcpyHostToDevice, s));
   if (n_chunks) {
     PRH_HIP(c, hipMemcpyAsync(t, cb.data(), size_t(n_chunks) * 4, hipMemcpyHostToDevice, s));
     PRH_HIP(c, hipMemcpyAsync(t + n_chunks, ce.data(), size_t(n_chunks) * 4, hipMemcpyHostToDevice, s));
   }
-  if (n_heavy) PRH_HIP(c, hipMemcpyAsync(t + 2 * n_chunks, hv.data(), size_t(n_heavy) * 4, hipMemcpyHostToDevice, s));
-  PRH_HIP(c, hipMemcpyAsync(t + 2 * n_chunks + n_heavy, hf.data(), (size_t(n_heavy) + 1) * 4, hipMemcpyHostToDevice, s));
+  PRH_HIP(c, hipMemcpyAsync(t + 2 * n_chunks, hf.data(), (size_t(n_heavy) + 1) * 4, hipMemcpyHostToDevice, s));
   prh::PprArgs A{};
-  for (int i = 0; i < 2; ++i) {
-    A.rank[i] = c->ppr_rank[i].p;
-    A.contrib[i] = c->ppr_contrib[i].p;
-  }
-  A.off = g->in_off;
-  A.src = g->in_src;
-  A.deg = g->outdeg;
+  for (int i = 0; i < 2; ++i) A.contrib[i] = c->ppr_contrib[i].p;
+  A.off = g->l_in_off;
+  A.src = g->l_in_src;
+  A.deg = g->l_outdeg;
+  A.perm = g->perm;
   A.seed_row = c->ppr_row.p;
   A.seed_mass = c->ppr_mass.p;
-  A.light = c->sched_in.p;
-  A.n_light = n_light;
+  A.order = c->sched_in.p;
+  A.n_low = n_low;
+  A.n_high = n_high;
+  A.n_heavy = n_heavy;
   A.chunk_beg = t;
   A.chunk_end = t + n_chunks;
+  A.heavy_first = t + 2 * n_chunks;
   A.n_chunks = n_chunks;
-  A.heavy_v = t + 2 * n_chunks;
-  A.heavy_first = t + 2 * n_chunks + n_heavy;
-  A.n_heavy = n_heavy;
   A.partial = c->ppr_partial.p;
   A.state = c->ppr_state.p;
   A.err = c->ppr_err.p;
   A.P = o->damping;
   A.tol = o->tolerance;
   A.k = k;
+  A.tile = tile;
+  A.cols = cols;
   A.max_iter = L;
   A.N = N;
   // Initialization (timed), then iterations as replays of a captured run of check_interval iterations.
   PRH_HIP(c, hipEventRecord(c->ev[0], s));
-  PRH_HIP(c, prh::launch_ppr_reset(A, s));
-  PRH_HIP(c, prh::launch_ppr_init(A, s));
+  PRH_HIP(c, prh::launch_ppr_setup(A, d_seeds, n_seeds, d_first, g->inv, c->ppr_row.p, c->ppr_mass.p, s));
   PRH_HIP(c, hipEventRecord(c->ev[1], s));
   const int chunk = std::max(1, c->tuning.check_interval);
   auto iterations_chunk = [&]() -> int {
-    for (int i = 0; i < chunk; ++i) PRH_HIP(c, prh::launch_ppr_iteration(A, s));
+    for (int i = 0; i < chunk; ++i) PRH_HIP(c, prh::launch_ppr_iteration(A, i, s));
+    PRH_HIP(c, prh::launch_ppr_advance(A, chunk, s));
     return PRH_SUCCESS;
   };
   hipGraphExec_t exec = nullptr;
@@ -159,7 +146,7 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
   if (exec) (void)hipGraphExecDestroy(exec);
   PRH_CHECK(status);
   PRH_HIP(c, hipEventRecord(c->ev[2], s));
-  PRH_HIP(c, prh::launch_ppr_collect(A, c->ppr_out.p, s));
+  PRH_HIP(c, prh::launch_ppr_ranks(A, c->ppr_out.p, s));
   PRH_HIP(c, hipMemcpyAsync(c->pinned, c->ppr_state.p, sizeof(prh::PprState), hipMemcpyDeviceToHost, s));
   PRH_CHECK(copy_to_host(c, ranks, c->ppr_out.p, size_t(N) * k * 8));  // synchronises the stream
   std::memcpy(&hs, c->pinned, sizeof(hs));

@@ -302,38 +302,58 @@ hipError_t sort_pairs_u32(void *tmp, size_t &tmp_bytes, const uint32_t *key_in, 
                           const uint32_t *val_in, uint32_t *val_out, size_t n, int end_bit, hipStream_t s);
 
 // ---- ppr.hip ----
-constexpr int kPprCols = 64;  // teleport columns per batch (one per lane)
+constexpr int kPprCols = 64;         // most teleport columns per call
+// Columns per tile (a million vertices, 17M edges, 64 columns, per solve: 8, 16, 32 and 64 take 149, 124, 116 and 123 ms).
+constexpr int kPprTile = 32;
+// In-degree up to which a row takes a lane group, not a wave: 16 batches of four edges in turn, about what a launch on
+// a small graph lasts (100K vertices, five columns: 2.67, 2.61, 2.61 and 3.45 ms per solve at 16, 32, 64 and 128; a
+// million, 64 columns: 116.3, 114.4, 113.9 and 112.5 ms).
+constexpr uint32_t kPprGroup = 64;
+
+// Columns of a tile for k columns: the power of two that holds them, at most kPprTile.
+inline int ppr_tile(int k) {
+  int t = 1;
+  while (t < k && t < kPprTile) t *= 2;
+  return t;
+}
+
+// Edges per chunk of a heavy row: eight rounds of a wave's eight steps in flight (a wave takes 128 / tile edges a step).
+inline uint32_t ppr_chunk(int tile) { return tile == 1 ? 4096u : 8192u / uint32_t(tile); }
 
 struct PprState {
-  int iter;              // index of the iteration the next launch performs
+  int iter;              // index of the first iteration of the next run
+  int rows;              // rows of the seed table in use
   int done[kPprCols];    // 0 while column j runs, else its number of iterations
 };
 
 struct PprArgs {
-  double *rank[2];                 // [N][64] ping-pong ranks
-  double *contrib[2];              // [N][64] ping-pong rank / out-degree
-  const uint32_t *off, *src, *deg;  // in-CSR and out-degrees
+  double *contrib[2];               // [tiles][N][tile] ping-pong rank / out-degree
+  const uint32_t *off, *src, *deg;  // layout in-CSR and out-degrees
+  const uint32_t *perm;             // layout row -> vertex
   const int32_t *seed_row;          // [N]: row of v in seed_mass, or -1
-  const double *seed_mass;          // [rows][64]: s_j[v]
-  const uint32_t *light;            // vertices with in-degree <= chunk
-  uint32_t n_light;
-  const uint32_t *chunk_beg, *chunk_end;  // edge ranges of the heavy vertices' chunks, heavy vertex by vertex
+  const double *seed_mass;          // [rows][cols]: s_j[v]
+  const uint32_t *order;            // rows by in-degree: [up to kPprGroup | up to the chunk size | heavier]
+  uint32_t n_low, n_high, n_heavy;
+  const uint32_t *chunk_beg, *chunk_end;  // edge ranges of the heavy rows' chunks, row by row
+  const uint32_t *heavy_first;            // chunks of heavy row h are [heavy_first[h], heavy_first[h+1])
   uint32_t n_chunks;
-  const uint32_t *heavy_v, *heavy_first;  // heavy vertices; chunks of heavy_v[h] are [heavy_first[h], heavy_first[h+1])
-  uint32_t n_heavy;
-  double *partial;                  // [n_chunks][64]
+  double *partial;                  // [n_chunks][cols]
   PprState *state;
-  unsigned long long *err;          // [max_iter][64] per-column L-inf change bits
+  unsigned long long *err;          // [max_iter][64] per column: 0 or kChanged
   double P, tol;
   int k;                            // columns in use (1..64)
+  int tile, cols;                   // columns per tile, and of all tiles
   int max_iter;
   uint32_t N;
 };
 
-hipError_t launch_ppr_reset(const PprArgs &a, hipStream_t s);
-hipError_t launch_ppr_init(const PprArgs &a, hipStream_t s);
-hipError_t launch_ppr_iteration(const PprArgs &a, hipStream_t s);  // identical launches every iteration
-hipError_t launch_ppr_collect(const PprArgs &a, double *out, hipStream_t s);
+// Start of a call: state cleared, the seed table built from `seeds` (the columns' seed sets, column j's being
+// seeds[first[j] .. first[j + 1]), turned into layout rows in place), the start contributions.
+hipError_t launch_ppr_setup(const PprArgs &a, uint32_t *seeds, uint32_t n_seeds, const uint32_t *first,
+                            const uint32_t *inv, int32_t *seed_row, double *mass, hipStream_t s);
+hipError_t launch_ppr_iteration(const PprArgs &a, int step, hipStream_t s);  // iteration state->iter + step
+hipError_t launch_ppr_advance(const PprArgs &a, int steps, hipStream_t s);
+hipError_t launch_ppr_ranks(const PprArgs &a, double *out, hipStream_t s);   // out[v * k + j]
 
 // ---- weighted.hip ----
 constexpr int kWeightedBands = 6;  // lanes per low row: 32, 16, 8, 4, 2, 1

@@ -117,3 +117,26 @@ def test_uncaptured_mode_matches_captured(monkeypatch):
         out[mode] = (res.ranks, res.iterations, got.ranks, got.iterations)
     assert np.array_equal(out["0"][0], out["1"][0]) and np.array_equal(out["0"][1], out["1"][1])
     assert np.array_equal(out["0"][2], out["1"][2]) and out["0"][3] == out["1"][3]
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 64])
+def test_tile_widths_and_row_classes(ctx, oracle_mod, k):
+    """Every tile width (and padded columns), on rows at the edges of the row classes: lane groups, waves, chunks.
+    Seed sets overlap, repeat a seed, and include vertices nobody but themselves links to. Bound: the sums of at most
+    40001 non-negative terms in two orders differ by 2 d 2^-53 of the sum, amplified by 1 / (1 - 0.85): 6e-11."""
+    from pagerank_amd import ppr_batched
+    from test_gpu_rows import degree_graph
+    n = 40961
+    y = degree_graph(n, 11)
+    rng = np.random.default_rng(k)
+    seeds = _seed_sets(n, k, 400, rng)
+    seeds[0] = np.array([n - 1, n - 1, 5, n - 2, 5, n - 1], dtype=np.uint32)
+    seeds[k - 1] = np.concatenate([seeds[k - 1], seeds[0]])
+    print(f"[ppr] tiles k={k} N={y.N} M={y.M}", flush=True)
+    res = ppr_batched(ctx.upload(y, with_out=False), seeds)
+    for j in sorted({0, k // 3, k // 2, k - 1}):
+        ref, it = oracle_mod.ppr(y, _teleport(n, seeds[j]))
+        assert abs(int(res.iterations[j]) - it) <= 1
+        if res.iterations[j] == it:
+            assert np.all(np.abs(res.ranks[:, j] - ref) <= 6e-11 * ref)
+        assert np.abs(res.ranks[:, j] - ref).max() <= 1e-9
