@@ -561,6 +561,7 @@ int prh_graph_update(prh_context *c, prh_graph *g, const uint32_t *del_u, const 
   g->plan_valid = false;
   free_sliced(c, g);
   free_binned(c, g->bin_t);
+  free_edge_of(c, g->bin);
   if (g->out_valid) {
     dev_free(c, g->out_chunks, std::max<size_t>(3 * size_t(g->out_n_chunks), 1) * 4);
     g->out_chunks = nullptr;

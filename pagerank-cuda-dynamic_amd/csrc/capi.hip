@@ -202,8 +202,8 @@ void prh_context_destroy(prh_context *c) {
     release(c, c->wt_x[i]);
     release(c, c->wt_z[i]);
   }
-  for (DevBuf<double> *b : {&c->wt_W, &c->wt_Wl, &c->wt_term, &c->wt_terml, &c->wt_r, &c->wt_rl, &c->wt_gwl,
-                            &c->wt_gsl, &c->wt_outM, &c->wt_outN})
+  for (DevBuf<double> *b : {&c->wt_W, &c->wt_Wl, &c->wt_term, &c->wt_terml, &c->wt_r, &c->wt_outM,
+                            &c->wt_outN})
     release(c, *b);
   release(c, c->wt_wout);
   release(c, c->wt_wl);

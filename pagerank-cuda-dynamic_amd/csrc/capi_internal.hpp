@@ -90,7 +90,7 @@ struct prh_context {
   prhc::DevBuf<prh::PprState> ppr_state;
   // weighted forward / adjoint
   // weighted forward / adjoint, on the degree-ordered layout ("l": layout order, else the caller's order)
-  prhc::DevBuf<double> wt_x[2], wt_z[2], wt_W, wt_Wl, wt_term, wt_terml, wt_r, wt_rl, wt_gwl, wt_gsl, wt_outM, wt_outN;
+  prhc::DevBuf<double> wt_x[2], wt_z[2], wt_W, wt_Wl, wt_term, wt_terml, wt_r, wt_outM, wt_outN;
   prhc::DevBuf<float> wt_wout, wt_wl;
   prhc::DevBuf<uint32_t> wt_chunks;       // heavy-row chunk tables of the weighted pull
   prhc::DevBuf<uint32_t> wt_sort, wt_sort_tmp;  // degree sort of its low rows
@@ -119,6 +119,9 @@ struct BinnedCache {
   uint32_t *base_off = nullptr, *base_src = nullptr, *slot_of = nullptr;
   uint64_t base_M = 0, base_cap = 0;  // base edges, and the capacity of base_src
   uint64_t slot_of_n = 0;             // entries of slot_of (the edges of the graph the plan was built from)
+  // Weighted solves: the caller's edge of every slot (the slot map composed with the layout's edge map), and its entries.
+  uint32_t *edge_of = nullptr;
+  uint64_t edge_of_n = 0;
   unsigned long long *ov_key = nullptr;
   uint32_t *ov_off = nullptr;
   double *ovX = nullptr;
@@ -314,6 +317,7 @@ int build_binned(prh_context *c, uint32_t N, uint64_t M, const uint32_t *off, co
                  const std::vector<uint32_t> &rowdeg, bool keep_slot, BinnedCache &bc);
 void free_binned(prh_context *c, BinnedCache &bc);
 void free_overlay(prh_context *c, BinnedCache &bc);
+void free_edge_of(prh_context *c, BinnedCache &bc);
 int build_binned_plan(prh_context *c, prh_graph *g, bool keep_slot = false);
 int build_binned_plan_t(prh_context *c, prh_graph *g);
 int build_rank_plan(prh_context *c, prh_graph *g);

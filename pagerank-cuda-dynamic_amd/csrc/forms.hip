@@ -244,7 +244,12 @@ int weighted_common(prh_context *c, const prh_graph *g, const float *w, const pr
   PRH_CHECK(stage(c, w, size_t(M), device, c->wt_wout, w_out));
   PRH_CHECK(ensure(c, c->wt_W, N));
   PRH_CHECK(ensure(c, c->wt_Wl, N));
-  PRH_HIP(c, prh::launch_out_weight_sum(g->out_off, *w_out, N, c->wt_W.p, hs));
+  PRH_CHECK(ensure(c, c->sched_out, N));
+  PRH_CHECK(ensure(c, c->tiles, size_t(3) * prh::partition_tiles(N)));
+  PRH_CHECK(ensure(c, c->counts, 8));
+  PRH_HIP(c, prh::launch_partition(g->out_off, N, prh::kSumLane, prh::kSumWave, c->sched_out.p, c->tiles.p, c->counts.p,
+                                   hs));
+  PRH_HIP(c, prh::launch_out_weight_sum(g->out_off, *w_out, N, c->sched_out.p, c->counts.p, c->wt_W.p, hs));
   PRH_HIP(c, prh::launch_gather_f64(c->wt_W.p, g->perm, N, c->wt_Wl.p, hs));
   PRH_CHECK(ensure(c, c->wt_wl, std::max<uint64_t>(1, M)));
   for (int i = 0; i < 2; ++i) {
@@ -359,6 +364,23 @@ int from_layout(prh_context *c, const double *src, const uint32_t *map, size_t n
   return PRH_SUCCESS;
 }
 
+// The weights in the slot order of a blocked plan (wt_wl), through the map from slots to the caller's edges: kept with
+// the plan, or composed for each weight where there is no room for it.
+int slot_weights(prh_context *c, BinnedCache &bc, const float *w, const uint32_t *eid, uint64_t M) {
+  if (!bc.edge_of && M) {
+    if (dev_alloc(c, reinterpret_cast<void **>(&bc.edge_of), M * 4) == PRH_SUCCESS) {
+      bc.edge_of_n = M;
+      PRH_HIP(c, prh::launch_permute_u32(eid, bc.plan.slot, M, bc.edge_of, c->stream));
+    } else {
+      bc.edge_of = nullptr;
+      c->error.clear();
+    }
+  }
+  if (bc.edge_of) PRH_HIP(c, prh::launch_permute_weights(w, bc.edge_of, M, c->wt_wl.p, c->stream));
+  else PRH_HIP(c, prh::launch_binned_weights(w, eid, bc.plan.slot, M, c->wt_wl.p, c->stream));
+  return PRH_SUCCESS;
+}
+
 int weighted_forward_impl(prh_context *c, const prh_graph *g, const float *w, const double *s, const prh_options *o,
                           double *ranks, prh_stats *st, bool device) {
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
@@ -375,7 +397,7 @@ int weighted_forward_impl(prh_context *c, const prh_graph *g, const float *w, co
     prh_graph *gm = const_cast<prh_graph *>(g);
     PRH_CHECK(build_binned_plan(c, gm, true));
     const float prep = gm->layout_prep.take() + gm->bin.prep.take();  // one-time preparation, as solve_impl reports it
-    PRH_HIP(c, prh::launch_binned_weights(w_out, g->l_in_eid, g->bin.plan.slot, M, c->wt_wl.p, hs));
+    PRH_CHECK(slot_weights(c, gm->bin, w_out, g->l_in_eid, M));
     prh::BinnedPlan plan = g->bin.plan;
     plan.ws = c->wt_wl.p;
     PRH_HIP(c, hipEventRecord(c->ev[0], hs));
@@ -446,7 +468,6 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
   PRH_CHECK(stage(c, gr, N, device, c->wt_term, &term));
   PRH_CHECK(stage(c, r, N, device, c->wt_r, &rr));
   PRH_CHECK(to_layout(c, g, term, c->wt_terml));
-  PRH_CHECK(to_layout(c, g, rr, c->wt_rl));
   const bool blocked = c->tuning.blocking > 0;  // through the propagation-blocked plan of the layout out-CSR
   prh::BinnedPlan plan{};
   prh::WeightedArgs A0{};
@@ -455,7 +476,7 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
     prh_graph *gm = const_cast<prh_graph *>(g);
     PRH_CHECK(build_binned_plan_t(c, gm));
     prep += gm->bin_t.prep.take();
-    PRH_HIP(c, prh::launch_binned_weights(w_out, g->l_out_eid, g->bin_t.plan.slot, M, c->wt_wl.p, hs));
+    PRH_CHECK(slot_weights(c, gm->bin_t, w_out, g->l_out_eid, M));
     plan = g->bin_t.plan;
     plan.ws = c->wt_wl.p;
   } else {
@@ -490,15 +511,24 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
     PRH_HIP(c, prh::launch_weighted_step(true, A, err, done, l, o->tolerance, hs));
     return PRH_SUCCESS;
   }, &n));
-  const double *lam_l = c->wt_x[n & 1].p;
-  PRH_CHECK(ensure(c, c->wt_gwl, std::max<uint64_t>(1, M)));
-  PRH_CHECK(ensure(c, c->wt_gsl, N));
-  PRH_HIP(c, prh::launch_weighted_grad(g->l_out_off, g->l_out_dst, c->wt_Wl.p, c->wt_rl.p, lam_l, c->wt_terml.p,
-                                       o->damping, N, c->wt_gwl.p, c->wt_gsl.p, hs));
+  // The gradients are computed in the caller's order, from the caller's CSR: only lambda goes back from the layout's.
+  double *lam_c = c->wt_z[0].p, *gw = grad_w, *gs = grad_s;
+  if (!device) {
+    PRH_CHECK(ensure(c, c->wt_outM, std::max<uint64_t>(1, M)));
+    PRH_CHECK(ensure(c, c->wt_outN, N));
+    gw = c->wt_outM.p;
+    gs = c->wt_outN.p;
+  }
+  PRH_HIP(c, prh::launch_scatter_f64(c->wt_x[n & 1].p, g->perm, N, lam_c, hs));
+  PRH_HIP(c, prh::launch_weighted_grad(g->out_off, g->out_dst, c->wt_W.p, rr, lam_c, term, o->damping, N, M,
+                                       c->wt_z[1].p, c->wt_x[(n + 1) & 1].p, gw, gs, hs));
   PRH_HIP(c, hipEventRecord(c->ev[2], hs));
-  if (lam) PRH_CHECK(from_layout(c, lam_l, g->perm, N, lam, device, c->wt_z[0]));
-  PRH_CHECK(from_layout(c, c->wt_gwl.p, g->l_out_eid, M, grad_w, device, c->wt_outM));
-  PRH_CHECK(from_layout(c, c->wt_gsl.p, g->perm, N, grad_s, device, c->wt_outN));
+  if (lam)
+    PRH_HIP(c, hipMemcpyAsync(lam, lam_c, size_t(N) * 8, device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, hs));
+  if (!device) {
+    if (M) PRH_HIP(c, hipMemcpyAsync(grad_w, gw, size_t(M) * 8, hipMemcpyDeviceToHost, hs));
+    PRH_HIP(c, hipMemcpyAsync(grad_s, gs, size_t(N) * 8, hipMemcpyDeviceToHost, hs));
+  }
   PRH_HIP(c, hipStreamSynchronize(hs));
   float t01 = 0, t12 = 0;
   PRH_HIP(c, hipEventElapsedTime(&t01, c->ev[0], c->ev[1]));

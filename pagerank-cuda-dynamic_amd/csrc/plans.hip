@@ -226,9 +226,16 @@ void free_binned(prh_context *c, BinnedCache &bc) {
   dev_free(c, bc.base_off, bc.base_off ? (size_t(N) + 1) * 4 : 0);
   dev_free(c, bc.base_src, bc.base_src ? std::max<size_t>(bc.base_cap, 4) * 4 : 0);
   dev_free(c, bc.slot_of, bc.slot_of ? std::max<size_t>(bc.slot_of_n, 4) * 4 : 0);
+  free_edge_of(c, bc);
   free_overlay(c, bc);
   bc.base_off = bc.base_src = bc.slot_of = nullptr;
   bc.base_M = bc.base_cap = bc.slot_of_n = 0;
+}
+
+void free_edge_of(prh_context *c, BinnedCache &bc) {
+  dev_free(c, bc.edge_of, bc.edge_of_n * 4);
+  bc.edge_of = nullptr;
+  bc.edge_of_n = 0;
 }
 
 void free_overlay(prh_context *c, BinnedCache &bc) {

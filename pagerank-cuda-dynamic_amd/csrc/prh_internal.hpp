@@ -388,17 +388,22 @@ hipError_t launch_weighted_step(bool adjoint, const WeightedArgs &A, unsigned lo
                                 double tol, hipStream_t s);
 // key[i] = 64 - degree of row order[i], for the first n rows (degrees <= 64).
 hipError_t launch_degree_keys(const uint32_t *off, const uint32_t *order, uint32_t n, uint32_t *key, hipStream_t s);
-hipError_t launch_out_weight_sum(const uint32_t *out_off, const float *w, uint32_t N, double *W, hipStream_t s);
+// Out-weight sums. order, counts (device): the rows partitioned by out-degree at kSumLane and kSumWave.
+constexpr uint32_t kSumLane = 64, kSumWave = 4096;  // out-degrees up to which a lane, a wave sums a row
+hipError_t launch_out_weight_sum(const uint32_t *out_off, const float *w, uint32_t N, const uint32_t *order,
+                                 const uint32_t *counts, double *W, hipStream_t s);
 // eid[k] = raw out-CSR slot of slot k of a degree-ordered layout CSR (transpose: its in-CSR, else its out-CSR).
 hipError_t launch_layout_edge_map(const uint32_t *l_off, const uint32_t *l_idx, const uint32_t *perm,
                                   const uint32_t *out_off, const uint32_t *out_dst, uint32_t N, bool transpose,
                                   uint32_t *eid, int *missing, hipStream_t s);
 hipError_t launch_permute_weights(const float *w_out, const uint32_t *in_eid, size_t M, float *w_in, hipStream_t s);
+hipError_t launch_permute_u32(const uint32_t *src, const uint32_t *idx, size_t M, uint32_t *dst, hipStream_t s);
 hipError_t launch_weighted_init(const double *start, const double *W, uint32_t N, bool adjoint, double *x, double *z,
                                 hipStream_t s);
+// Every row needs an edge. fu, su: scratch of N doubles each.
 hipError_t launch_weighted_grad(const uint32_t *out_off, const uint32_t *out_dst, const double *W, const double *r,
-                                const double *lam, const double *g, double P, uint32_t N, double *grad_w,
-                                double *grad_s, hipStream_t s);
+                                const double *lam, const double *g, double P, uint32_t N, uint64_t M, double *fu,
+                                double *su, double *grad_w, double *grad_s, hipStream_t s);
 
 // ---- layout.hip ----
 hipError_t launch_invert(const uint32_t *perm, uint32_t N, uint32_t *inv, hipStream_t s);

@@ -29,16 +29,31 @@ __device__ __forceinline__ double wfinish(const WeightedArgs &A, uint32_t i, dou
   return fabs(a - A.x_old[i]);
 }
 
-template <int STEP>
-__device__ __forceinline__ double wgather(const WeightedArgs &A, uint32_t e, uint32_t end) {
+// Sum of w z over edges i, i + STEP, ... < n of the row whose edges start at b, U of them in flight: a batch costs two
+// round trips, and two at a time left a wave's row of 4096 edges a chain of 64.
+template <int STEP, int U>
+__device__ __forceinline__ double wgather(const WeightedArgs &A, uint32_t b, uint32_t i, uint32_t n) {
+  const uint32_t *idx = A.idx + b;
+  const float *w = A.w + b;
   double s0 = 0.0, s1 = 0.0;
-  for (; e + STEP < end; e += 2 * STEP) {
-    const uint32_t u0 = A.idx[e], u1 = A.idx[e + STEP];
-    const float w0 = A.w[e], w1 = A.w[e + STEP];
-    s0 += double(w0) * A.z[u0];
-    s1 += double(w1) * A.z[u1];
+  for (; i < n; i += U * STEP) {
+    uint32_t u[U];
+    float f[U];
+    double x[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const bool in = i + k * STEP < n;
+      u[k] = in ? idx[i + k * STEP] : 0u;
+      f[k] = in ? w[i + k * STEP] : 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) x[k] = i + k * STEP < n ? A.z[u[k]] : 0.0;
+#pragma unroll
+    for (int k = 0; k < U; k += 2) {
+      s0 += double(f[k]) * x[k];
+      if (k + 1 < U) s1 += double(f[k + 1]) * x[k + 1];
+    }
   }
-  for (; e < end; e += STEP) s0 += double(A.w[e]) * A.z[A.idx[e]];
   return s0 + s1;
 }
 
@@ -54,7 +69,8 @@ __device__ __forceinline__ void band_rows(const WeightedArgs &A, uint32_t rb, ui
     uint32_t v = 0;
     if (i < re) {
       v = A.sched.order[i];
-      s = wgather<W>(A, A.off[v] + j, A.off[v + 1]);
+      const uint32_t b = A.off[v];
+      s = wgather<W, 2>(A, b, j, A.off[v + 1] - b);
     }
     s = group_sum<W>(s);
     if (i < re && j == 0) emax = fmax(emax, wfinish<ADJOINT>(A, v, s));
@@ -70,7 +86,8 @@ __global__ __launch_bounds__(kBlock) void weighted_step_kernel(WeightedArgs A, u
   __shared__ double lds[kWavesPerBlock];
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   if (blockIdx.x < A.n_chunks) {  // block-uniform
-    double s = group_sum<kWave>(wgather<kBlock>(A, A.chunk_beg[blockIdx.x] + threadIdx.x, A.chunk_end[blockIdx.x]));
+    const uint32_t cb = A.chunk_beg[blockIdx.x];
+    const double s = group_sum<kWave>(wgather<kBlock, 8>(A, cb, threadIdx.x, A.chunk_end[blockIdx.x] - cb));
     if (lane == 0) lds[w] = s;
     __syncthreads();
     if (threadIdx.x == 0) A.partial[blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
@@ -83,8 +100,8 @@ __global__ __launch_bounds__(kBlock) void weighted_step_kernel(WeightedArgs A, u
     const uint32_t n = A.sched.n_high;
     for (uint32_t i = b * kWavesPerBlock + w; i < n; i += nb_high * kWavesPerBlock) {
       const uint32_t v = order[i];
-      double s = wgather<kWave>(A, A.off[v] + lane, A.off[v + 1]);
-      s = group_sum<kWave>(s);
+      const uint32_t rb = A.off[v];
+      const double s = group_sum<kWave>(wgather<kWave, 8>(A, rb, lane, A.off[v + 1] - rb));
       if (lane == 0) emax = fmax(emax, wfinish<ADJOINT>(A, v, s));
     }
   } else {
@@ -122,15 +139,54 @@ __global__ __launch_bounds__(kBlock) void weighted_heavy_kernel(WeightedArgs A, 
   report_change(ctl, emax);
 }
 
-// W_u = sum of u's out-weights (FP64), one wave per row.
-__global__ __launch_bounds__(kBlock) void out_weight_sum_kernel(const uint32_t *out_off, const float *w, uint32_t N,
-                                                                double *W) {
-  const int wv = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  for (uint32_t u = blockIdx.x * kWavesPerBlock + wv; u < N; u += gridDim.x * kWavesPerBlock) {
-    double s = 0.0;
-    for (uint32_t e = out_off[u] + lane; e < out_off[u + 1]; e += kWave) s += double(w[e]);
-    s = group_sum<kWave>(s);
-    if (lane == 0) W[u] = s;
+// Sum of w[i], w[i + STEP], ... below n, eight loads in flight.
+template <int STEP>
+__device__ __forceinline__ double weight_sum(const float *w, uint32_t i, uint32_t n) {
+  double s0 = 0.0, s1 = 0.0;
+  for (; i < n; i += 8 * STEP) {
+    float f[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) f[k] = i + k * STEP < n ? w[i + k * STEP] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) {
+      s0 += double(f[k]);
+      s1 += double(f[k + 1]);
+    }
+  }
+  return s0 + s1;
+}
+
+// W_u = sum of u's out-weights (FP64): a lane, a wave or a workgroup per row by its class in `order` (the rows
+// partitioned by out-degree: counts[0] up to kSumLane, counts[1] up to kSumWave, counts[2] heavier; device words). The
+// first nb_hub workgroups take the heaviest rows, the next nb_wave the middle ones. With a wave for every row and one
+// load in flight the hubs set the time: 1M vertices, 17M edges 897 -> 58 us, and 16 us for the partition.
+__global__ __launch_bounds__(kBlock) void out_weight_sum_kernel(const uint32_t *out_off, const float *w,
+                                                                const uint32_t *order, const uint32_t *counts,
+                                                                uint32_t nb_hub, uint32_t nb_wave, double *W) {
+  __shared__ double part[kWavesPerBlock];
+  const uint32_t t = threadIdx.x, wv = t / kWave, lane = t & (kWave - 1);
+  const uint32_t n_lane = counts[0], n_wave = counts[1], n_hub = counts[2];
+  if (blockIdx.x < nb_hub) {
+    for (uint32_t i = blockIdx.x; i < n_hub; i += nb_hub) {  // block-uniform
+      const uint32_t u = order[n_lane + n_wave + i], b = out_off[u];
+      const double s = group_sum<kWave>(weight_sum<kBlock>(w + b, t, out_off[u + 1] - b));
+      if (lane == 0) part[wv] = s;
+      __syncthreads();
+      if (t == 0) W[u] = (part[0] + part[1]) + (part[2] + part[3]);
+      __syncthreads();
+    }
+  } else if (blockIdx.x < nb_hub + nb_wave) {
+    for (uint32_t i = (blockIdx.x - nb_hub) * kWavesPerBlock + wv; i < n_wave; i += nb_wave * kWavesPerBlock) {
+      const uint32_t u = order[n_lane + i], b = out_off[u];
+      const double s = group_sum<kWave>(weight_sum<kWave>(w + b, lane, out_off[u + 1] - b));
+      if (lane == 0) W[u] = s;
+    }
+  } else {
+    const uint32_t nb = gridDim.x - nb_hub - nb_wave;
+    for (uint32_t i = (blockIdx.x - nb_hub - nb_wave) * kBlock + t; i < n_lane; i += nb * kBlock) {
+      const uint32_t u = order[i], b = out_off[u];
+      W[u] = weight_sum<1>(w + b, 0, out_off[u + 1] - b);
+    }
   }
 }
 
@@ -168,6 +224,12 @@ __global__ __launch_bounds__(kBlock) void permute_weights_kernel(const float *w_
     w_in[k] = w_out[in_eid[k]];
 }
 
+__global__ __launch_bounds__(kBlock) void permute_u32_kernel(const uint32_t *src, const uint32_t *idx, size_t M,
+                                                             uint32_t *dst) {
+  for (size_t k = size_t(blockIdx.x) * kBlock + threadIdx.x; k < M; k += size_t(gridDim.x) * kBlock)
+    dst[k] = src[idx[k]];
+}
+
 // x = z = start (adjoint: lam0 = g) or x = s, z = s / W (forward: r0 = s).
 __global__ __launch_bounds__(kBlock) void weighted_init_kernel(const double *start, const double *W, uint32_t N,
                                                                int adjoint, double *x, double *z) {
@@ -178,18 +240,86 @@ __global__ __launch_bounds__(kBlock) void weighted_init_kernel(const double *sta
   }
 }
 
-// dL/dw (out-CSR order) and dL/ds, one wave per source row.
-__global__ __launch_bounds__(kBlock) void weighted_grad_kernel(const uint32_t *out_off, const uint32_t *out_dst,
-                                                               const double *W, const double *r, const double *lam,
-                                                               const double *g, double P, uint32_t N,
-                                                               double *grad_w, double *grad_s) {
-  const int wv = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  for (uint32_t u = blockIdx.x * kWavesPerBlock + wv; u < N; u += gridDim.x * kWavesPerBlock) {
+// Per source u: dL/ds_u, and the factors of its edges' gradients dL/dw_uv = fu (lam_v - su).
+__global__ __launch_bounds__(kBlock) void weighted_factors_kernel(const double *W, const double *r, const double *lam,
+                                                                  const double *g, double P, uint32_t N, double *fu,
+                                                                  double *su, double *grad_s) {
+  for (uint32_t u = blockIdx.x * kBlock + threadIdx.x; u < N; u += gridDim.x * kBlock) {
     const double lu = lam[u];
-    const double su = (lu - g[u]) / P;
-    const double fu = P * r[u] / W[u];
-    for (uint32_t e = out_off[u] + lane; e < out_off[u + 1]; e += kWave) grad_w[e] = fu * (lam[out_dst[e]] - su);
-    if (lane == 0) grad_s[u] = (1 - P) * lu;
+    su[u] = (lu - g[u]) / P;
+    fu[u] = P * r[u] / W[u];
+    grad_s[u] = (1 - P) * lu;
+  }
+}
+
+constexpr uint32_t kGradEdges = 4096;  // edges per workgroup of the gradient
+
+// dL/dw in the caller's edge order, so that the gradients are written once and in sequence, kGradEdges edges a
+// workgroup however the rows fall (every row has an edge). A wave finds the tile's first row (64 offsets a round); the
+// rows that start in the tile leave their number at their first edge, and a running maximum turns that into every
+// edge's row. (A wave per row of the layout, and the result scattered to the caller's order: 507 + 120 us on 1M
+// vertices, 17M edges, bound by the hubs' rows; a workgroup per 256 rows 1758 us, bound by the 256 that hold the hubs;
+// this: 123 us, and 15 us for the factors.)
+__global__ __launch_bounds__(kBlock) void weighted_grad_kernel(const uint32_t *out_off, const uint32_t *out_dst,
+                                                               const double *lam, const double *fu, const double *su,
+                                                               uint32_t N, uint64_t M, double *grad_w) {
+  constexpr uint32_t E = kGradEdges / kBlock;  // edges per thread
+  __shared__ uint16_t row[kGradEdges];
+  __shared__ uint32_t first, top[kWavesPerBlock];
+  const uint32_t t = threadIdx.x, wv = t / kWave, lane = t & (kWave - 1);
+  const uint64_t e0 = uint64_t(blockIdx.x) * kGradEdges;
+  const uint32_t n = uint32_t(min(uint64_t(kGradEdges), M - e0));
+  if (wv == 0) {  // the last row with off[row] <= e0
+    uint64_t lo = 0, hi = N;
+    while (hi - lo > 1) {
+      const uint64_t step = (hi - lo + kWave - 1) / kWave, at = lo + lane * step;
+      const uint32_t k = __popcll(__ballot(at < hi && out_off[at] <= e0));  // at least 1: lane 0
+      hi = min(hi, lo + k * step);
+      lo += (k - 1) * step;
+    }
+    if (lane == 0) first = uint32_t(lo);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) row[k * kBlock + t] = 0;
+  __syncthreads();
+  const uint32_t r0 = first;
+  for (uint32_t i = 1 + t; i <= kGradEdges && r0 + i < N; i += kBlock) {
+    const uint64_t b = out_off[r0 + i] - e0;  // row r0 + i > r0 starts after e0
+    if (b >= n) break;
+    row[b] = uint16_t(i);
+  }
+  __syncthreads();
+  // Running maximum: thread t over its E edges, then over the threads before it.
+  uint32_t m[E], best = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) m[k] = best = max(best, uint32_t(row[t * E + k]));
+  uint32_t up = best;  // inclusive over the wave
+#pragma unroll
+  for (int d = 1; d < kWave; d *= 2) {
+    const uint32_t o = __shfl_up(up, d);
+    if (lane >= uint32_t(d)) up = max(up, o);
+  }
+  if (lane == kWave - 1) top[wv] = up;
+  uint32_t before = __shfl_up(up, 1);
+  if (lane == 0) before = 0;
+  __syncthreads();
+  for (uint32_t k = 0; k < wv; ++k) before = max(before, top[k]);
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) row[t * E + k] = uint16_t(max(before, m[k]));
+  __syncthreads();
+  for (uint32_t i = t; i < n; i += 8 * kBlock) {
+    uint32_t v[8];
+    double x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = i + k * kBlock < n ? out_dst[e0 + i + k * kBlock] : 0u;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = i + k * kBlock < n ? lam[v[k]] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (i + k * kBlock >= n) break;
+      const uint32_t u = r0 + row[i + k * kBlock];
+      grad_w[e0 + i + k * kBlock] = fu[u] * (x[k] - su[u]);
+    }
   }
 }
 
@@ -235,9 +365,11 @@ hipError_t launch_degree_keys(const uint32_t *off, const uint32_t *order, uint32
   return hipGetLastError();
 }
 
-hipError_t launch_out_weight_sum(const uint32_t *out_off, const float *w, uint32_t N, double *W, hipStream_t s) {
+hipError_t launch_out_weight_sum(const uint32_t *out_off, const float *w, uint32_t N, const uint32_t *order,
+                                 const uint32_t *counts, double *W, hipStream_t s) {
   if (!N) return hipSuccess;
-  out_weight_sum_kernel<<<blocks(N, kWavesPerBlock, 16384), kBlock, 0, s>>>(out_off, w, N, W);
+  const uint32_t nb_hub = 256, nb_wave = blocks(N, 16 * kWavesPerBlock, 2048), nb_lane = blocks(N, kBlock, 8192);
+  out_weight_sum_kernel<<<nb_hub + nb_wave + nb_lane, kBlock, 0, s>>>(out_off, w, order, counts, nb_hub, nb_wave, W);
   return hipGetLastError();
 }
 
@@ -256,6 +388,12 @@ hipError_t launch_permute_weights(const float *w_out, const uint32_t *in_eid, si
   return hipGetLastError();
 }
 
+hipError_t launch_permute_u32(const uint32_t *src, const uint32_t *idx, size_t M, uint32_t *dst, hipStream_t s) {
+  if (!M) return hipSuccess;
+  permute_u32_kernel<<<blocks(M, kBlock, 16384), kBlock, 0, s>>>(src, idx, M, dst);
+  return hipGetLastError();
+}
+
 hipError_t launch_weighted_init(const double *start, const double *W, uint32_t N, bool adjoint, double *x, double *z,
                                 hipStream_t s) {
   if (!N) return hipSuccess;
@@ -264,11 +402,13 @@ hipError_t launch_weighted_init(const double *start, const double *W, uint32_t N
 }
 
 hipError_t launch_weighted_grad(const uint32_t *out_off, const uint32_t *out_dst, const double *W, const double *r,
-                                const double *lam, const double *g, double P, uint32_t N, double *grad_w,
-                                double *grad_s, hipStream_t s) {
+                                const double *lam, const double *g, double P, uint32_t N, uint64_t M, double *fu,
+                                double *su, double *grad_w, double *grad_s, hipStream_t s) {
   if (!N) return hipSuccess;
-  weighted_grad_kernel<<<blocks(N, kWavesPerBlock, 16384), kBlock, 0, s>>>(out_off, out_dst, W, r, lam, g, P, N,
-                                                                           grad_w, grad_s);
+  weighted_factors_kernel<<<blocks(N, kBlock, 8192), kBlock, 0, s>>>(W, r, lam, g, P, N, fu, su, grad_s);
+  if (M)
+    weighted_grad_kernel<<<uint32_t((M + kGradEdges - 1) / kGradEdges), kBlock, 0, s>>>(out_off, out_dst, lam, fu, su, N,
+                                                                                       M, grad_w);
   return hipGetLastError();
 }
 

@@ -146,3 +146,35 @@ def test_fp64_inputs_get_fp64_gradients(ctx):
     assert np.array_equal(r.detach().cpu().numpy(), fw.ranks)
     assert np.abs(wt.grad.cpu().numpy() - gw).max() <= 1e-15
     assert np.abs(st.grad.cpu().numpy() - gs).max() <= 1e-15
+
+
+@pytest.mark.parametrize("blocking", [0, 2048], ids=["rows", "blocked"])
+@pytest.mark.parametrize("flip", [False, True], ids=["in", "out"])
+def test_row_classes_and_gradient_tiles(ctx, oracle_mod, flip, blocking):
+    """Rows at the edges of the degree classes (a lane, a wave, a workgroup; chunks) as in-rows or as out-rows, and the
+    gradient's tiles of 4096 edges cutting them: the gradient from the solver's own lambda equals the oracle's formula up
+    to the rounding of W (sums of at most 40001 terms in two orders: 2 * 40001 * 2^-53 < 1e-11 of it)."""
+    from pagerank_amd import HostGraph, Tuning, weighted_adjoint, weighted_pagerank
+    from test_gpu_rows import degree_graph
+    y = degree_graph(40961, 5)
+    if flip:
+        y = HostGraph.from_edges(y.N, y.out_edg, y.out_sources())
+    rng = np.random.default_rng(3)
+    w, c, s = rng.uniform(0.5, 1.5, y.M).astype(np.float32), rng.standard_normal(y.N), np.full(y.N, 1.0 / y.N)
+    print(f"[adjoint] rows flip={flip} blocking={blocking} N={y.N} M={y.M}", flush=True)
+    old = ctx.get_tuning()
+    ctx.set_tuning(Tuning(**{**old.__dict__, "blocking": blocking}))
+    try:
+        _forward_and_adjoint(ctx, oracle_mod, y, w, c, s)
+        yg = ctx.upload(y)
+        r = weighted_pagerank(yg, w, s).ranks
+        g = 2 * c * r
+        lam, gw, gs, _ = weighted_adjoint(yg, w, r, g)
+    finally:
+        ctx.set_tuning(old)
+    W = np.add.reduceat(w.astype(np.float64), y.out_off[:-1].astype(np.int64))
+    gw_o, gs_o = oracle_mod.weighted_grad(y, W, r, lam, g)
+    u, v = y.out_sources(), y.out_edg
+    size = (0.85 * r / W)[u] * (np.abs(lam[v]) + (np.abs(lam - g) / 0.85)[u])
+    assert np.all(np.abs(gw - gw_o) <= 1e-11 * size)
+    assert np.all(np.abs(gs - gs_o) <= 1e-15 * np.abs(lam))
