@@ -86,7 +86,8 @@ typedef struct prh_tuning {
                              summed by a second launch [16384] */
   int low_width;          /* lanes per vertex of in-degree <= switch_degree: 1, 2, 4, 8, 16 or 32; 0 = by degree
                              band, W lanes for in-degree in (W, 2W] (the weighted solves always use bands) [0] */
-  int check_interval;     /* iterations launched between host reads of the device convergence flag [8] */
+  int check_interval;     /* most iterations launched ahead of the device, which tells the host when it has converged;
+                             batched PPR: iterations per replayed HIP graph [8] */
   int source_slices;      /* Static / Naive-dynamic: 0 = row kernel; 1, 2, 4 or 8 = sum each row slice by slice,
                              source u in slice (u / 16) mod source_slices, slice x on the workgroups b with
                              b mod source_slices = x (8: one slice per XCD and its L2) [0] */
@@ -260,7 +261,7 @@ int prh_autotune(prh_context *context, const prh_graph *graph, const char *cache
  * ranks: PRH_STATIC (from 1/N), PRH_NAIVE_DYNAMIC, PRH_DYNAMIC_TRAVERSAL (the closure's levels run on the device,
  * each only while the one before it marked a vertex), PRH_DYNAMIC_FRONTIER or PRH_PRUNE_DYNAMIC_FRONTIER. The
  * batch application, the update plan's patch and the marking run as one captured HIP graph, the traversal closure as
- * a captured graph of 8 levels and the iterations as a captured graph of 8 iterations, each replayed until the
+ * a captured graph of 8 levels and the iterations as a captured graph of 4 iterations, each replayed until the
  * device reports it done. When the context's tuning asks for propagation blocking with blocks of at most 8192
  * vertices, the session builds that plan of the base graph and patches it per batch (deleted slots flagged dead,
  * other inserted edges kept in an overlay), as prh_graph_update does; otherwise it runs the row plan. Batch ids are

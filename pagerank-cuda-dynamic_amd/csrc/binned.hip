@@ -159,6 +159,7 @@ __global__ __launch_bounds__(kBinBlock) void expand_kernel(BinnedPlan P, const d
     const uint32_t a = __builtin_nontemporal_load(s32 + p);
     __builtin_nontemporal_store(d2{c[a & 0xFFFFu], c[a >> 16]}, x2 + p);
   }
+  report_begun(ctl);
 }
 
 constexpr uint32_t kPairStart = 0x8000u, kRunStart = 0x4000u;
@@ -321,6 +322,7 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
   }
   wg_store_costs<VARIANT, kBinWaves>(A, cost, blockIdx.x, lds_cost);
   report_change(ctl, emax);
+  report_begun(ctl);
 }
 
 // Split bins, one workgroup per unit (bin, first partial row, rows, first vertex | mode << 31):
@@ -409,13 +411,15 @@ hipError_t binned_update(const RankArgs &A, const BinnedPlan &P, const LoopCtl &
                          hipEvent_t mark) {
   const uint8_t *naff = Traits<VARIANT>::frontier && extend ? A.naff : nullptr;
   constexpr bool kFromRanks = !Traits<VARIANT>::weighted;
+  LoopCtl rest = ctl;  // only the first launch tells the host
+  if (P.n_ex) rest.host = nullptr;
   if (P.n_ex) expand_kernel<B, kFromRanks><<<P.n_ex, kBinBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, ctl);
   if (P.ov_n) {
     const uint32_t g = (P.ov_n + kBlock - 1) / kBlock;
-    overlay_expand_kernel<kFromRanks><<<g < 4096 ? g : 4096, kBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, ctl);
+    overlay_expand_kernel<kFromRanks><<<g < 4096 ? g : 4096, kBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, rest);
   }
-  accumulate_kernel<B, VARIANT><<<P.n_ac, kBinBlock, 0, s>>>(A, P, ctl);
-  if (P.n_multi) finish_bins_kernel<VARIANT><<<P.n_multi, kBinBlock, 0, s>>>(A, P, ctl);
+  accumulate_kernel<B, VARIANT><<<P.n_ac, kBinBlock, 0, s>>>(A, P, rest);
+  if (P.n_multi) finish_bins_kernel<VARIANT><<<P.n_multi, kBinBlock, 0, s>>>(A, P, rest);
   if (mark) {
     const hipError_t e = hipEventRecord(mark, s);
     if (e != hipSuccess) return e;
@@ -628,9 +632,8 @@ hipError_t binned_update_variant(int variant, const RankArgs &A, const BinnedPla
 
 }  // namespace
 
-hipError_t launch_binned_update(int variant, const RankArgs &A, const BinnedPlan &P, unsigned long long *err,
-                                int *done, int l, double tol, bool extend, hipStream_t s, hipEvent_t mark) {
-  const LoopCtl ctl{err, done, l, tol};
+hipError_t launch_binned_update(int variant, const RankArgs &A, const BinnedPlan &P, const LoopCtl &ctl, bool extend,
+                                hipStream_t s, hipEvent_t mark) {
   switch (P.B) {
     case 1024: return binned_update_variant<1024>(variant, A, P, ctl, extend, s, mark);
     case 2048: return binned_update_variant<2048>(variant, A, P, ctl, extend, s, mark);

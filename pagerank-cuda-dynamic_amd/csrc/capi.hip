@@ -144,7 +144,9 @@ int prh_context_create(int device, prh_context **out) {
   prh_default_tuning(&c->tuning);
   if (const char *e = std::getenv("PRH_GRAPH_CAPTURE")) c->capture = std::strcmp(e, "0") != 0;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void **>(&c->pinned), kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc(reinterpret_cast<void **>(&c->pinned), kPinnedBytes, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void **>(&c->progress), kProgressBytes,
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     (void)hipGetLastError();
     prh_context_destroy(c);
     return PRH_ERROR_DEVICE;
@@ -216,6 +218,7 @@ void prh_context_destroy(prh_context *c) {
   for (auto &e : c->kev)
     if (e) (void)hipEventDestroy(e);
   if (c->pinned) (void)hipHostFree(c->pinned);
+  if (c->progress) (void)hipHostFree(c->progress);
   if (c->staging) (void)hipHostFree(c->staging);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;

@@ -23,7 +23,7 @@
 
 namespace prhc {
 
-constexpr size_t kPinnedBytes = 4096;
+constexpr size_t kPinnedBytes = 4096, kProgressBytes = 64;
 
 constexpr size_t kStagingBytes = size_t(64) << 20;
 
@@ -96,6 +96,9 @@ struct prh_context {
   prhc::DevBuf<uint32_t> wt_sort, wt_sort_tmp;  // degree sort of its low rows
   prhc::DevBuf<double> wt_partial;        // their sums
   uint64_t *pinned = nullptr;       // small host-pinned readback area (kPinnedBytes)
+  // Pinned words that a running iteration loop writes (LoopCtl::host): [0] iterations begun, [1] iterations performed
+  // once it has stopped.
+  int *progress = nullptr;
   // Launch mode of the iteration loops that replay captured HIP graphs (batched PPR, the streaming session): true =
   // captured graphs; false (PRH_GRAPH_CAPTURE=0 in the environment at context creation) = the same launches issued
   // one by one, for tools that trace kernels.
@@ -336,6 +339,21 @@ int stage_batch(prh_context *c, const prh_graph *g, const uint32_t *du, const ui
                 const uint32_t *iu, size_t ni, bool host, DevBatch &b);
 int mark_affected(prh_context *c, const prh_graph *g, int method, const DevBatch &b, const prh::ExtendArgs &xo);
 int ensure_workspace(prh_context *c, uint32_t N, bool dynamic, int L);
+// Iterations the host keeps enqueued ahead of the device in a loop over m edges (the device reports in pinned memory; a
+// copy of the flag and a wait for the stream every eight iterations took 25 us each: RMAT-10 743 -> 480 us per solve
+// without them, RMAT-16 809 -> 680 us, 1M vertices blocked 3.79 -> 3.71 ms): enough to cover the enqueueing of an
+// iteration's launches (small graphs' iterations last as long as one or two launches take to enqueue), few enough that
+// the launches left over after the loop has stopped cost little; at most check_interval.
+inline int iterations_ahead(const prh_context *c, uint64_t m) {
+  return std::max(1, std::min(c->tuning.check_interval, m < (uint64_t(1) << 22) ? 6 : 3));
+}
+void reset_progress(prh_context *c);
+// Iterations performed by a loop that has stopped, 0 while it runs.
+inline int loop_stopped(const prh_context *c) { return __atomic_load_n(c->progress + 1, __ATOMIC_ACQUIRE); }
+// Waits until the loop has begun `begun` iterations, has stopped, or nothing enqueued is left to run.
+int wait_progress(prh_context *c, int begun);
+// After the last launch of a loop: *n = its iterations (max_iter if none of them stopped it).
+int end_loop(prh_context *c, int max_iter, int *n);
 int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options *o, const uint32_t *du,
                const uint32_t *dv, size_t nd, const uint32_t *iu, size_t ni, const double *q, double *ranks,
                prh_stats *st, bool host, bool account_prep);

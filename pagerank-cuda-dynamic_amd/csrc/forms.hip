@@ -115,6 +115,7 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
   A.cols = cols;
   A.max_iter = L;
   A.N = N;
+  A.host = c->progress;
   // Initialization (timed), then iterations as replays of a captured run of check_interval iterations.
   PRH_HIP(c, hipEventRecord(c->ev[0], s));
   PRH_HIP(c, prh::launch_ppr_setup(A, d_seeds, n_seeds, d_first, g->inv, c->ppr_row.p, c->ppr_mass.p, s));
@@ -128,20 +129,13 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
   hipGraphExec_t exec = nullptr;
   int status = L > 0 && c->capture ? capture_graph(c, iterations_chunk, &exec) : PRH_SUCCESS;
   prh::PprState hs{};
-  for (int launched = 0; status == PRH_SUCCESS && launched < L; launched += chunk) {
-    hipError_t e = hipSuccess;
-    if (exec) e = hipGraphLaunch(exec, s);
-    else if ((status = iterations_chunk()) != PRH_SUCCESS) break;
-    if (e == hipSuccess) e = hipMemcpyAsync(c->pinned, c->ppr_state.p, sizeof(prh::PprState), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
+  // A run is launched when the one before it has begun its last iteration, so that the device goes on without waiting.
+  reset_progress(c);
+  for (int launched = 0; status == PRH_SUCCESS && launched < L && !loop_stopped(c); launched += chunk) {
+    if (!exec) status = iterations_chunk();
+    else if (const hipError_t e = hipGraphLaunch(exec, s); e != hipSuccess)
       status = fail(c, PRH_ERROR_DEVICE, "batched iterations: %s", hipGetErrorString(e));
-      break;
-    }
-    std::memcpy(&hs, c->pinned, sizeof(hs));
-    bool all = true;
-    for (int j = 0; j < k; ++j) all = all && hs.done[j] != 0;
-    if (all) break;
+    if (status == PRH_SUCCESS) status = wait_progress(c, std::min(L, launched + chunk));
   }
   if (exec) (void)hipGraphExecDestroy(exec);
   PRH_CHECK(status);
@@ -162,33 +156,23 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
   return PRH_SUCCESS;
 }
 
-// Up to L iterations of step(l, err, done) -- launches honouring the device stop control of iteration l -- with
-// the device flag polled every check_interval iterations. *n receives the number of iterations performed.
+// Up to L iterations of step(ctl) -- launches honouring the device stop control of iteration ctl.l -- a few of them
+// enqueued ahead of the device. *n receives the number of iterations performed.
 template <class F>
-int run_iterations(prh_context *c, int L, double tol, F step, int *n) {
+int run_iterations(prh_context *c, uint64_t M, int L, double tol, F step, int *n) {
   hipStream_t s = c->stream;
   PRH_CHECK(ensure(c, c->loop, size_t(L) + 1));
   unsigned long long *err = c->loop.p;
   int *done = reinterpret_cast<int *>(c->loop.p + L);
   PRH_HIP(c, prh::launch_fill_u64(err, 0ull, size_t(L) + 1, s));
-  const int check = std::max(1, c->tuning.check_interval);
-  int result = -1, launched = 0;
+  const int ahead = iterations_ahead(c, M);
+  reset_progress(c);
   for (int l = 0; l < L; ++l) {
-    PRH_CHECK(step(l, err, done));
-    launched = l + 1;
-    if (launched % check == 0 || launched == L) {
-      PRH_HIP(c, hipMemcpyAsync(c->pinned, err + l, 8, hipMemcpyDeviceToHost, s));
-      PRH_HIP(c, hipMemcpyAsync(c->pinned + 1, done, sizeof(int), hipMemcpyDeviceToHost, s));
-      PRH_HIP(c, hipStreamSynchronize(s));
-      double el;
-      std::memcpy(&el, c->pinned, 8);
-      const int d = *reinterpret_cast<const int *>(c->pinned + 1);
-      if (d > 0) { result = d; break; }
-      if (el < tol) { result = launched; break; }
-    }
+    PRH_CHECK(wait_progress(c, l - ahead + 1));
+    if (loop_stopped(c)) break;
+    PRH_CHECK(step(prh::LoopCtl{err, done, l, L, tol, c->progress}));
   }
-  *n = result < 0 ? launched : result;
-  return PRH_SUCCESS;
+  return end_loop(c, L, n);
 }
 
 // Device copy of a caller array: the pointer itself for device memory, else staged into `buf`.
@@ -404,12 +388,13 @@ int weighted_forward_impl(prh_context *c, const prh_graph *g, const float *w, co
     PRH_HIP(c, prh::launch_weighted_init(c->wt_terml.p, c->wt_Wl.p, N, false, c->wt_x[0].p, c->wt_z[0].p, hs));
     PRH_HIP(c, hipEventRecord(c->ev[1], hs));
     int n = 0;
-    PRH_CHECK(run_iterations(c, o->max_iterations, o->tolerance, [&](int l, unsigned long long *err, int *done) -> int {
+    PRH_CHECK(run_iterations(c, M, o->max_iterations, o->tolerance, [&](const prh::LoopCtl &ctl) -> int {
+    const int l = ctl.l;
       prh::RankArgs A{c->wt_x[(l + 1) & 1].p, c->wt_x[l & 1].p, c->wt_z[(l + 1) & 1].p, c->wt_z[l & 1].p, nullptr,
                       nullptr, g->l_in_off, g->l_in_src, nullptr, 0.0, o->damping, 0.0, 0.0, nullptr};
       A.term = c->wt_terml.p;
       A.W = c->wt_Wl.p;
-      PRH_HIP(c, prh::launch_binned_update(prh::kWeightedForward, A, plan, err, done, l, o->tolerance, false, hs));
+      PRH_HIP(c, prh::launch_binned_update(prh::kWeightedForward, A, plan, ctl, false, hs));
       return PRH_SUCCESS;
     }, &n));
     PRH_HIP(c, hipEventRecord(c->ev[2], hs));
@@ -429,7 +414,8 @@ int weighted_forward_impl(prh_context *c, const prh_graph *g, const float *w, co
   PRH_HIP(c, prh::launch_weighted_init(c->wt_terml.p, c->wt_Wl.p, N, false, c->wt_x[0].p, c->wt_z[0].p, hs));
   PRH_HIP(c, hipEventRecord(c->ev[1], hs));
   int n = 0;
-  PRH_CHECK(run_iterations(c, o->max_iterations, o->tolerance, [&](int l, unsigned long long *err, int *done) -> int {
+  PRH_CHECK(run_iterations(c, M, o->max_iterations, o->tolerance, [&](const prh::LoopCtl &ctl) -> int {
+    const int l = ctl.l;
     prh::WeightedArgs A = A0;
     A.off = g->l_in_off;
     A.idx = g->l_in_src;
@@ -441,7 +427,7 @@ int weighted_forward_impl(prh_context *c, const prh_graph *g, const float *w, co
     A.term = c->wt_terml.p;
     A.W = c->wt_Wl.p;
     A.P = o->damping;
-    PRH_HIP(c, prh::launch_weighted_step(false, A, err, done, l, o->tolerance, hs));
+    PRH_HIP(c, prh::launch_weighted_step(false, A, ctl, hs));
     return PRH_SUCCESS;
   }, &n));
   PRH_HIP(c, hipEventRecord(c->ev[2], hs));
@@ -487,14 +473,15 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
   PRH_HIP(c, prh::launch_weighted_init(c->wt_terml.p, c->wt_Wl.p, N, true, c->wt_x[0].p, c->wt_z[0].p, hs));
   PRH_HIP(c, hipEventRecord(c->ev[1], hs));
   int n = 0;
-  PRH_CHECK(run_iterations(c, o->max_iterations, o->tolerance, [&](int l, unsigned long long *err, int *done) -> int {
+  PRH_CHECK(run_iterations(c, M, o->max_iterations, o->tolerance, [&](const prh::LoopCtl &ctl) -> int {
+    const int l = ctl.l;
     if (blocked) {  // lam_new = g + (P / W) * sum over out-edges of w * lam_old, gathered straight from lam_old
       double *x_new = c->wt_x[(l + 1) & 1].p, *x_old = c->wt_x[l & 1].p;
       prh::RankArgs A{x_new, x_old, x_new, x_old, nullptr, nullptr, g->l_out_off, g->l_out_dst, nullptr,
                       0.0, o->damping, 0.0, 0.0, nullptr};
       A.term = c->wt_terml.p;
       A.W = c->wt_Wl.p;
-      PRH_HIP(c, prh::launch_binned_update(prh::kWeightedAdjoint, A, plan, err, done, l, o->tolerance, false, hs));
+      PRH_HIP(c, prh::launch_binned_update(prh::kWeightedAdjoint, A, plan, ctl, false, hs));
       return PRH_SUCCESS;
     }
     prh::WeightedArgs A = A0;
@@ -508,7 +495,7 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
     A.term = c->wt_terml.p;
     A.W = c->wt_Wl.p;
     A.P = o->damping;
-    PRH_HIP(c, prh::launch_weighted_step(true, A, err, done, l, o->tolerance, hs));
+    PRH_HIP(c, prh::launch_weighted_step(true, A, ctl, hs));
     return PRH_SUCCESS;
   }, &n));
   // The gradients are computed in the caller's order, from the caller's CSR: only lambda goes back from the layout's.

@@ -306,14 +306,13 @@ hipError_t launch_mark_partial(uint8_t *naff, uint8_t *vaff, const uint32_t *del
   return hipGetLastError();
 }
 
-hipError_t launch_extend(const ExtendArgs &A, unsigned long long *err, int *done, int l, double tol, hipStream_t s) {
+hipError_t launch_extend(const ExtendArgs &A, const LoopCtl &ctl, hipStream_t s) {
   const uint32_t nb_high =
       clamp_blocks(size_t(A.sched.n_high) + (A.chunk_row ? 0u : A.sched.n_huge), kWavesPerBlock, 4096);
   const uint32_t nb_low = clamp_blocks(A.sched.n_low, kBlock / kLowLanes, 8192);
   const uint32_t nb_chunk = A.chunk_row ? clamp_blocks(A.n_chunks, kWavesPerBlock, 4096) : 0u;
   if (nb_high + nb_low + nb_chunk == 0) return hipSuccess;
-  const LoopCtl ctl{err, done, l, tol};
-  extend_kernel<<<nb_high + nb_low + nb_chunk, kBlock, 0, s>>>(A, nb_high, nb_low, ctl, err ? 1 : 0);
+  extend_kernel<<<nb_high + nb_low + nb_chunk, kBlock, 0, s>>>(A, nb_high, nb_low, ctl, ctl.err ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -343,20 +342,16 @@ hipError_t launch_extend_batch_keys(uint8_t *vaff, uint8_t *naff, const unsigned
   return hipGetLastError();
 }
 
-hipError_t launch_direction(const double *stats, uint32_t n, int *direction, unsigned long long *err, int *done, int l,
-                            double tol, hipStream_t s) {
-  const LoopCtl ctl{err, done, l, tol};
+hipError_t launch_direction(const double *stats, uint32_t n, int *direction, const LoopCtl &ctl, hipStream_t s) {
   direction_kernel<<<1, kDirThreads, 0, s>>>(stats, n, direction, ctl);
   return hipGetLastError();
 }
 
-hipError_t launch_extend_pull(const PullArgs &A, unsigned long long *err, int *done, int l, double tol,
-                              hipStream_t s) {
+hipError_t launch_extend_pull(const PullArgs &A, const LoopCtl &ctl, hipStream_t s) {
   const uint32_t nb_wave = clamp_blocks(A.n_wave, kWavesPerBlock, 2048);
   const uint32_t nb_group = clamp_blocks(size_t(A.n_group) - A.n_wave, kBlock / kPullLanes, 4096);
   const uint32_t nb_one = clamp_blocks(size_t(A.N) - A.n_group, kBlock, 4096);
   if (nb_wave + nb_group + nb_one == 0) return hipSuccess;
-  const LoopCtl ctl{err, done, l, tol};
   extend_pull_kernel<<<nb_wave + nb_group + nb_one, kBlock, 0, s>>>(A, nb_wave, nb_group, nb_one, ctl);
   return hipGetLastError();
 }

@@ -215,6 +215,7 @@ __global__ __launch_bounds__(kBlock, KT >= 16 ? 8 : 1) void ppr_gather_kernel(Pp
         for (int k = 0; k < S::kVec; ++k) p[k] = s.x[k];
       }
     }
+    if (!FINAL && blockIdx.x == 0 && threadIdx.x == 0) tell_host(A.host, q.l + 1);
     return;
   }
   b -= nb_chunk;
@@ -240,7 +241,10 @@ __global__ __launch_bounds__(kBlock, KT >= 16 ? 8 : 1) void ppr_gather_kernel(Pp
       finish_row<KT, FINAL>(A, q, v, row, s, out, emax);
     }
   }
-  if constexpr (!FINAL) report_columns<KT>(A, q, emax);
+  if constexpr (!FINAL) {
+    report_columns<KT>(A, q, emax);
+    if (blockIdx.x == 0 && threadIdx.x == 0) tell_host(A.host, q.l + 1);
+  }
 }
 
 // Heavy rows: add the chunk partials (lane group g takes chunks g, g + groups, ...) and finish.
@@ -265,12 +269,18 @@ __global__ __launch_bounds__(kBlock) void ppr_combine_kernel(PprArgs A, int step
 }
 
 // After a run of `steps` iterations: the columns whose last one was below the tolerance are done; the next run's index.
+// Tells the host how far it is, and when no column is left.
 __global__ __launch_bounds__(kWave) void ppr_advance_kernel(PprArgs A, int steps) {
   const int j = threadIdx.x, l = A.state->iter + steps - 1;
-  if (j < A.k && l < A.max_iter && A.state->done[j] == 0 &&
-      __longlong_as_double((long long)A.err[size_t(l) * kPprCols + j]) < A.tol)
-    A.state->done[j] = l + 1;
-  if (j == 0) A.state->iter = l + 1;
+  int d = j < A.k ? A.state->done[j] : 1;
+  if (d == 0 && l < A.max_iter && __longlong_as_double((long long)A.err[size_t(l) * kPprCols + j]) < A.tol)
+    A.state->done[j] = d = l + 1;
+  const bool all = __ballot(d == 0) == 0;
+  if (j == 0) {
+    A.state->iter = l + 1;
+    if (all) tell_host(A.host + 1, 1);
+    else tell_host(A.host, l + 1);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void ppr_reset_kernel(PprArgs A, int32_t *seed_row, double *mass, size_t rows) {

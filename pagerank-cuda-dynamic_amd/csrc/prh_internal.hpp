@@ -11,10 +11,15 @@ constexpr int kWave = 64;    // CDNA wavefront width
 constexpr int kBlock = 256;  // every kernel here runs 4 waves per workgroup
 constexpr int kWavesPerBlock = kBlock / kWave;
 
-// Device view of a loop's convergence state (see LoopCtl in prh_device.hpp).
-struct LoopState {
-  unsigned long long *err;  // [capacity] per-iteration L-inf bits
-  int *done;                // single int
+// Control of an iteration loop on the device (see prh_device.hpp).
+struct LoopCtl {
+  unsigned long long *err;  // [max iterations] FP64 bits, zeroed before the loop: 0 or kChanged
+  int *done;                // 0 while running, else the number of iterations performed
+  int l;                    // this launch's iteration index, or -1 - i: index done[1] + i (replayed graphs, where the
+                            // same launch serves many iterations and a device word holds the run's first index)
+  int max_iter;             // iterations from this index on do nothing
+  double tol;
+  int *host;                // pinned host memory, or null: [0] iterations begun, [1] iterations performed once stopped
 };
 
 // Solver variant bits, as the reference's template switches <DYNAMIC, FRONTIER, PRUNE>
@@ -224,12 +229,12 @@ inline uint32_t finish_chunked_grid(uint32_t n_chunked) {
 }
 // Rank update of iteration l: the rank kernel, then (if the plan has chunked rows) their combining kernel. `mark`,
 // when non-null, is recorded between the two, so that it times the rank kernel alone.
-hipError_t launch_rank_update(int variant, const RankArgs &A, const RankPlan &plan, unsigned long long *err,
-                              int *done, int l, double tol, hipStream_t s, hipEvent_t mark = nullptr);
+hipError_t launch_rank_update(int variant, const RankArgs &A, const RankPlan &plan, const LoopCtl &ctl, hipStream_t s,
+                              hipEvent_t mark = nullptr);
 // Plain update through the source-sliced plan: the gather launch, then the finish launch; `mark` (optional) is
 // recorded between them.
-hipError_t launch_sliced_update(const RankArgs &A, const SlicedPlan &plan, unsigned long long *err, int *done, int l,
-                                double tol, hipStream_t s, hipEvent_t mark = nullptr);
+hipError_t launch_sliced_update(const RankArgs &A, const SlicedPlan &plan, const LoopCtl &ctl, hipStream_t s,
+                                hipEvent_t mark = nullptr);
 hipError_t launch_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t s);
 hipError_t launch_fill_u8(uint8_t *p, uint8_t v, size_t n, hipStream_t s);
 hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, size_t n, hipStream_t s);
@@ -249,11 +254,10 @@ hipError_t launch_gather_ranges(const uint32_t *off, const uint32_t *ids, size_t
 // (frontier variants, every iteration after the first): the extension of the previous iteration's frontier
 // (A.naff) happens inside this update, so no separate extension launch follows it. `mark`, when non-null, is
 // recorded after the last kernel.
-hipError_t launch_binned_update(int variant, const RankArgs &A, const BinnedPlan &P, unsigned long long *err,
-                                int *done, int l, double tol, bool extend, hipStream_t s, hipEvent_t mark = nullptr);
+hipError_t launch_binned_update(int variant, const RankArgs &A, const BinnedPlan &P, const LoopCtl &ctl, bool extend,
+                                hipStream_t s, hipEvent_t mark = nullptr);
 // Rank update of iteration l through the banded plan (window.hip); unweighted variants only.
-hipError_t launch_window_update(int variant, const RankArgs &A, const WindowPlan &W, unsigned long long *err, int *done,
-                                int l, double tol, hipStream_t s);
+hipError_t launch_window_update(int variant, const RankArgs &A, const WindowPlan &W, const LoopCtl &ctl, hipStream_t s);
 // *out = the largest |source - destination| over the in-CSR's edges.
 hipError_t launch_max_spread(const uint32_t *off, const uint32_t *src, uint32_t N, uint32_t *out, hipStream_t s);
 // In-place update of a plan (see binned.hip): dead flags and fresh overlay entries from a batch's tidied in-CSR keys
@@ -345,6 +349,7 @@ struct PprArgs {
   int tile, cols;                   // columns per tile, and of all tiles
   int max_iter;
   uint32_t N;
+  int *host;                        // pinned host memory: [0] iterations begun, [1] 1 once every column is done
 };
 
 // Start of a call: state cleared, the seed table built from `seeds` (the columns' seed sets, column j's being
@@ -384,8 +389,7 @@ struct WeightedArgs {
 constexpr uint32_t kWeightedChunk = 4096;
 
 // One Jacobi step: the chunk sums, the wave rows, the low-row bands, then (with chunks) the heavy rows' finish.
-hipError_t launch_weighted_step(bool adjoint, const WeightedArgs &A, unsigned long long *err, int *done, int l,
-                                double tol, hipStream_t s);
+hipError_t launch_weighted_step(bool adjoint, const WeightedArgs &A, const LoopCtl &ctl, hipStream_t s);
 // key[i] = 64 - degree of row order[i], for the first n rows (degrees <= 64).
 hipError_t launch_degree_keys(const uint32_t *off, const uint32_t *order, uint32_t n, uint32_t *key, hipStream_t s);
 // Out-weight sums. order, counts (device): the rows partitioned by out-degree at kSumLane and kSumWave.
@@ -477,7 +481,7 @@ hipError_t launch_refresh_chunks(const uint32_t *item_row, const uint32_t *row_f
                                  hipStream_t s);
 hipError_t launch_mark_batch(uint8_t *naff, uint8_t *vaff, const unsigned long long *dkeys, const uint32_t *nd,
                              const unsigned long long *ikeys, const uint32_t *ni, uint32_t cap_total, hipStream_t s);
-hipError_t launch_advance(int *l, int *done, const unsigned long long *err, double tol, int max_iter, hipStream_t s);
+hipError_t launch_advance(const LoopCtl &ctl, int n, hipStream_t s);
 // Device-driven traversal closure (lvl: [0] level, [1] stop, [2], [3] changed flags of even and odd levels): the
 // step before a level stops the closure when the previous level marked nothing, else clears this level's flag; the
 // advance after it moves to the next level unless stopped.
@@ -502,13 +506,10 @@ hipError_t launch_extend_batch_keys(uint8_t *vaff, uint8_t *naff, const unsigned
                                     const unsigned long long *ik, const uint32_t *ni, uint32_t cap,
                                     const uint32_t *off, const uint32_t *dst, uint32_t *cnt, uint32_t *start,
                                     void *tmp, size_t &tmp_bytes, hipStream_t s);
-hipError_t launch_extend(const ExtendArgs &A, unsigned long long *err, int *done, int l, double tol,
-                         hipStream_t s);
+hipError_t launch_extend(const ExtendArgs &A, const LoopCtl &ctl, hipStream_t s);
 // Sums the per-workgroup costs the rank launches left in stats[0 .. 2 n) and sets *direction to 1 (pull) when
 // pulling is cheaper, else 0 (push). Honours iteration l's control like the extension.
-hipError_t launch_direction(const double *stats, uint32_t n, int *direction, unsigned long long *err, int *done, int l,
-                            double tol, hipStream_t s);
-hipError_t launch_extend_pull(const PullArgs &A, unsigned long long *err, int *done, int l, double tol,
-                              hipStream_t s);
+hipError_t launch_direction(const double *stats, uint32_t n, int *direction, const LoopCtl &ctl, hipStream_t s);
+hipError_t launch_extend_pull(const PullArgs &A, const LoopCtl &ctl, hipStream_t s);
 
 }  // namespace prh

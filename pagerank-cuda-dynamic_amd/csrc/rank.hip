@@ -272,6 +272,7 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
   __shared__ double lds_cost[2 * kWavesPerBlock];
   store_costs<VARIANT>(A, cost, blockIdx.x, lds_cost);
   report_change(ctl, emax);
+  report_begun(ctl);
 }
 
 // Chunked rows, after the rank kernel of the same iteration: one wave per row adds the row's chunk partials (in a
@@ -424,6 +425,7 @@ __global__ __launch_bounds__(kBlock) void sliced_finish_kernel(RankArgs A, Slice
     }
   }
   report_change(ctl, emax);
+  report_begun(ctl);
 }
 
 // r = a = 1/N (or keep r as loaded and copy it to a); contributions cr = ca = r/deg.
@@ -509,10 +511,9 @@ inline uint32_t map_grid(size_t n) {
 
 }  // namespace
 
-hipError_t launch_rank_update(int variant, const RankArgs &A, const RankPlan &P, unsigned long long *err, int *done,
-                              int l, double tol, hipStream_t s, hipEvent_t mark) {
+hipError_t launch_rank_update(int variant, const RankArgs &A, const RankPlan &P, const LoopCtl &ctl, hipStream_t s,
+                              hipEvent_t mark) {
   if (P.blocks == 0) return mark ? hipEventRecord(mark, s) : hipSuccess;
-  const LoopCtl ctl{err, done, l, tol};
   switch (variant) {
     case kPlain: return launch_variant<kPlain>(A, P, ctl, s, mark);
     case kTraversal: return launch_variant<kTraversal>(A, P, ctl, s, mark);
@@ -522,9 +523,8 @@ hipError_t launch_rank_update(int variant, const RankArgs &A, const RankPlan &P,
   }
 }
 
-hipError_t launch_sliced_update(const RankArgs &A, const SlicedPlan &P, unsigned long long *err, int *done, int l,
-                                double tol, hipStream_t s, hipEvent_t mark) {
-  const LoopCtl ctl{err, done, l, tol};
+hipError_t launch_sliced_update(const RankArgs &A, const SlicedPlan &P, const LoopCtl &ctl, hipStream_t s,
+                                hipEvent_t mark) {
   const uint32_t gather_blocks = P.blocks_per_slice * uint32_t(P.slices);
   if (gather_blocks) sliced_gather_kernel<<<gather_blocks, kBlock, 0, s>>>(P, A.cr, ctl);
   if (mark) {

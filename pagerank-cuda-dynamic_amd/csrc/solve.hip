@@ -1,9 +1,9 @@
 // solve.hip -- the solver driver: restates pagerankInvokeCuda + pagerankLoopCuU (pagerankCuda.hxx:675-692,
 // :713-849) for one HIP stream. Per repeat, partition (and initial ranks) = initialization time, affected marking =
 // marking time, iterations = computation time, each measured with HIP events. Iterations run without a host
-// round trip per iteration: convergence is detected on the device (LoopCtl), and the host polls the device flag
-// only every check_interval iterations, so the iteration count and final ranks equal those of the per-iteration
-// check.
+// round trip per iteration: convergence is detected on the device (LoopCtl), the device tells the host in pinned memory
+// how far it is, and the host keeps a few iterations enqueued ahead of it until the device says it has stopped, so the
+// iteration count and final ranks equal those of the per-iteration check.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -83,12 +83,45 @@ int mark_affected(prh_context *c, const prh_graph *g, int method, const DevBatch
     T.fresh = fresh;
     T.changed = c->flags.p + 1;
     T.direction = nullptr;
-    PRH_HIP(c, prh::launch_extend(T, nullptr, nullptr, 0, 0.0, s));
+    PRH_HIP(c, prh::launch_extend(T, prh::LoopCtl{}, s));
     PRH_HIP(c, hipMemcpyAsync(c->pinned, c->flags.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     PRH_HIP(c, hipStreamSynchronize(s));
     if (*reinterpret_cast<int *>(c->pinned) == 0) break;
     std::swap(front, fresh);
   }
+  return PRH_SUCCESS;
+}
+
+void reset_progress(prh_context *c) {
+  __atomic_store_n(c->progress, 0, __ATOMIC_RELAXED);
+  __atomic_store_n(c->progress + 1, 0, __ATOMIC_RELEASE);
+}
+
+int wait_progress(prh_context *c, int begun) {
+  using clock = std::chrono::steady_clock;
+  const auto wait = std::chrono::milliseconds(100);
+  clock::time_point next;
+  for (unsigned i = 1; !loop_stopped(c) && __atomic_load_n(c->progress, __ATOMIC_ACQUIRE) < begun; ++i) {
+    if (i % 1024) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    // Long iterations, or launches that failed: ask the stream now and then (a query adds a marker to it).
+    const auto now = clock::now();
+    if (i == 1024) next = now + wait;
+    if (now < next) continue;
+    next = now + wait;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipSuccess) break;
+    if (e != hipErrorNotReady) return fail(c, PRH_ERROR_DEVICE, "iterations: %s", hipGetErrorString(e));
+  }
+  return PRH_SUCCESS;
+}
+
+int end_loop(prh_context *c, int max_iter, int *n) {
+  if (!loop_stopped(c)) PRH_HIP(c, hipStreamSynchronize(c->stream));
+  const int k = loop_stopped(c);
+  *n = k ? k : max_iter;
   return PRH_SUCCESS;
 }
 
@@ -190,7 +223,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   int iterations = 0;
   unsigned long long *err = c->loop.p;
   int *done = reinterpret_cast<int *>(c->loop.p + L);
-  const int check = std::max(1, c->tuning.check_interval);
+  const int ahead = iterations_ahead(c, g->M);
   const prh::RankPlan &plan = g->plan;
   // Extension direction (frontier variants): 0 push only, 1 chosen per iteration from the rank launch's costs,
   // 2 pull only. The pull form splits rows at in-degree 64 (a wave each) and 4 (8 lanes each).
@@ -229,23 +262,25 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     if (frontier && dir_mode != 1) PRH_HIP(c, prh::launch_fill_i32(dir, dir_mode == 2 ? 1 : 0, 1, s));
     const double P = o->damping;
     const double C0 = (1 - P) / N;
-    int n = -1, launched = 0;
+    reset_progress(c);
     for (int l = 0; l < L; ++l) {
+      PRH_CHECK(wait_progress(c, l - ahead + 1));
+      if (loop_stopped(c)) break;
+      const prh::LoopCtl ctl{err, done, l, L, o->tolerance, c->progress};
       prh::RankArgs A{c->rank[(l + 1) & 1].p, c->rank[l & 1].p, c->contrib[(l + 1) & 1].p, c->contrib[l & 1].p,
                       c->naff.p, c->vaff.p, g->l_in_off, g->l_in_src, g->l_outdeg, C0, P, o->frontier_tolerance,
                       o->prune_tolerance, dir_auto ? c->ext_stats.p : nullptr};
       if (c->ktiming) PRH_HIP(c, hipEventRecord(c->kev[2 * l], s));
       hipEvent_t mark = c->ktiming ? c->kev[2 * l + 1] : nullptr;
       if (binned)
-        PRH_HIP(c, prh::launch_binned_update(variant, A, g->bin.plan, err, done, l, o->tolerance, frontier && l > 0, s,
-                                             mark));
+        PRH_HIP(c, prh::launch_binned_update(variant, A, g->bin.plan, ctl, frontier && l > 0, s, mark));
       else if (window) {
-        PRH_HIP(c, prh::launch_window_update(variant, A, g->win, err, done, l, o->tolerance, s));
+        PRH_HIP(c, prh::launch_window_update(variant, A, g->win, ctl, s));
         if (mark) PRH_HIP(c, hipEventRecord(mark, s));
-      } else if (sliced) PRH_HIP(c, prh::launch_sliced_update(A, g->sliced, err, done, l, o->tolerance, s, mark));
-      else PRH_HIP(c, prh::launch_rank_update(variant, A, plan, err, done, l, o->tolerance, s, mark));
+      } else if (sliced) PRH_HIP(c, prh::launch_sliced_update(A, g->sliced, ctl, s, mark));
+      else PRH_HIP(c, prh::launch_rank_update(variant, A, plan, ctl, s, mark));
       if (frontier && !binned) {  // the blocked plan extends inside the next iteration's update
-        if (dir_auto) PRH_HIP(c, prh::launch_direction(c->ext_stats.p, stat_slots, dir, err, done, l, o->tolerance, s));
+        if (dir_auto) PRH_HIP(c, prh::launch_direction(c->ext_stats.p, stat_slots, dir, ctl, s));
         prh::ExtendArgs E = xo;
         E.vaff = c->vaff.p;
         E.naff = c->naff.p;
@@ -254,24 +289,14 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
         E.fresh = nullptr;
         E.changed = nullptr;
         E.direction = dir;
-        PRH_HIP(c, prh::launch_extend(E, err, done, l, o->tolerance, s));
-        if (dir_mode != 0) PRH_HIP(c, prh::launch_extend_pull(pull, err, done, l, o->tolerance, s));
-      }
-      launched = l + 1;
-      if (launched % check == 0 || launched == L) {
-        PRH_HIP(c, hipMemcpyAsync(c->pinned, err + l, 8, hipMemcpyDeviceToHost, s));
-        PRH_HIP(c, hipMemcpyAsync(c->pinned + 1, done, sizeof(int), hipMemcpyDeviceToHost, s));
-        PRH_HIP(c, hipStreamSynchronize(s));
-        double el;
-        std::memcpy(&el, c->pinned, 8);
-        const int d = *reinterpret_cast<const int *>(c->pinned + 1);
-        if (d > 0) { n = d; break; }
-        if (el < o->tolerance) { n = launched; break; }
+        PRH_HIP(c, prh::launch_extend(E, ctl, s));
+        if (dir_mode != 0) PRH_HIP(c, prh::launch_extend_pull(pull, ctl, s));
       }
     }
-    if (n < 0) n = launched;
     PRH_HIP(c, hipEventRecord(c->ev[3], s));
     PRH_HIP(c, hipEventSynchronize(c->ev[3]));
+    int n = 0;
+    PRH_CHECK(end_loop(c, L, &n));
     float t01 = 0, t12 = 0, t23 = 0;
     PRH_HIP(c, hipEventElapsedTime(&t01, c->ev[0], c->ev[1]));
     PRH_HIP(c, hipEventElapsedTime(&t12, c->ev[1], c->ev[2]));

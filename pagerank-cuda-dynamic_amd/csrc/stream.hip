@@ -454,14 +454,15 @@ __global__ __launch_bounds__(kBlock) void copy_u8_kernel(uint8_t *dst, const uin
   for (size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += size_t(gridDim.x) * kBlock) dst[i] = src[i];
 }
 
-// After iteration l's launches: stop when its L-inf change is below tolerance (done = l + 1 iterations) or when
-// the iteration cap is reached; otherwise move to iteration l + 1.
-__global__ void advance_kernel(int *l, int *done, const unsigned long long *err, double tol, int max_iter) {
-  if (*done) return;
-  const int i = *l;
-  const double e = __longlong_as_double((long long)err[i]);
-  if (e < tol || i + 1 >= max_iter) *done = i + 1;
-  else *l = i + 1;
+// After a run of n iterations from index done[1]: stopped when the last one's change was below tolerance or the cap is
+// reached (the iterations themselves see to the ones before it); otherwise the next run's first index.
+__global__ void advance_kernel(LoopCtl ctl, int n) {
+  if (*ctl.done) return;
+  const int next = ctl.done[1] + n, last = next - 1;
+  if (last >= ctl.max_iter) *ctl.done = ctl.max_iter;
+  else if (__longlong_as_double((long long)ctl.err[last]) < ctl.tol || next >= ctl.max_iter) *ctl.done = next;
+  else ctl.done[1] = next;
+  if (*ctl.done && ctl.host) tell_host(ctl.host + 1, *ctl.done);
 }
 
 }  // namespace
@@ -587,8 +588,8 @@ hipError_t launch_copy_u8(uint8_t *dst, const uint8_t *src, size_t n, hipStream_
   return hipGetLastError();
 }
 
-hipError_t launch_advance(int *l, int *done, const unsigned long long *err, double tol, int max_iter, hipStream_t s) {
-  advance_kernel<<<1, 1, 0, s>>>(l, done, err, tol, max_iter);
+hipError_t launch_advance(const LoopCtl &ctl, int n, hipStream_t s) {
+  advance_kernel<<<1, 1, 0, s>>>(ctl, n);
   return hipGetLastError();
 }
 

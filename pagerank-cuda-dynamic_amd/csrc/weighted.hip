@@ -91,6 +91,7 @@ __global__ __launch_bounds__(kBlock) void weighted_step_kernel(WeightedArgs A, u
     if (lane == 0) lds[w] = s;
     __syncthreads();
     if (threadIdx.x == 0) A.partial[blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+    report_begun(ctl);
     return;
   }
   const uint32_t b = blockIdx.x - A.n_chunks;
@@ -121,6 +122,7 @@ __global__ __launch_bounds__(kBlock) void weighted_step_kernel(WeightedArgs A, u
     }
   }
   report_change(ctl, emax);
+  report_begun(ctl);
 }
 
 // Heavy rows, after the step of the same iteration: a wave per row adds its chunk sums in chunk order.
@@ -353,9 +355,7 @@ hipError_t launch_step(const WeightedArgs &A, const LoopCtl &ctl, hipStream_t s)
 
 }  // namespace
 
-hipError_t launch_weighted_step(bool adjoint, const WeightedArgs &A, unsigned long long *err, int *done, int l,
-                                double tol, hipStream_t s) {
-  const LoopCtl ctl{err, done, l, tol};
+hipError_t launch_weighted_step(bool adjoint, const WeightedArgs &A, const LoopCtl &ctl, hipStream_t s) {
   return adjoint ? launch_step<true>(A, ctl, s) : launch_step<false>(A, ctl, s);
 }
 

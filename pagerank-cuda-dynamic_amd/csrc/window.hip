@@ -144,6 +144,7 @@ __global__ __launch_bounds__(kBinBlock) void window_update_kernel(RankArgs A, Wi
   }
   wg_store_costs<VARIANT, kWinWaves>(A, cost, blockIdx.x, lds_cost);
   report_change(ctl, emax);
+  report_begun(ctl);
 }
 
 template <int S>
@@ -174,9 +175,7 @@ __global__ __launch_bounds__(kBlock) void max_spread_kernel(const uint32_t *off,
 
 }  // namespace
 
-hipError_t launch_window_update(int variant, const RankArgs &A, const WindowPlan &W, unsigned long long *err,
-                                int *done, int l, double tol, hipStream_t s) {
-  const LoopCtl ctl{err, done, l, tol};
+hipError_t launch_window_update(int variant, const RankArgs &A, const WindowPlan &W, const LoopCtl &ctl, hipStream_t s) {
   switch (W.S) {
     case kWindowRingSmall: return window_variant<kWindowRingSmall>(variant, A, W, ctl, s);
     case kWindowRingLarge: return window_variant<kWindowRingLarge>(variant, A, W, ctl, s);
