@@ -27,6 +27,8 @@
 // LDS additions are made in arrival order, so the sums repeat only to rounding, not bit for bit. Every vertex gets
 // its full in-sum; the update from it is the other plans' (update.hpp), so the dynamic variants carry unaffected
 // vertices over and set their prune and frontier flags as the row kernel does.
+#include <algorithm>
+
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
 
@@ -99,15 +101,56 @@ __device__ __forceinline__ double contrib1(const double *cr, const double *r, co
   else return cr[v];
 }
 
+// The overlay's values for this iteration (the launch's last workgroups): entry i takes its source's contribution,
+// negated when the source was in the last frontier, as X does. The entry count is ov_off[bins].
+template <bool FROM_RANKS>
+__device__ __forceinline__ void overlay_expand(const BinnedPlan &P, const double *cr, const double *r,
+                                               const uint32_t *deg, const uint8_t *naff, uint32_t block,
+                                               uint32_t blocks) {
+  const uint32_t n = P.ov_off[(P.N + P.B - 1) / P.B];
+  for (uint32_t i = block * kBinBlock + threadIdx.x; i < n; i += blocks * kBinBlock) {
+    const uint32_t u = uint32_t(P.ov_key[i]);
+    const double c = contrib1<FROM_RANKS>(cr, r, deg, u);
+    P.ovX[i] = naff && naff[u] ? -c : c;
+  }
+}
+
 template <int B, bool FROM_RANKS>
 __global__ __launch_bounds__(kBinBlock) void expand_kernel(BinnedPlan P, const double *cr, const double *r,
                                                            const uint32_t *deg, const uint8_t *naff, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
   if (iter_index(ctl) == 0) naff = nullptr;  // the first iteration extends nothing (the marking did)
+  if (blockIdx.x >= P.n_ex) {
+    overlay_expand<FROM_RANKS>(P, cr, r, deg, naff, blockIdx.x - P.n_ex, gridDim.x - P.n_ex);
+    report_begun(ctl);
+    return;
+  }
   __shared__ double c[B];
   const uint4 it = P.ex_item[blockIdx.x];  // block, first entry, end entry
   const uint32_t base = it.x * uint32_t(B);
   const uint32_t n = min(uint32_t(B), P.N - base);
+  // Pairs of entries: thread t takes pairs p = t + m * kBinBlock of the even-aligned range (16-byte stores, with the
+  // non-temporal hint: X is read back only by the next kernel, and keeping it out of L2 helps both); a lone first
+  // or last entry is written on its own. A batch is eight source-id loads per lane before their stores (four: 4351
+  // against 4229 us per update at 2.04B edges); the first one, an item's only one as a rule, is loaded before the block's
+  // contributions, so that the item waits for memory once less (RMAT-20: 18.0 -> 16.2 us, RMAT-24: 235 -> 231 us).
+  const uint32_t k0 = it.y + (it.y & 1u), k1 = max(k0, it.z & ~1u);
+  const uint32_t *s32 = reinterpret_cast<const uint32_t *>(P.src16);
+  d2 *x2 = reinterpret_cast<d2 *>(P.X);
+  const uint32_t p1 = k1 / 2;
+  uint32_t p = k0 / 2 + threadIdx.x;
+  uint32_t a[8];
+  auto ids = [&]() {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = p + u * kBinBlock < p1 ? __builtin_nontemporal_load(s32 + p + u * kBinBlock) : 0u;
+  };
+  auto entries = [&]() {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (p + u * kBinBlock < p1)
+        __builtin_nontemporal_store(d2{c[a[u] & 0xFFFFu], c[a[u] >> 16]}, x2 + p + u * kBinBlock);
+  };
+  ids();
   // Pairs of contributions a lane (base is a multiple of B, so the pairs are 16-byte aligned); an odd n leaves one.
   if (naff) {
     const uint16_t *f2 = reinterpret_cast<const uint16_t *>(naff + base);
@@ -129,35 +172,14 @@ __global__ __launch_bounds__(kBinBlock) void expand_kernel(BinnedPlan P, const d
     c[n - 1] = naff && naff[base + n - 1] ? -x : x;
   }
   __syncthreads();
-  // Pairs of entries: thread t takes pairs p = t + m * kBinBlock of the even-aligned range (16-byte stores, with the
-  // non-temporal hint: X is read back only by the next kernel, and keeping it out of L2 helps both); a lone first
-  // or last entry is written on its own.
-  uint32_t k0 = it.y, k1 = it.z;
-  if (k0 & 1u) {
-    if (threadIdx.x == 0) P.X[k0] = c[ld_nt(P.src16 + k0)];
-    ++k0;
+  if (threadIdx.x == 0) {
+    if (k0 > it.y && it.y < it.z) P.X[it.y] = c[ld_nt(P.src16 + it.y)];
+    if (it.z > k1) P.X[it.z - 1] = c[ld_nt(P.src16 + it.z - 1)];
   }
-  if (k1 > k0 && (k1 & 1u)) {
-    if (threadIdx.x == 0) P.X[k1 - 1] = c[ld_nt(P.src16 + k1 - 1)];
-    --k1;
-  }
-  const uint32_t *s32 = reinterpret_cast<const uint32_t *>(P.src16);
-  d2 *x2 = reinterpret_cast<d2 *>(P.X);
-  const uint32_t p0 = k0 / 2, p1 = k1 / 2;
-  uint32_t p = p0 + threadIdx.x;
-  // Eight source-id loads in flight per lane before their stores (four: 4351 against 4229 us per update at 2.04B
-  // edges).
-  for (; p + 7 * kBinBlock < p1; p += 8 * kBinBlock) {
-    uint32_t a[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = __builtin_nontemporal_load(s32 + p + u * kBinBlock);
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      __builtin_nontemporal_store(d2{c[a[u] & 0xFFFFu], c[a[u] >> 16]}, x2 + p + u * kBinBlock);
-  }
-  for (; p < p1; p += kBinBlock) {
-    const uint32_t a = __builtin_nontemporal_load(s32 + p);
-    __builtin_nontemporal_store(d2{c[a & 0xFFFFu], c[a >> 16]}, x2 + p);
+  entries();
+  for (p += 8 * kBinBlock; p < p1; p += 8 * kBinBlock) {
+    ids();
+    entries();
   }
   report_begun(ctl);
 }
@@ -292,7 +314,7 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
     }
   }
   // Edges an in-place update inserted outside the plan (the overlay, sorted by destination): the bin's first item
-  // adds them, each with its source's value that overlay_expand_kernel wrote this iteration (negative: a frontier
+  // adds them, each with its source's value that expand wrote this iteration (negative: a frontier
   // source, as in X).
   if (P.ov_n && (blockIdx.x == 0 || P.ac_item[blockIdx.x - 1].x != it.x)) {
     const uint32_t o1 = P.ov_off[it.x + 1];
@@ -389,34 +411,16 @@ __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, Binn
   report_change(ctl, emax);
 }
 
-// The overlay's values for this iteration: entry i takes its source's contribution, negated when the source was in
-// the last frontier (naff, frontier variants after their first iteration), as expand does for X. It runs between
-// expand and accumulate: accumulate overwrites naff with the new frontier. The entry count is ov_off[bins].
-template <bool FROM_RANKS>
-__global__ __launch_bounds__(kBlock) void overlay_expand_kernel(BinnedPlan P, const double *cr, const double *r,
-                                                                const uint32_t *deg, const uint8_t *naff,
-                                                                LoopCtl ctl) {
-  if (!iteration_begin(ctl)) return;
-  if (iter_index(ctl) == 0) naff = nullptr;
-  const uint32_t n = P.ov_off[(P.N + P.B - 1) / P.B];
-  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    const uint32_t u = uint32_t(P.ov_key[i]);
-    const double c = contrib1<FROM_RANKS>(cr, r, deg, u);
-    P.ovX[i] = naff && naff[u] ? -c : c;
-  }
-}
-
 template <int B, int VARIANT>
 hipError_t binned_update(const RankArgs &A, const BinnedPlan &P, const LoopCtl &ctl, bool extend, hipStream_t s,
                          hipEvent_t mark) {
   const uint8_t *naff = Traits<VARIANT>::frontier && extend ? A.naff : nullptr;
   constexpr bool kFromRanks = !Traits<VARIANT>::weighted;
   LoopCtl rest = ctl;  // only the first launch tells the host
-  if (P.n_ex) rest.host = nullptr;
-  if (P.n_ex) expand_kernel<B, kFromRanks><<<P.n_ex, kBinBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, ctl);
-  if (P.ov_n) {
-    const uint32_t g = (P.ov_n + kBlock - 1) / kBlock;
-    overlay_expand_kernel<kFromRanks><<<g < 4096 ? g : 4096, kBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, rest);
+  const uint32_t ov = std::min((P.ov_n + kBinBlock - 1) / kBinBlock, 1024u);
+  if (P.n_ex + ov) {
+    rest.host = nullptr;
+    expand_kernel<B, kFromRanks><<<P.n_ex + ov, kBinBlock, 0, s>>>(P, A.cr, A.r, A.deg, naff, ctl);
   }
   accumulate_kernel<B, VARIANT><<<P.n_ac, kBinBlock, 0, s>>>(A, P, rest);
   if (P.n_multi) finish_bins_kernel<VARIANT><<<P.n_multi, kBinBlock, 0, s>>>(A, P, rest);
