@@ -46,10 +46,10 @@ __device__ __forceinline__ uint32_t ld_nt(const uint32_t *p) { return __builtin_
 __device__ __forceinline__ uint32_t ld_nt(const uint16_t *p) { return __builtin_nontemporal_load(p); }
 
 // Vertex v of a bin from its in-sum: updated (update.hpp), or carried over when a dynamic variant left it
-// unaffected; `extend` (frontier variants: an in-neighbour was in the last frontier) marks it affected first. Its
-// extension costs are added to `cost` (frontier variants with A.stats). Returns the L-inf term.
+// unaffected; `extend` (frontier variants: an in-neighbour was in the last frontier) marks it affected first. Returns the
+// L-inf term.
 template <int VARIANT>
-__device__ __forceinline__ double bin_finish(const RankArgs &A, uint32_t v, double cv, CostAcc &cost, bool extend) {
+__device__ __forceinline__ double bin_finish(const RankArgs &A, uint32_t v, double cv, bool extend) {
   if constexpr (VARIANT == kWeightedForward) {  // r = (1-P) s + P sum, gathered value r / W
     const double av = fma(A.P, cv, (1 - A.P) * A.term[v]);
     A.a[v] = av;
@@ -75,8 +75,6 @@ __device__ __forceinline__ double bin_finish(const RankArgs &A, uint32_t v, doub
     copy_vertex<VARIANT, false>(A, v, rv, 0.0);
     f.affected = false;
   }
-  if constexpr (Traits<VARIANT>::frontier)
-    if (A.stats) cost.add(f, A.off[v + 1] - A.off[v], A.deg[v]);
   return e;
 }
 
@@ -263,7 +261,6 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
   constexpr bool kDeadBit = B <= 8192;
   __shared__ double sum[B];
   __shared__ uint8_t ext[EXT ? B : 1];
-  __shared__ double lds_cost[2 * kBinWaves];
   const uint4 it = P.ac_item[blockIdx.x];  // bin, first slot, end slot, partial row (kWholeBin: none)
   for (uint32_t i = threadIdx.x; i < uint32_t(B); i += kBinBlock) {
     sum[i] = 0.0;
@@ -333,16 +330,14 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
   __syncthreads();
   const uint32_t b0 = it.x * uint32_t(B);
   const uint32_t nb = min(uint32_t(B), P.N - b0);
-  CostAcc cost;
   double emax = 0.0;
   if (it.w == kWholeBin) {
     for (uint32_t i = threadIdx.x; i < nb; i += kBinBlock)
-      emax = fmax(emax, bin_finish<VARIANT>(A, b0 + i, sum[i], cost, EXT && ext[EXT ? i : 0]));
+      emax = fmax(emax, bin_finish<VARIANT>(A, b0 + i, sum[i], EXT && ext[EXT ? i : 0]));
   } else {
     double *p = P.partial + size_t(it.w) * B;
     for (uint32_t i = threadIdx.x; i < nb; i += kBinBlock) p[i] = EXT && ext[EXT ? i : 0] ? -sum[i] : sum[i];
   }
-  wg_store_costs<VARIANT, kBinWaves>(A, cost, blockIdx.x, lds_cost);
   report_change(ctl, emax);
   report_begun(ctl);
 }
@@ -355,8 +350,6 @@ template <int VARIANT>
 __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, BinnedPlan P, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
   __shared__ double part[kBinWaves][kWave];
-  __shared__ double lds_cost[2 * kBinWaves];
-  CostAcc cost;
   const uint4 m = P.multi[blockIdx.x];
   const bool split = (m.w >> 31) != 0;
   const uint32_t first = m.w & 0x7FFFFFFFu;
@@ -386,7 +379,7 @@ __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, Binn
         s1 += take(p[size_t(k + 1) * P.B]);
       }
       if (k < m.z) s0 += take(p[size_t(k) * P.B]);
-      emax = bin_finish<VARIANT>(A, v, s0 + s1, cost, flag);
+      emax = bin_finish<VARIANT>(A, v, s0 + s1, flag);
     }
   } else {
     double s0 = 0.0, s1 = 0.0;
@@ -404,10 +397,9 @@ __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, Binn
       double t = 0.0;
       flag = false;
       for (int q = 0; q < kBinWaves; ++q) t += take(part[q][lane]);
-      emax = bin_finish<VARIANT>(A, v, t, cost, flag);
+      emax = bin_finish<VARIANT>(A, v, t, flag);
     }
   }
-  wg_store_costs<VARIANT, kBinWaves>(A, cost, P.n_ac + blockIdx.x, lds_cost);
   report_change(ctl, emax);
 }
 

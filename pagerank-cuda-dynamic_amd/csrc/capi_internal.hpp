@@ -69,8 +69,8 @@ struct prh_context {
   prhc::DevBuf<uint8_t> vaff, naff, buff;
   prhc::DevBuf<uint32_t> sched_in, sched_out, tiles, counts, batch, scratch_u32;
   prhc::DevBuf<unsigned long long> loop;  // [L] error bits, then one slot holding `done`
-  prhc::DevBuf<int> flags;                // [0] validation bits, [1] traversal "changed", [2] extension direction
-  prhc::DevBuf<double> ext_stats;         // per rank workgroup: pull and push costs of the next extension
+  prhc::DevBuf<int> flags;                // [0] validation bits, [1] traversal "changed"
+  prhc::DevBuf<double> ext_stats;         // pull and push costs of the next extension, two iterations in turn
   prhc::DevBuf<uint32_t> ext_chunks;      // initial extension: chunk counts and their scan per batch source
   prhc::DevBuf<uint8_t> ext_tmp;          // its scan's temporary storage
   // in-place graph updates: per-row degree change, changed-row flags, new degrees (kept between updates)

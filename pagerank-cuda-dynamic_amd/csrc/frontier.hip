@@ -49,22 +49,20 @@ constexpr int kLowPerLane = 64 / kLowLanes;      // edges per lane (out-degree <
 // High out-degree vertices: one wave per vertex. Low ones (out-degree <= 64): kLowLanes lanes per vertex, each
 // lane loading all of its (at most kLowPerLane) targets before marking any, so that the loads overlap. Huge ones,
 // when the chunk table is given: one wave per chunk of kExtendChunk edges (blocks past nb_high + nb_low).
-__global__ __launch_bounds__(kBlock) void extend_kernel(ExtendArgs A, uint32_t nb_high, uint32_t nb_low, LoopCtl ctl,
-                                                        int use_ctl) {
-  if (use_ctl && !iteration_continues(ctl)) return;
-  if (A.direction && *A.direction != 0) return;
+__device__ __forceinline__ void push_rows(const ExtendArgs &A, uint32_t block, uint32_t nb_high, uint32_t nb_low,
+                                          uint32_t blocks) {
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  if (blockIdx.x >= nb_high + nb_low) {
-    const uint32_t nw = (gridDim.x - nb_high - nb_low) * kWavesPerBlock;
-    for (uint32_t k = (blockIdx.x - nb_high - nb_low) * kWavesPerBlock + w; k < A.n_chunks; k += nw) {
+  if (block >= nb_high + nb_low) {
+    const uint32_t nw = (blocks - nb_high - nb_low) * kWavesPerBlock;
+    for (uint32_t k = (block - nb_high - nb_low) * kWavesPerBlock + w; k < A.n_chunks; k += nw) {
       const uint32_t u = A.chunk_row[k];
       if (!A.naff[u]) continue;
       for (uint32_t e = A.chunk_beg[k] + lane; e < A.chunk_end[k]; e += kWave) mark(A, A.dst[e]);
     }
-  } else if (blockIdx.x < nb_high) {
+  } else if (block < nb_high) {
     const uint32_t n = A.sched.n_high + (A.chunk_row ? 0u : A.sched.n_huge);
     const uint32_t *order = A.sched.order + A.sched.n_low;
-    for (uint32_t i = blockIdx.x * kWavesPerBlock + w; i < n; i += nb_high * kWavesPerBlock) {
+    for (uint32_t i = block * kWavesPerBlock + w; i < n; i += nb_high * kWavesPerBlock) {
       const uint32_t u = order[i];
       if (!A.naff[u]) continue;
       const uint32_t beg = A.off[u], end = A.off[u + 1];
@@ -74,7 +72,7 @@ __global__ __launch_bounds__(kBlock) void extend_kernel(ExtendArgs A, uint32_t n
     const uint32_t n = A.sched.n_low;
     constexpr uint32_t kGroups = kBlock / kLowLanes;
     const uint32_t g = threadIdx.x / kLowLanes, j = threadIdx.x % kLowLanes;
-    for (uint32_t i = (blockIdx.x - nb_high) * kGroups + g; i < n; i += nb_low * kGroups) {
+    for (uint32_t i = (block - nb_high) * kGroups + g; i < n; i += nb_low * kGroups) {
       const uint32_t u = A.sched.order[i];
       if (!A.naff[u]) continue;
       const uint32_t beg = A.off[u], end = A.off[u + 1];
@@ -91,6 +89,12 @@ __global__ __launch_bounds__(kBlock) void extend_kernel(ExtendArgs A, uint32_t n
       for (uint32_t e = beg + kLowLanes * kLowPerLane + j; e < end; e += kLowLanes) mark(A, A.dst[e]);
     }
   }
+}
+
+// Traversal levels: one push, unless *A.direction stops it.
+__global__ __launch_bounds__(kBlock) void extend_kernel(ExtendArgs A, uint32_t nb_high, uint32_t nb_low) {
+  if (A.direction && *A.direction != 0) return;
+  push_rows(A, blockIdx.x, nb_high, nb_low, gridDim.x);
 }
 
 constexpr uint32_t kBatchChunk = 1024;  // edges of one source per wave-sized work unit of extend_batch
@@ -211,48 +215,16 @@ __global__ __launch_bounds__(kBlock) void extend_batch_keys_kernel(const unsigne
   }
 }
 
-constexpr int kDirThreads = 1024;
-
-// One workgroup: totals of the per-workgroup costs, then the choice (pull only when strictly cheaper).
-__global__ __launch_bounds__(kDirThreads) void direction_kernel(const double *stats, uint32_t n, int *direction,
-                                                                LoopCtl ctl) {
-  if (!iteration_continues(ctl)) return;
-  __shared__ double lds[2 * (kDirThreads / kWave)];
-  double pull = 0.0, push = 0.0;
-  for (uint32_t i = threadIdx.x; i < n; i += kDirThreads) {
-    pull += stats[2 * size_t(i)];
-    push += stats[2 * size_t(i) + 1];
-  }
-  pull = group_sum<kWave>(pull);
-  push = group_sum<kWave>(push);
-  const int w = threadIdx.x / kWave;
-  if ((threadIdx.x & (kWave - 1)) == 0) {
-    lds[w] = pull;
-    lds[kDirThreads / kWave + w] = push;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0.0, b = 0.0;
-    for (int k = 0; k < kDirThreads / kWave; ++k) {
-      a += lds[k];
-      b += lds[kDirThreads / kWave + k];
-    }
-    *direction = a < b ? 1 : 0;
-  }
-}
-
 constexpr int kPullLanes = 8;
 
 // Pull form of the extension over the in-CSR rows (rows sorted by in-degree, descending): a wave per row for
 // rows [0, n_wave), kPullLanes lanes per row for [n_wave, n_group), one lane per row after that. Only rows not yet
 // affected look at their in-neighbours, and stop at the first one in the frontier.
-__global__ __launch_bounds__(kBlock) void extend_pull_kernel(PullArgs A, uint32_t nb_wave, uint32_t nb_group,
-                                                             uint32_t nb_one, LoopCtl ctl) {
-  if (!iteration_continues(ctl)) return;
-  if (*A.direction != 1) return;
+__device__ __forceinline__ void pull_rows(const PullArgs &A, uint32_t block, uint32_t nb_wave, uint32_t nb_group,
+                                          uint32_t nb_one) {
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  if (blockIdx.x < nb_wave) {
-    for (uint32_t v = blockIdx.x * kWavesPerBlock + w; v < A.n_wave; v += nb_wave * kWavesPerBlock) {
+  if (block < nb_wave) {
+    for (uint32_t v = block * kWavesPerBlock + w; v < A.n_wave; v += nb_wave * kWavesPerBlock) {
       if (A.vaff[v]) continue;  // wave-uniform
       const uint32_t b = A.off[v], e = A.off[v + 1];
       for (uint32_t k = b; k < e; k += kWave) {
@@ -263,11 +235,11 @@ __global__ __launch_bounds__(kBlock) void extend_pull_kernel(PullArgs A, uint32_
         }
       }
     }
-  } else if (blockIdx.x < nb_wave + nb_group) {
+  } else if (block < nb_wave + nb_group) {
     const uint32_t g = threadIdx.x / kPullLanes, j = threadIdx.x % kPullLanes;
     constexpr uint32_t kGroups = kBlock / kPullLanes;
     const uint32_t first = A.n_wave;
-    for (uint32_t r0 = first + (blockIdx.x - nb_wave) * kGroups; r0 < A.n_group; r0 += nb_group * kGroups) {
+    for (uint32_t r0 = first + (block - nb_wave) * kGroups; r0 < A.n_group; r0 += nb_group * kGroups) {
       const uint32_t v = r0 + g;  // rows r0 .. r0 + kGroups - 1 in this round (block-uniform loop)
       bool hit = false;
       if (v < A.n_group && !A.vaff[v]) {
@@ -279,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void extend_pull_kernel(PullArgs A, uint32_
       if (j == 0 && group_bits) A.vaff[v] = 1;
     }
   } else {
-    for (uint32_t v = A.n_group + (blockIdx.x - nb_wave - nb_group) * kBlock + threadIdx.x; v < A.N;
+    for (uint32_t v = A.n_group + (block - nb_wave - nb_group) * kBlock + threadIdx.x; v < A.N;
          v += nb_one * kBlock) {
       if (A.vaff[v]) continue;
       const uint32_t b = A.off[v], e = A.off[v + 1];
@@ -289,6 +261,41 @@ __global__ __launch_bounds__(kBlock) void extend_pull_kernel(PullArgs A, uint32_
           break;
         }
     }
+  }
+}
+
+struct ExtendGrid {
+  uint32_t high, low, push;        // push: workgroups of the high and low classes, and in all
+  uint32_t wave, group, one, pull;  // pull: workgroups per row class, and in all
+};
+
+// The DF / DF-P extension of an iteration: push or pull, whichever the rank launch found cheaper. Its workgroups added
+// their costs to kCostShards pairs of sums (stats; sums of whole numbers, the same in any order); every workgroup reads
+// them and comes to the same choice (pull only when strictly cheaper), or to none where no row is unaffected or none in
+// the frontier. The first workgroup clears the sums of the next iteration's launch. (A launch to choose, one to push and
+// one to pull took 2.7 + 3.6 + 2.6 us per iteration on RMAT-16, this 4.0 us; DF on RMAT-16 1315 -> 1015 us per solve.)
+__global__ __launch_bounds__(kBlock) void extend_either_kernel(ExtendArgs E, PullArgs P, const double *stats,
+                                                               double *next_stats, int mode, ExtendGrid G,
+                                                               LoopCtl ctl) {
+  __shared__ double cost[2];
+  if (!iteration_continues(ctl)) return;
+  double pull = 1.0, push = 1.0;
+  if (mode == 1) {
+    if (threadIdx.x < 2 * kCostShards) {  // one sum a lane: 16 of pull, 16 of push
+      const double t = group_sum<kCostShards>(stats[threadIdx.x * kCostStride]);
+      if (threadIdx.x % kCostShards == 0) cost[threadIdx.x / kCostShards] = t;
+    }
+    if (blockIdx.x == 0)
+      for (uint32_t i = threadIdx.x; i < kCostSums; i += kBlock) next_stats[i] = 0.0;
+    __syncthreads();
+    pull = cost[0];
+    push = cost[1];
+    if (pull == 0.0 || push == 0.0) return;
+  }
+  if (mode == 2 || (mode == 1 && pull < push)) {
+    if (blockIdx.x < G.pull) pull_rows(P, blockIdx.x, G.wave, G.group, G.one);
+  } else {
+    if (blockIdx.x < G.push) push_rows(E, blockIdx.x, G.high, G.low, G.push);
   }
 }
 
@@ -306,13 +313,35 @@ hipError_t launch_mark_partial(uint8_t *naff, uint8_t *vaff, const uint32_t *del
   return hipGetLastError();
 }
 
-hipError_t launch_extend(const ExtendArgs &A, const LoopCtl &ctl, hipStream_t s) {
-  const uint32_t nb_high =
-      clamp_blocks(size_t(A.sched.n_high) + (A.chunk_row ? 0u : A.sched.n_huge), kWavesPerBlock, 4096);
-  const uint32_t nb_low = clamp_blocks(A.sched.n_low, kBlock / kLowLanes, 8192);
-  const uint32_t nb_chunk = A.chunk_row ? clamp_blocks(A.n_chunks, kWavesPerBlock, 4096) : 0u;
-  if (nb_high + nb_low + nb_chunk == 0) return hipSuccess;
-  extend_kernel<<<nb_high + nb_low + nb_chunk, kBlock, 0, s>>>(A, nb_high, nb_low, ctl, ctl.err ? 1 : 0);
+namespace {
+
+ExtendGrid push_grid(const ExtendArgs &A) {
+  ExtendGrid g{};
+  g.high = clamp_blocks(size_t(A.sched.n_high) + (A.chunk_row ? 0u : A.sched.n_huge), kWavesPerBlock, 4096);
+  g.low = clamp_blocks(A.sched.n_low, kBlock / kLowLanes, 8192);
+  g.push = g.high + g.low + (A.chunk_row ? clamp_blocks(A.n_chunks, kWavesPerBlock, 4096) : 0u);
+  return g;
+}
+
+}  // namespace
+
+hipError_t launch_extend(const ExtendArgs &A, hipStream_t s) {
+  const ExtendGrid g = push_grid(A);
+  if (!g.push) return hipSuccess;
+  extend_kernel<<<g.push, kBlock, 0, s>>>(A, g.high, g.low);
+  return hipGetLastError();
+}
+
+hipError_t launch_extend_either(const ExtendArgs &E, const PullArgs &P, const double *stats, double *next_stats,
+                                int mode, const LoopCtl &ctl, hipStream_t s) {
+  ExtendGrid g = push_grid(E);
+  g.wave = clamp_blocks(P.n_wave, kWavesPerBlock, 2048);
+  g.group = clamp_blocks(size_t(P.n_group) - P.n_wave, kBlock / kPullLanes, 4096);
+  g.one = clamp_blocks(size_t(P.N) - P.n_group, kBlock, 4096);
+  g.pull = g.wave + g.group + g.one;
+  const uint32_t n = mode == 0 ? g.push : mode == 2 ? g.pull : g.push > g.pull ? g.push : g.pull;
+  if (!n) return hipSuccess;
+  extend_either_kernel<<<n, kBlock, 0, s>>>(E, P, stats, next_stats, mode, g, ctl);
   return hipGetLastError();
 }
 
@@ -339,20 +368,6 @@ hipError_t launch_extend_batch_keys(uint8_t *vaff, uint8_t *naff, const unsigned
   hipError_t e = scan_u32(tmp, tmp_bytes, cnt, start, n + 1, s);
   if (e != hipSuccess) return e;
   extend_batch_keys_kernel<<<1024, kBlock, 0, s>>>(dk, nd, ik, ni, cap, off, dst, start, vaff);
-  return hipGetLastError();
-}
-
-hipError_t launch_direction(const double *stats, uint32_t n, int *direction, const LoopCtl &ctl, hipStream_t s) {
-  direction_kernel<<<1, kDirThreads, 0, s>>>(stats, n, direction, ctl);
-  return hipGetLastError();
-}
-
-hipError_t launch_extend_pull(const PullArgs &A, const LoopCtl &ctl, hipStream_t s) {
-  const uint32_t nb_wave = clamp_blocks(A.n_wave, kWavesPerBlock, 2048);
-  const uint32_t nb_group = clamp_blocks(size_t(A.n_group) - A.n_wave, kBlock / kPullLanes, 4096);
-  const uint32_t nb_one = clamp_blocks(size_t(A.N) - A.n_group, kBlock, 4096);
-  if (nb_wave + nb_group + nb_one == 0) return hipSuccess;
-  extend_pull_kernel<<<nb_wave + nb_group + nb_one, kBlock, 0, s>>>(A, nb_wave, nb_group, nb_one, ctl);
   return hipGetLastError();
 }
 

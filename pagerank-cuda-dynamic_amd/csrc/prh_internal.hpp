@@ -80,6 +80,8 @@ struct RankPlan {
   uint32_t n_chunked;
 };
 
+constexpr uint32_t kCostShards = 16, kCostStride = 16, kCostSums = 2 * kCostShards * kCostStride;
+
 struct RankArgs {
   double *a;          // new ranks
   const double *r;    // old ranks
@@ -91,8 +93,9 @@ struct RankArgs {
   const uint32_t *src;  // in-CSR sources [M]
   const uint32_t *deg;  // out-degree [N]
   double C0, P, D, C;  // teleport share (1-P)/N, damping, frontier and prune tolerances
-  // Frontier variants, optional: per workgroup, [2 b] = in-edges of the rows left unaffected (the cost of pulling
-  // the next extension) and [2 b + 1] = out-edges of the rows put in the frontier (the cost of pushing it).
+  // Frontier variants, optional: kCostSums doubles, of which workgroup b adds to two (b mod kCostShards, kCostStride apart):
+  // the in-edges of the rows it left unaffected (the cost of pulling the next extension) and, kCostShards sums on, the
+  // out-edges of the rows it put in the frontier (the cost of pushing it).
   double *stats;
   // Weighted variants: the teleport share s (forward) or the seed g (adjoint), and the out-weight sums W; there a
   // holds the new values, ca the new gathered values (a / W forward, a adjoint), cr the old ones.
@@ -107,7 +110,7 @@ struct ExtendArgs {
   Schedule sched;        // out-degree partition
   uint8_t *fresh;        // optional: also set for newly marked vertices (traversal levels)
   int *changed;          // optional: set to 1 when a vertex is newly marked
-  const int *direction;  // optional: the push runs only while *direction == 0 (see launch_direction)
+  const int *direction;  // optional: launch_extend runs only while *direction == 0
   // optional: the huge class (sched.n_huge rows after the high ones) as chunks of at most kExtendChunk edges,
   // chunk k covering edges [chunk_beg[k], chunk_end[k]) of row chunk_row[k]; without it huge rows take a wave each
   const uint32_t *chunk_beg = nullptr, *chunk_end = nullptr, *chunk_row = nullptr;
@@ -122,7 +125,6 @@ struct PullArgs {
   const uint8_t *naff;
   const uint32_t *off, *src;  // in-CSR (degree-ordered layout)
   uint32_t n_wave, n_group, N;
-  const int *direction;       // runs only while *direction == 1
 };
 
 // Source-sliced plan of the plain update (Static / Naive-dynamic). Source u belongs to slice
@@ -506,10 +508,10 @@ hipError_t launch_extend_batch_keys(uint8_t *vaff, uint8_t *naff, const unsigned
                                     const unsigned long long *ik, const uint32_t *ni, uint32_t cap,
                                     const uint32_t *off, const uint32_t *dst, uint32_t *cnt, uint32_t *start,
                                     void *tmp, size_t &tmp_bytes, hipStream_t s);
-hipError_t launch_extend(const ExtendArgs &A, const LoopCtl &ctl, hipStream_t s);
-// Sums the per-workgroup costs the rank launches left in stats[0 .. 2 n) and sets *direction to 1 (pull) when
-// pulling is cheaper, else 0 (push). Honours iteration l's control like the extension.
-hipError_t launch_direction(const double *stats, uint32_t n, int *direction, const LoopCtl &ctl, hipStream_t s);
-hipError_t launch_extend_pull(const PullArgs &A, const LoopCtl &ctl, hipStream_t s);
+hipError_t launch_extend(const ExtendArgs &A, hipStream_t s);
+// The extension after iteration ctl.l's rank launch: mode 0 push, 2 pull, 1 the cheaper by the costs that launch added to
+// `stats` (kCostSums doubles); next_stats, the next iteration's, is cleared.
+hipError_t launch_extend_either(const ExtendArgs &E, const PullArgs &P, const double *stats, double *next_stats,
+                                int mode, const LoopCtl &ctl, hipStream_t s);
 
 }  // namespace prh

@@ -50,25 +50,6 @@ __device__ __forceinline__ RowOperands row_operands(const RankArgs &A, uint32_t 
   return o;
 }
 
-// Workgroup totals of the costs to A.stats[2 slot], [2 slot + 1]. Every thread must call it.
-template <int VARIANT>
-__device__ __forceinline__ void store_costs(const RankArgs &A, CostAcc c, uint32_t slot, double *lds8) {
-  if constexpr (Traits<VARIANT>::frontier) {
-    if (!A.stats) return;
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const double pull = group_sum<kWave>(c.pull), push = group_sum<kWave>(c.push);
-    if (lane == 0) {
-      lds8[w] = pull;
-      lds8[kWavesPerBlock + w] = push;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      A.stats[2 * size_t(slot)] = (lds8[0] + lds8[1]) + (lds8[2] + lds8[3]);
-      A.stats[2 * size_t(slot) + 1] = (lds8[4] + lds8[5]) + (lds8[6] + lds8[7]);
-    }
-  }
-}
-
 // On graphs whose contributions fit the L2s a launch is bound by its longest chain of dependent loads, not by bytes
 // (RMAT-16: 29 us per iteration for 1 M gathers that the L2s serve in 5). One batch of U strided edges e, e + STEP,
 // ...: all U source ids are loaded before the first gather and all gathers are in flight together, so a batch costs
@@ -270,7 +251,7 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
     }
   }
   __shared__ double lds_cost[2 * kWavesPerBlock];
-  store_costs<VARIANT>(A, cost, blockIdx.x, lds_cost);
+  add_costs<VARIANT, kWavesPerBlock>(A, cost, lds_cost);
   report_change(ctl, emax);
   report_begun(ctl);
 }
@@ -280,7 +261,6 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
 template <int VARIANT>
 __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, RankPlan P, uint32_t n_rows, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;  // same outcome as the rank kernel's entry test of this iteration
-  __shared__ double lds_cost[2 * kWavesPerBlock];
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   double emax = 0.0;
   CostAcc cost;
@@ -303,7 +283,8 @@ __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, Rank
       cost.add(f, in_deg, d);
     }
   }
-  store_costs<VARIANT>(A, cost, P.blocks + blockIdx.x, lds_cost);
+  __shared__ double lds_cost[2 * kWavesPerBlock];
+  add_costs<VARIANT, kWavesPerBlock>(A, cost, lds_cost);
   report_change(ctl, emax);
 }
 

@@ -61,12 +61,12 @@ struct prh_stream {
   uint32_t *ext_cnt = nullptr, *ext_start = nullptr;  // the initial extension's chunks per batch entry [2 cap + 1]
   void *sort_tmp = nullptr, *scan_tmp = nullptr;
   size_t sort_bytes = 0, scan_bytes = 0;
-  double *rank[2] = {}, *contrib[2] = {}, *stats = nullptr;
+  double *rank[2] = {}, *contrib[2] = {}, *costs = nullptr;
   uint8_t *vaff = nullptr, *naff = nullptr;
-  int *ctl = nullptr;  // [0] done, [1] iteration index (adjacent, as LoopCtl expects), [2] direction, [3] flags
+  int *ctl = nullptr;  // [0] done, [1] first iteration of the replay (adjacent, as LoopCtl expects), [3] flags
   unsigned long long *err = nullptr;
   prh::RankPlan plan{};
-  uint32_t n_items = 0, chunk = 0, stat_slots = 0, pull_wave = 0, pull_group = 0;
+  uint32_t n_items = 0, chunk = 0, pull_wave = 0, pull_group = 0;
   hipGraphExec_t apply[2] = {}, iter[2] = {}, closure[2] = {};
   std::vector<std::pair<void *, size_t>> bufs;
   bool broken = false;
@@ -203,8 +203,7 @@ int stream_apply_body(prh_stream *S, int p) {
       PRH_HIP(c, prh::launch_copy_u8(S->front[0], S->vaff, N, s));
       PRH_HIP(c, prh::launch_fill_i32(S->lvl, 0, 4, s));
     } else if (!S->blocked) {
-      const int mode = c->tuning.extension_direction;
-      if (mode != 1) PRH_HIP(c, prh::launch_fill_i32(S->ctl + 2, mode == 2 ? 1 : 0, 1, s));
+      PRH_HIP(c, prh::launch_fill_u64(reinterpret_cast<unsigned long long *>(S->costs), 0ull, 2 * prh::kCostSums, s));
     }
   }
   return PRH_SUCCESS;
@@ -225,7 +224,7 @@ int stream_closure_body(prh_stream *S, int q) {
     PRH_HIP(c, prh::launch_fill_u8(S->front[(k + 1) & 1], 0, S->N, s));
     prh::ExtendArgs E{S->vaff, S->front[k & 1], S->out_off[q], S->out_dst[q], os, S->front[(k + 1) & 1],
                       S->lvl + 2 + (k & 1), S->lvl + 1};
-    PRH_HIP(c, prh::launch_extend(E, prh::LoopCtl{}, s));
+    PRH_HIP(c, prh::launch_extend(E, s));
     PRH_HIP(c, prh::launch_closure_advance(S->lvl, s));
   }
   return PRH_SUCCESS;
@@ -241,13 +240,16 @@ int stream_iter_body(prh_stream *S, int q) {
   const bool frontier = S->variant >= prh::kFrontier;
   const int mode = c->tuning.extension_direction;
   unsigned long long *err = S->err;
-  int *done = S->ctl, *dir = S->ctl + 2, *host = c->progress;
+  int *done = S->ctl, *host = c->progress;
+  auto costs = [&](int i) {
+    return frontier && mode == 1 && !S->blocked ? S->costs + prh::kCostSums * (i & 1) : nullptr;
+  };
   const prh::Schedule os{S->sched_order, S->sched_low, S->sched_high, 0};
-  const prh::PullArgs pull{S->vaff, S->naff, S->in_off[q], S->in_src[q], S->pull_wave, S->pull_group, S->N, dir};
+  const prh::PullArgs pull{S->vaff, S->naff, S->in_off[q], S->in_src[q], S->pull_wave, S->pull_group, S->N};
   for (int i = 0; i < kStreamChunk; ++i) {
     prh::RankArgs A{S->rank[(i + 1) & 1], S->rank[i & 1], S->contrib[(i + 1) & 1], S->contrib[i & 1], S->naff,
                     S->vaff, S->in_off[q], S->in_src[q], S->outdeg, C0, P, o.frontier_tolerance, o.prune_tolerance,
-                    frontier && mode == 1 && !S->blocked ? S->stats : nullptr};
+                    costs(i)};
     const prh::LoopCtl ctl{err, done, -1 - i, o.max_iterations, o.tolerance, host};
     if (S->blocked) {  // the frontier's extension happens inside the update (from the second iteration on)
       PRH_HIP(c, prh::launch_binned_update(S->variant, A, S->bplan, ctl, frontier, s));
@@ -255,10 +257,8 @@ int stream_iter_body(prh_stream *S, int q) {
     }
     PRH_HIP(c, prh::launch_rank_update(S->variant, A, S->plan, ctl, s));
     if (frontier) {
-      if (mode == 1) PRH_HIP(c, prh::launch_direction(S->stats, S->stat_slots, dir, ctl, s));
-      prh::ExtendArgs E{S->vaff, S->naff, S->out_off[q], S->out_dst[q], os, nullptr, nullptr, dir};
-      PRH_HIP(c, prh::launch_extend(E, ctl, s));
-      if (mode != 0) PRH_HIP(c, prh::launch_extend_pull(pull, ctl, s));
+      const prh::ExtendArgs E{S->vaff, S->naff, S->out_off[q], S->out_dst[q], os, nullptr, nullptr, nullptr};
+      PRH_HIP(c, prh::launch_extend_either(E, pull, costs(i), costs(i + 1), mode, ctl, s));
     }
   }
   PRH_HIP(c, prh::launch_advance(prh::LoopCtl{err, done, -1, o.max_iterations, o.tolerance, host}, kStreamChunk, s));
@@ -388,8 +388,7 @@ int prh_stream_create(prh_context *c, const prh_graph *g, prh_method method, con
       S->plan.row_first = t + 3 * size_t(S->n_items);
       S->plan.partial = part;
     }
-    S->stat_slots = S->plan.blocks + (nc ? prh::finish_chunked_grid(nc) : 0);
-    step(stream_alloc(S, &S->stats, 2 * size_t(std::max<uint32_t>(S->stat_slots, 1))));
+    step(stream_alloc(S, &S->costs, 2 * prh::kCostSums));
     S->pull_wave = layout_rows_above(g, 64);
     S->pull_group = layout_rows_above(g, 4);
   }

@@ -83,7 +83,7 @@ int mark_affected(prh_context *c, const prh_graph *g, int method, const DevBatch
     T.fresh = fresh;
     T.changed = c->flags.p + 1;
     T.direction = nullptr;
-    PRH_HIP(c, prh::launch_extend(T, prh::LoopCtl{}, s));
+    PRH_HIP(c, prh::launch_extend(T, s));
     PRH_HIP(c, hipMemcpyAsync(c->pinned, c->flags.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     PRH_HIP(c, hipStreamSynchronize(s));
     if (*reinterpret_cast<int *>(c->pinned) == 0) break;
@@ -229,14 +229,9 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   // 2 pull only. The pull form splits rows at in-degree 64 (a wave each) and 4 (8 lanes each).
   const int dir_mode = frontier ? c->tuning.extension_direction : 0;
   const bool dir_auto = dir_mode == 1 && !binned;
-  // Per-workgroup extension costs: one slot per workgroup of the launches that finish vertices.
-  const uint32_t stat_slots = binned   ? g->bin.plan.n_ac + g->bin.plan.n_multi
-                              : window ? g->win.wgs
-                                       : plan.blocks + (plan.n_chunked ? prh::finish_chunked_grid(plan.n_chunked) : 0);
-  if (dir_auto) PRH_CHECK(ensure(c, c->ext_stats, 2 * size_t(std::max<uint32_t>(stat_slots, 1))));
-  int *dir = frontier ? c->flags.p + 2 : nullptr;
+  if (dir_auto) PRH_CHECK(ensure(c, c->ext_stats, 2 * prh::kCostSums));  // the sums of two iterations in turn
   const prh::PullArgs pull{c->vaff.p, c->naff.p, g->l_in_off, g->l_in_src, layout_rows_above(g, 64),
-                           layout_rows_above(g, 4), N, dir};
+                           layout_rows_above(g, 4), N};
   for (int rep = 0; rep < o->repeat; ++rep) {
     if (q) PRH_CHECK(load_initial_ranks(c, g, q, host));  // untimed, as the reference's q copy (pagerankCuda.hxx:810)
     PRH_HIP(c, hipEventRecord(c->ev[0], s));
@@ -259,9 +254,12 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     PRH_HIP(c, hipEventRecord(c->ev[2], s));
     // Iterations.
     PRH_HIP(c, prh::launch_fill_u64(err, 0ull, size_t(L) + 1, s));
-    if (frontier && dir_mode != 1) PRH_HIP(c, prh::launch_fill_i32(dir, dir_mode == 2 ? 1 : 0, 1, s));
+    if (dir_auto)
+      PRH_HIP(c, prh::launch_fill_u64(reinterpret_cast<unsigned long long *>(c->ext_stats.p), 0ull,
+                                      2 * prh::kCostSums, s));
     const double P = o->damping;
     const double C0 = (1 - P) / N;
+    auto costs = [&](int l) { return dir_auto ? c->ext_stats.p + prh::kCostSums * (l & 1) : nullptr; };
     reset_progress(c);
     for (int l = 0; l < L; ++l) {
       PRH_CHECK(wait_progress(c, l - ahead + 1));
@@ -269,7 +267,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       const prh::LoopCtl ctl{err, done, l, L, o->tolerance, c->progress};
       prh::RankArgs A{c->rank[(l + 1) & 1].p, c->rank[l & 1].p, c->contrib[(l + 1) & 1].p, c->contrib[l & 1].p,
                       c->naff.p, c->vaff.p, g->l_in_off, g->l_in_src, g->l_outdeg, C0, P, o->frontier_tolerance,
-                      o->prune_tolerance, dir_auto ? c->ext_stats.p : nullptr};
+                      o->prune_tolerance, costs(l)};
       if (c->ktiming) PRH_HIP(c, hipEventRecord(c->kev[2 * l], s));
       hipEvent_t mark = c->ktiming ? c->kev[2 * l + 1] : nullptr;
       if (binned)
@@ -280,7 +278,6 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       } else if (sliced) PRH_HIP(c, prh::launch_sliced_update(A, g->sliced, ctl, s, mark));
       else PRH_HIP(c, prh::launch_rank_update(variant, A, plan, ctl, s, mark));
       if (frontier && !binned) {  // the blocked plan extends inside the next iteration's update
-        if (dir_auto) PRH_HIP(c, prh::launch_direction(c->ext_stats.p, stat_slots, dir, ctl, s));
         prh::ExtendArgs E = xo;
         E.vaff = c->vaff.p;
         E.naff = c->naff.p;
@@ -288,9 +285,8 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
         E.dst = g->l_out_dst;
         E.fresh = nullptr;
         E.changed = nullptr;
-        E.direction = dir;
-        PRH_HIP(c, prh::launch_extend(E, ctl, s));
-        if (dir_mode != 0) PRH_HIP(c, prh::launch_extend_pull(pull, ctl, s));
+        E.direction = nullptr;
+        PRH_HIP(c, prh::launch_extend_either(E, pull, costs(l), costs(l + 1), dir_mode, ctl, s));
       }
     }
     PRH_HIP(c, hipEventRecord(c->ev[3], s));

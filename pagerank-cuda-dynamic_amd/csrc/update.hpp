@@ -70,10 +70,11 @@ struct CostAcc {
   }
 };
 
-// Workgroup totals of the extension costs to A.stats[2 slot], [2 slot + 1] (frontier variants with A.stats), for a
-// workgroup of WAVES waves. Every thread must call it.
+// Adds the workgroup's extension costs to sums of A.stats (frontier variants with A.stats), for a workgroup of WAVES waves.
+// The costs are whole numbers, so the sums do not depend on the order. The sums lie a cache line apart: atomics on one
+// line queue (an atomic per wave on eight lines doubled the rank launch's time on RMAT-16). Every thread must call it.
 template <int VARIANT, int WAVES>
-__device__ __forceinline__ void wg_store_costs(const RankArgs &A, const CostAcc &c, uint32_t slot, double *lds) {
+__device__ __forceinline__ void add_costs(const RankArgs &A, const CostAcc &c, double *lds) {
   if constexpr (Traits<VARIANT>::frontier) {
     if (!A.stats) return;
     const int w = threadIdx.x / kWave;
@@ -83,14 +84,11 @@ __device__ __forceinline__ void wg_store_costs(const RankArgs &A, const CostAcc 
       lds[WAVES + w] = push;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      double a = 0.0, b = 0.0;
-      for (int i = 0; i < WAVES; ++i) {
-        a += lds[i];
-        b += lds[WAVES + i];
-      }
-      A.stats[2 * size_t(slot)] = a;
-      A.stats[2 * size_t(slot) + 1] = b;
+    if (threadIdx.x < 2) {  // thread 0: pull, thread 1: push
+      double t = 0.0;
+      for (int i = 0; i < WAVES; ++i) t += lds[threadIdx.x * WAVES + i];
+      if (t > 0.0)
+        unsafeAtomicAdd(A.stats + (threadIdx.x * kCostShards + blockIdx.x % kCostShards) * kCostStride, t);
     }
   }
 }

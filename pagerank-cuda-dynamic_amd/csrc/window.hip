@@ -28,7 +28,6 @@ namespace prh {
 namespace {
 
 constexpr uint32_t kWinRows = kBinBlock;  // rows per chunk, one per thread
-constexpr int kWinWaves = kBinBlock / kWave;
 constexpr int kWinIds = 6;  // source ids a row loads ahead of its chunk; further ones are read when it is summed
 
 struct WinRow {
@@ -68,7 +67,6 @@ __global__ __launch_bounds__(kBinBlock) void window_update_kernel(RankArgs A, Wi
   static_assert(S >= int(kWinRows) + 2, "ring smaller than a chunk");
   constexpr uint32_t R = kWinRows;
   __shared__ double ring[S];
-  __shared__ double lds_cost[2 * kWinWaves];
   const uint32_t N = W.N, H = W.H, t = threadIdx.x;
   const uint32_t a = uint32_t(uint64_t(blockIdx.x) * N / gridDim.x);
   const uint32_t z = uint32_t(uint64_t(blockIdx.x + 1) * N / gridDim.x);  // this workgroup's rows [a, z)
@@ -142,7 +140,8 @@ __global__ __launch_bounds__(kBinBlock) void window_update_kernel(RankArgs A, Wi
       ne = ne2;
     }
   }
-  wg_store_costs<VARIANT, kWinWaves>(A, cost, blockIdx.x, lds_cost);
+  __shared__ double lds_cost[2 * (kBinBlock / kWave)];
+  add_costs<VARIANT, kBinBlock / kWave>(A, cost, lds_cost);
   report_change(ctl, emax);
   report_begun(ctl);
 }
