@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -11,6 +12,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "capi_internal.hpp"
@@ -79,6 +81,27 @@ int Temps::get_bytes(void **p, size_t bytes) {
   return PRH_SUCCESS;
 }
 
+namespace {
+
+constexpr size_t kSlots = 8, kSlotBytes = kStagingBytes / kSlots;  // the staging area's slots
+
+int ensure_staging(prh_context *c) {
+  if (!c->staging && hipHostMalloc(reinterpret_cast<void **>(&c->staging), kStagingBytes, hipHostMallocDefault) !=
+                         hipSuccess) {
+    (void)hipGetLastError();
+    c->staging = nullptr;
+    return fail(c, PRH_ERROR_OUT_OF_MEMORY, "pinned staging area (%zu bytes)", kStagingBytes);
+  }
+  for (auto &e : c->copy_ev)
+    if (!e) PRH_HIP(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return PRH_SUCCESS;
+}
+
+}  // namespace
+
+// Chunk i of kSlotBytes goes through slot i mod kSlots: the calling thread issues the device copies as slots come free,
+// and worker t of T moves chunks t, t + T, ... on to the caller's memory. That memory is as a rule fresh, and its page
+// faults, not the bus, set the time of one thread: 537 MB in one thread without overlap about 48 ms, like this 11 ms.
 int copy_to_host(prh_context *c, void *dst, const void *src, size_t n) {
   hipStream_t s = c->stream;
   if (n <= kStagingBytes) {
@@ -86,18 +109,63 @@ int copy_to_host(prh_context *c, void *dst, const void *src, size_t n) {
     PRH_HIP(c, hipStreamSynchronize(s));
     return PRH_SUCCESS;
   }
-  if (!c->staging && hipHostMalloc(reinterpret_cast<void **>(&c->staging), kStagingBytes, hipHostMallocDefault) !=
-                         hipSuccess) {
-    (void)hipGetLastError();
-    c->staging = nullptr;
-    return fail(c, PRH_ERROR_OUT_OF_MEMORY, "pinned staging area (%zu bytes)", kStagingBytes);
+  PRH_CHECK(ensure_staging(c));
+  const size_t chunks = (n + kSlotBytes - 1) / kSlotBytes;
+  const auto bytes = [&](size_t i) { return std::min(kSlotBytes, n - i * kSlotBytes); };
+  std::atomic<size_t> issued{0}, freed[kSlots] = {};  // chunks whose copy is issued; copies out of each slot
+  std::atomic<int> team{0}, error{hipSuccess};        // team: number of workers, once known; -1: none
+  auto work = [&](int t) {
+    int T;
+    while ((T = team.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
+    if (T < 0 || hipSetDevice(c->device) != hipSuccess) {
+      if (T > 0) error = hipErrorInvalidDevice;
+      return;
+    }
+    for (size_t i = size_t(t); i < chunks; i += size_t(T)) {
+      while (issued.load(std::memory_order_acquire) <= i) {
+        if (error != hipSuccess) return;
+        std::this_thread::yield();
+      }
+      const hipError_t e = hipEventSynchronize(c->copy_ev[i % kSlots]);
+      if (e != hipSuccess) {
+        error = e;
+        return;
+      }
+      std::memcpy(static_cast<uint8_t *>(dst) + i * kSlotBytes, c->staging + i % kSlots * kSlotBytes, bytes(i));
+      freed[i % kSlots].fetch_add(1, std::memory_order_release);
+    }
+  };
+  std::vector<std::thread> workers;
+  try {
+    const unsigned cores = std::thread::hardware_concurrency();
+    const int want = int(std::min<size_t>(std::max(1u, std::min(8u, cores / 2)), chunks));
+    workers.reserve(size_t(want));
+    for (int t = 0; t < want; ++t) workers.emplace_back(work, t);
+  } catch (...) {  // fewer threads than wanted, or none
   }
-  for (size_t o = 0; o < n; o += kStagingBytes) {
-    const size_t m = std::min(kStagingBytes, n - o);
-    PRH_HIP(c, hipMemcpyAsync(c->staging, static_cast<const uint8_t *>(src) + o, m, hipMemcpyDeviceToHost, s));
-    PRH_HIP(c, hipStreamSynchronize(s));
-    std::memcpy(static_cast<uint8_t *>(dst) + o, c->staging, m);
+  const int T = int(workers.size());
+  team.store(T ? T : -1, std::memory_order_release);
+  for (size_t i = 0; i < chunks && error == hipSuccess; ++i) {
+    const size_t k = i % kSlots;
+    while (T && freed[k].load(std::memory_order_acquire) < i / kSlots && error == hipSuccess) std::this_thread::yield();
+    hipError_t e = hipMemcpyAsync(c->staging + k * kSlotBytes, static_cast<const uint8_t *>(src) + i * kSlotBytes,
+                                  bytes(i), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipEventRecord(c->copy_ev[k], s);
+    if (e != hipSuccess) {
+      error = e;
+      break;
+    }
+    issued.store(i + 1, std::memory_order_release);
+    if (!T) {
+      PRH_HIP(c, hipStreamSynchronize(s));
+      std::memcpy(static_cast<uint8_t *>(dst) + i * kSlotBytes, c->staging + k * kSlotBytes, bytes(i));
+    }
   }
+  for (auto &t : workers) t.join();
+  const hipError_t e = hipStreamSynchronize(s);
+  if (error == hipSuccess) error = e;
+  if (error != hipSuccess)
+    return fail(c, PRH_ERROR_DEVICE, "copy to the host: %s", hipGetErrorString(hipError_t(error.load())));
   return PRH_SUCCESS;
 }
 
@@ -220,6 +288,8 @@ void prh_context_destroy(prh_context *c) {
   if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->progress) (void)hipHostFree(c->progress);
   if (c->staging) (void)hipHostFree(c->staging);
+  for (auto &e : c->copy_ev)
+    if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }

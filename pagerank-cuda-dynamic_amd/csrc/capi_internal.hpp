@@ -104,6 +104,7 @@ struct prh_context {
   // one by one, for tools that trace kernels.
   bool capture = true;
   uint8_t *staging = nullptr;  // host-pinned staging area of large device-to-host copies (kStagingBytes), on demand
+  hipEvent_t copy_ev[8] = {};  // its slots' copies
   uint32_t *noalloc_scratch = nullptr;  // device address of noalloc.hip's fixed scratch on this device
   hipEvent_t ev[4] = {};
   bool ktiming = false;
@@ -301,8 +302,8 @@ struct DevBatch {
   size_t ND = 0, NI = 0;
 };
 
-// Device-to-host copy of n bytes into caller (pageable) memory on the context's stream, synchronously: in chunks of
-// kStagingBytes through the context's pinned staging area when n exceeds one chunk, else directly (capi.hip).
+// Device-to-host copy of n bytes into caller (pageable) memory on the context's stream, synchronously: through the
+// context's pinned staging area by several threads when n exceeds its size (kStagingBytes), else directly (capi.hip).
 int copy_to_host(prh_context *c, void *dst, const void *src, size_t n);
 
 // plans.hip

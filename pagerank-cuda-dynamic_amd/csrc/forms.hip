@@ -513,7 +513,7 @@ int weighted_adjoint_impl(prh_context *c, const prh_graph *g, const float *w, co
   if (lam)
     PRH_HIP(c, hipMemcpyAsync(lam, lam_c, size_t(N) * 8, device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, hs));
   if (!device) {
-    if (M) PRH_HIP(c, hipMemcpyAsync(grad_w, gw, size_t(M) * 8, hipMemcpyDeviceToHost, hs));
+    if (M) PRH_CHECK(copy_to_host(c, grad_w, gw, size_t(M) * 8));
     PRH_HIP(c, hipMemcpyAsync(grad_s, gs, size_t(N) * 8, hipMemcpyDeviceToHost, hs));
   }
   PRH_HIP(c, hipStreamSynchronize(hs));

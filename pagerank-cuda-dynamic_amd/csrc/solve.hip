@@ -316,7 +316,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   if (host) {
     double *tmp = c->contrib[(iterations + 1) & 1].p;
     PRH_HIP(c, prh::launch_scatter_f64(res, g->perm, N, tmp, s));
-    PRH_HIP(c, hipMemcpyAsync(ranks, tmp, size_t(N) * 8, hipMemcpyDeviceToHost, s));
+    PRH_CHECK(copy_to_host(c, ranks, tmp, size_t(N) * 8));
   } else {
     PRH_HIP(c, prh::launch_scatter_f64(res, g->perm, N, ranks, s));
   }

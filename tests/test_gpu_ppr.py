@@ -140,3 +140,22 @@ def test_tile_widths_and_row_classes(ctx, oracle_mod, k):
         if res.iterations[j] == it:
             assert np.all(np.abs(res.ranks[:, j] - ref) <= 6e-11 * ref)
         assert np.abs(res.ranks[:, j] - ref).max() <= 1e-9
+
+
+def test_ranks_larger_than_the_staging_area(ctx, oracle_mod):
+    """72 MB of ranks: copied to the host in slots of the 64 MB staging area by several threads, the last one in part."""
+    from pagerank_amd import HostGraph, ppr_batched
+    n, k = 140001, 64
+    rng = np.random.default_rng(4)
+    src = np.concatenate([rng.integers(0, n, 300000), np.arange(n)]).astype(np.uint32)
+    dst = np.concatenate([rng.integers(0, n, 300000), (np.arange(n) + 1) % n]).astype(np.uint32)
+    y = HostGraph.from_edges(n, src, dst)
+    seeds = _seed_sets(n, k, 300, rng)
+    print(f"[ppr] staging N={y.N} M={y.M}", flush=True)
+    yg = ctx.upload(y, with_out=False)
+    for _ in range(2):
+        res = ppr_batched(yg, seeds)
+        assert np.abs(res.ranks.sum(axis=0) - 1.0).max() < 1e-8
+    for j in (0, 31, 63):
+        ref, it = oracle_mod.ppr(y, _teleport(n, seeds[j]))
+        assert abs(int(res.iterations[j]) - it) <= 1 and np.abs(res.ranks[:, j] - ref).max() <= 1e-9
