@@ -161,6 +161,35 @@ struct SliceBases {
   uint32_t item[kMaxSlices];  // first item id of slice x
 };
 
+// Iterations [first, last) of a small graph's solve in one workgroup (every unweighted variant, rows in order of
+// in-degree; small.hip): from rank[first & 1] and, for the dynamic variants, the affected flags; stops after the iteration
+// whose changes stay below tol. The ranks after iteration n - 1 go to rank[n & 1]. Rows [band[k], band[k + 1]) take 64 >> k
+// lanes each and make the items [item[k], item[k + 1]), 1 << k rows in each.
+constexpr int kSmallBlock = 1024;
+constexpr uint32_t kSmallLds = 156 * 1024;
+constexpr uint32_t kSmallEdges = 16;   // edges per lane, at most, for rows of up to 64 times as many
+constexpr int kSmallIterations = 256;  // iterations per launch, so that no launch lasts long whatever the options
+struct SmallArgs {
+  double *rank[2];
+  const uint32_t *off, *src, *deg;
+  uint8_t *vaff;
+  uint32_t N;
+  uint32_t band[8], item[8];
+  uint32_t rounds;  // of all items: 512 bytes of ids each
+  double C0, P, D, C, tol;
+  int first, last;
+  int *host;  // pinned host memory: [0] = last once done without stopping, [1] = iterations performed if stopped
+};
+// Rounds of four edges a lane for a row of this in-degree, 64 >> k lanes each.
+__host__ __device__ inline uint32_t small_rounds(uint32_t in_degree, int k) {
+  const uint32_t per_round = 256u >> k;
+  return (in_degree + per_round - 1) / per_round;
+}
+// LDS bytes: contributions twice and ranks, the ids, the items, 16-bit out-degrees and two flags a vertex.
+inline uint64_t small_lds(uint64_t N, uint64_t items, uint64_t rounds) {
+  return 28 * N + 17 + 512 * rounds + 4 * items;
+}
+
 // Propagation-blocked plan of the rank update (every variant; binned.hip). Layout rows are cut into runs
 // of B vertices: source blocks and destination bins, both numbered s, b = vertex / B. Slots (one per edge) are
 // ordered bin-major (bin, source block, destination, source); X holds the slots' contributions block-major (block,
@@ -212,6 +241,9 @@ struct WindowPlan {
   uint32_t S;    // ring entries: kWindowRingSmall or kWindowRingLarge
   uint32_t wgs;  // workgroups
 };
+
+// ---- small.hip ----
+hipError_t launch_small_solve(int variant, const SmallArgs &A, hipStream_t s);
 
 // ---- partition.hip ----
 // Stable 3-way partition of [0,N) by degree d = off[v+1]-off[v]: d <= t1, t1 < d <= t2, d > t2.

@@ -153,6 +153,20 @@ static int load_initial_ranks(prh_context *c, const prh_graph *g, const double *
   return PRH_SUCCESS;
 }
 
+// The bands and items of a small graph's solve; false if the graph does not fit. (That the ids' 16-bit byte offsets hold
+// every vertex follows from the size of LDS.)
+static bool small_plan(const prh_graph *g, prh::SmallArgs &A) {
+  if (g->layout != 0 || g->updated || g->M > 65535 || prh::small_lds(g->N, 0, g->M / 256) > prh::kSmallLds) return false;
+  A.N = g->N;
+  A.band[0] = A.item[0] = A.rounds = 0;
+  for (int k = 0; k < 7; ++k) {
+    A.band[k + 1] = k == 6 ? g->N : std::max(A.band[k], layout_rows_above(g, prh::kSmallEdges * (32u >> k)));
+    for (uint32_t v = A.band[k]; v < A.band[k + 1]; v += 1u << k) A.rounds += prh::small_rounds(g->sorted_deg[v], k);
+    A.item[k + 1] = A.item[k] + (A.band[k + 1] - A.band[k] + (1u << k) - 1) / (1u << k);
+  }
+  return prh::small_lds(g->N, A.item[7], A.rounds) <= prh::kSmallLds && A.item[7] <= prh::kSmallBlock;
+}
+
 int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options *o, const uint32_t *du,
                const uint32_t *dv, size_t nd, const uint32_t *iu, size_t ni, const double *q, double *ranks,
                prh_stats *st, bool host, bool account_prep) {
@@ -188,6 +202,9 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   const bool binned = c->tuning.blocking > 0;
   const bool window = !binned && c->tuning.window != 0 && g->layout == 1;
   const bool sliced = !binned && !window && variant == prh::kPlain && c->tuning.source_slices > 0 && g->layout == 0;
+  // A row plan's small graph runs its iterations in one workgroup. (Timed launches are one per iteration.)
+  prh::SmallArgs sm{};
+  const bool small = !binned && !window && !sliced && !c->ktiming && small_plan(g, sm);
   if (!binned) PRH_CHECK(ensure_in_csr(c, gm));  // the other plans read the in-CSR in every iteration
   if (binned) PRH_CHECK(build_binned_plan(c, gm));
   else if (window) PRH_CHECK(build_window_plan(c, gm));
@@ -240,7 +257,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     // The out-degree schedule serves the traversal levels and the row plan's frontier extension; the initial
     // extension runs from the batch list and the blocked plan extends inside its update.
     prh::ExtendArgs xo{};
-    if (dynamic && (method == PRH_DYNAMIC_TRAVERSAL || (frontier && !binned))) {
+    if (dynamic && (method == PRH_DYNAMIC_TRAVERSAL || (frontier && !binned && !small))) {
       PRH_CHECK(out_schedule(c, gm, xo));
       if (account_prep) prep += gm->out_prep.take();
     }
@@ -261,7 +278,27 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     const double C0 = (1 - P) / N;
     auto costs = [&](int l) { return dir_auto ? c->ext_stats.p + prh::kCostSums * (l & 1) : nullptr; };
     reset_progress(c);
-    for (int l = 0; l < L; ++l) {
+    if (small) {
+      sm.rank[0] = c->rank[0].p;
+      sm.rank[1] = c->rank[1].p;
+      sm.off = g->l_in_off;
+      sm.src = g->l_in_src;
+      sm.deg = g->l_outdeg;
+      sm.vaff = c->vaff.p;
+      sm.C0 = C0;
+      sm.P = P;
+      sm.D = o->frontier_tolerance;
+      sm.C = o->prune_tolerance;
+      sm.tol = o->tolerance;
+      sm.host = c->progress;
+    }
+    for (int l = 0; small && l < L && !loop_stopped(c); l = sm.last) {
+      sm.first = l;
+      sm.last = L - l > prh::kSmallIterations ? l + prh::kSmallIterations : L;
+      PRH_HIP(c, prh::launch_small_solve(variant, sm, s));
+      PRH_CHECK(wait_progress(c, sm.last));
+    }
+    for (int l = 0; !small && l < L; ++l) {
       PRH_CHECK(wait_progress(c, l - ahead + 1));
       if (loop_stopped(c)) break;
       const prh::LoopCtl ctl{err, done, l, L, o->tolerance, c->progress};

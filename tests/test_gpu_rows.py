@@ -42,3 +42,39 @@ def test_row_classes(ctx, oracle_mod, n, method):
     if res.iterations == it:
         assert np.all(np.abs(res.ranks - ref) <= 6e-11 * ref)
     assert np.abs(res.ranks - ref).max() <= 1e-9
+
+
+def small_graph(n: int, seed: int):
+    """The first rows have the degrees of DEGREES that n allows, up to 1025 (in all 12,000 edges); the rest 1 to 3."""
+    from pagerank_amd import HostGraph
+    rng = np.random.RandomState(seed)
+    src, dst = [rng.randint(0, n, 2 * n)], [np.arange(2 * n) % n]
+    for i, d in enumerate([d for d in DEGREES if d <= min(1025, n // 2)]):
+        src.append((i + 1 + rng.randint(0, n - d) + np.arange(d - 1)) % n)
+        dst.append(np.full(d - 1, i))
+    return HostGraph.from_edges(n, np.concatenate(src).astype(np.uint32), np.concatenate(dst).astype(np.uint32))
+
+
+@pytest.mark.parametrize("method", range(5), ids=["static", "ND", "DT", "DF", "DFP"])
+@pytest.mark.parametrize("n", [1, 63, 65, 1023, 1100, 2049, 2900, 3600, 5800])
+def test_small_graphs(ctx, oracle_mod, n, method):
+    """Sizes on both sides of what one workgroup's LDS holds. The bound is test_row_classes' with sums of at most 1,100
+    terms: 1.6e-12. Then 600 iterations at tolerance 0, which take several launches."""
+    from pagerank_amd import Batch, PagerankOptions, apply_batch, solve
+    x = small_graph(n, n)
+    q, _, _ = oracle_mod.pagerank_cuda(oracle_mod.STATIC, x)
+    b = Batch.random(x, max(1, n // 100), 0.8, seed=3) if n > 1 else Batch.empty()
+    y = apply_batch(x, b)
+    yg = ctx.upload(y)
+    args = (b if method else None, q if method else None)
+    print(f"[small] N={y.N} M={y.M} method={method}", flush=True)
+    for tolerance, iterations in ((1e-10, 500), (0.0, 600)):
+        o = PagerankOptions(tolerance=tolerance, maxIterations=iterations)
+        res = solve(yg, method, o, batch=args[0], q=args[1])
+        ref, it, _ = oracle_mod.pagerank_cuda(method, y, *args, tolerance=tolerance, max_iterations=iterations)
+        assert abs(res.iterations - it) <= 1 and (tolerance or res.iterations == it)
+        if res.iterations == it:
+            assert np.all(np.abs(res.ranks - ref) <= 1.6e-12 * ref)
+        assert np.abs(res.ranks - ref).max() <= 1e-9
+        again = solve(yg, method, o, batch=args[0], q=args[1])
+        assert np.array_equal(again.ranks, res.ranks)
