@@ -92,9 +92,10 @@ typedef struct prh_tuning {
                              source u in slice (u / 16) mod source_slices, slice x on the workgroups b with
                              b mod source_slices = x (8: one slice per XCD and its L2) [0] */
   uint32_t block_edges;   /* edges per workgroup of the rank kernels, fewer on small graphs (>= 256) [2048] */
-  int extension_direction; /* DF / DF-P extension: 0 push along out-edges of frontier vertices; 1 push or pull
-                              (unaffected rows look for a frontier in-neighbour), whichever the last rank launch
-                              found cheaper; 2 pull. The flags, hence the results, are the same for all [1] */
+  int extension_direction; /* DF / DF-P extension: 0 push along out-edges of frontier vertices; 1 pull
+                              (unaffected rows look for a frontier in-neighbour) within the next rank launch up to
+                              2^24 edges, above that push or pull, whichever the last rank launch found cheaper;
+                              2 pull. The flags, hence the results, are the same for all [1] */
   int blocking;            /* every method, the weighted solves too: 0 = pull kernels above; 1024, 2048, 4096,
                               8192 or 16384 = propagation blocking with source blocks and destination bins of this
                               many vertices (each iteration expands contributions through LDS into a buffer with

@@ -540,8 +540,9 @@ int build_rank_plan(prh_context *c, prh_graph *g) {
   g->plan_valid = false;
   PRH_CHECK(dev_alloc(c, reinterpret_cast<void **>(&g->chunk_tables), tb));
   g->chunk_tables_bytes = tb;
-  PRH_CHECK(dev_alloc(c, reinterpret_cast<void **>(&g->chunk_partial), std::max<size_t>(16, size_t(n_items) * 8)));
-  g->chunk_partial_bytes = std::max<size_t>(16, size_t(n_items) * 8);
+  const size_t pb = std::max<size_t>(16, size_t(n_items) * 12);  // sums, then the items' frontier flags
+  PRH_CHECK(dev_alloc(c, reinterpret_cast<void **>(&g->chunk_partial), pb));
+  g->chunk_partial_bytes = pb;
   uint32_t *tp = g->chunk_tables;
   if (n_items) {
     PRH_HIP(c, hipMemcpy(tp, item_row.data(), size_t(n_items) * 4, hipMemcpyHostToDevice));
@@ -555,6 +556,7 @@ int build_rank_plan(prh_context *c, prh_graph *g) {
   p.item_end = tp + 2 * size_t(n_items);
   p.row_first = tp + 3 * size_t(n_items);
   p.partial = g->chunk_partial;
+  p.hit = reinterpret_cast<uint32_t *>(g->chunk_partial + n_items);
   p.n_chunked = n_chunked;
   add(prh::kChunkedRows, 0, 0, n_items, 1, n_items);
   // Block rows, then wave rows.

@@ -74,9 +74,11 @@ struct RankPlan {
   int nsec;
   uint32_t blocks;
   // Chunked rows (the heaviest in-degrees, rows 0..n_chunked-1): item i covers edges [item_beg[i], item_end[i]) of
-  // row item_row[i] and leaves its sum in partial[i]; row r owns items [row_first[r], row_first[r+1]).
+  // row item_row[i] and leaves its sum in partial[i] (and in hit[i] whether it saw the last frontier, where the launch
+  // extends it: RankArgs::prev); row r owns items [row_first[r], row_first[r+1]).
   const uint32_t *item_row, *item_beg, *item_end, *row_first;
   double *partial;
+  uint32_t *hit;
   uint32_t n_chunked;
 };
 
@@ -100,6 +102,10 @@ struct RankArgs {
   // Weighted variants: the teleport share s (forward) or the seed g (adjoint), and the out-weight sums W; there a
   // holds the new values, ca the new gathered values (a / W forward, a adjoint), cr the old ones.
   const double *term = nullptr, *W = nullptr;
+  // Frontier variants on the row plan, optional: the neighbour-affected flags of the iteration before.
+  // The launch then does that iteration's extension itself (a row not affected becomes so if an in-neighbour has the
+  // flag); naff is another buffer.
+  const uint8_t *prev = nullptr;
 };
 
 struct ExtendArgs {

@@ -135,6 +135,30 @@ __device__ __forceinline__ double block_gather_sum(const uint32_t *src, const do
   return t;
 }
 
+// Whether an in-neighbour among edges b + i, b + i + STEP, ... < e was in the last iteration's frontier.
+template <int STEP>
+__device__ __forceinline__ bool any_frontier(const uint8_t *prev, const uint32_t *src, uint32_t b, uint32_t e,
+                                             uint32_t i) {
+  src += b;
+  e -= b;
+  uint32_t hit = 0;
+  for (; i < e && !hit; i += 4 * STEP) {
+    uint32_t u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = k * STEP < e - i ? src[i + k * STEP] : 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) hit |= k * STEP < e - i ? prev[u[k]] : 0u;
+  }
+  return hit != 0;
+}
+
+// After the update of a row that the extension within this launch (RankArgs::prev) made affected.
+template <int VARIANT>
+__device__ __forceinline__ void keep_fresh(const RankArgs &A, uint32_t v, bool fresh, const RowFlags &f) {
+  if constexpr (Traits<VARIANT>::frontier)
+    if (fresh && f.affected) A.vaff[v] = 1;
+}
+
 // One workgroup per chunk item: its partial sum goes to the item's slot; rows are finished by
 // finish_chunked_kernel after this launch (the kernel boundary makes every chunk's partial visible).
 template <int VARIANT>
@@ -143,9 +167,16 @@ __device__ __forceinline__ void chunked_rows(const RankArgs &A, const RankPlan &
   const uint32_t ib = S.begin + blk * S.per_block, ie = min(S.end, ib + S.per_block);
   for (uint32_t it = ib; it < ie; ++it) {  // block-uniform
     const uint32_t v = P.item_row[it];
-    if (!affected<VARIANT>(A, v)) continue;
-    const double t = block_gather_sum(A.src, A.cr, P.item_beg[it], P.item_end[it], lds);
-    if (threadIdx.x == 0) P.partial[it] = t;
+    const bool test = Traits<VARIANT>::frontier && A.prev;  // a row not affected: its sum may be needed all the same
+    const bool upd = affected<VARIANT>(A, v);
+    if (!upd && !test) continue;
+    const uint32_t b = P.item_beg[it], e = P.item_end[it];
+    const double t = block_gather_sum(A.src, A.cr, b, e, lds);
+    const bool hit = test && !upd && __syncthreads_or(any_frontier<kBlock>(A.prev, A.src, b, e, threadIdx.x)) != 0;
+    if (threadIdx.x == 0) {
+      P.partial[it] = t;
+      if (test) P.hit[it] = hit;
+    }
   }
 }
 
@@ -155,12 +186,18 @@ __device__ __forceinline__ void block_rows(const RankArgs &A, const RankSection 
                                            double &emax, CostAcc &cost) {
   const uint32_t rb = S.begin + blk * S.per_block, re = min(S.end, rb + S.per_block);
   for (uint32_t v = rb; v < re; ++v) {  // block-uniform
-    const RowOperands o = row_operands<VARIANT>(A, v);
+    RowOperands o = row_operands<VARIANT>(A, v);
     RowFlags f;
+    bool fresh = false;
+    if constexpr (Traits<VARIANT>::frontier) {
+      if (A.prev && !o.upd)
+        o.upd = fresh = __syncthreads_or(any_frontier<kBlock>(A.prev, A.src, o.b, o.e, threadIdx.x)) != 0;
+    }
     const double t = o.upd ? block_gather_sum(A.src, A.cr, o.b, o.e, lds) : 0.0;
     if (threadIdx.x == 0) {
       if (o.upd) {
         emax = fmax(emax, finish_vertex<VARIANT>(A, v, t, o.d, o.rv, o.crv, f));
+        keep_fresh<VARIANT>(A, v, fresh, f);
       } else {
         copy_vertex<VARIANT>(A, v, o.rv, o.crv);
         f.affected = false;
@@ -176,8 +213,13 @@ __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   const uint32_t rb = S.begin + blk * S.per_block, re = min(S.end, rb + S.per_block);
   for (uint32_t v = rb + w; v < re; v += kWavesPerBlock) {  // wave-uniform
-    const RowOperands o = row_operands<VARIANT>(A, v);
+    RowOperands o = row_operands<VARIANT>(A, v);
     RowFlags f;
+    bool fresh = false;
+    if constexpr (Traits<VARIANT>::frontier) {
+      if (A.prev && !o.upd)
+        o.upd = fresh = __ballot(any_frontier<kWave>(A.prev, A.src, o.b, o.e, lane)) != 0;
+    }
     if (!o.upd) {
       if (lane == 0) {
         copy_vertex<VARIANT>(A, v, o.rv, o.crv);
@@ -189,6 +231,7 @@ __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &
     const double acc = group_sum<kWave>(gather_sum<kWave>(A.src, A.cr, o.b, o.e, lane));
     if (lane == 0) {
       emax = fmax(emax, finish_vertex<VARIANT>(A, v, acc, o.d, o.rv, o.crv, f));
+      keep_fresh<VARIANT>(A, v, fresh, f);
       cost.add(f, o.e - o.b, o.d);
     }
   }
@@ -206,15 +249,23 @@ __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection 
     const bool valid = v < re;
     RowOperands o{};
     double acc = 0.0;
-    if (valid) {
-      o = row_operands<VARIANT>(A, v);
-      if (o.upd) acc = group_gather_sum<W>(A.src, A.cr, o.b, o.e, j);
+    bool fresh = false;
+    if (valid) o = row_operands<VARIANT>(A, v);
+    if constexpr (Traits<VARIANT>::frontier) {
+      if (A.prev) {
+        const unsigned long long hits =
+            __ballot(valid && !o.upd && any_frontier<W>(A.prev, A.src, o.b, o.e, j));
+        fresh = (hits >> (g * W) & ((1ull << W) - 1)) != 0;
+        o.upd = o.upd || fresh;
+      }
     }
+    if (valid && o.upd) acc = group_gather_sum<W>(A.src, A.cr, o.b, o.e, j);
     acc = group_sum<W>(acc);  // all lanes active again here
     if (valid && j == 0) {
       RowFlags f;
       if (o.upd) {
         emax = fmax(emax, finish_vertex<VARIANT>(A, v, acc, o.d, o.rv, o.crv, f));
+        keep_fresh<VARIANT>(A, v, fresh, f);
       } else {
         copy_vertex<VARIANT>(A, v, o.rv, o.crv);
         f.affected = false;
@@ -267,7 +318,15 @@ __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, Rank
   for (uint32_t v = blockIdx.x * kWavesPerBlock + w; v < n_rows; v += gridDim.x * kWavesPerBlock) {
     const uint32_t in_deg = A.off[v + 1] - A.off[v], d = A.deg[v];
     RowFlags f;
-    if (!affected<VARIANT>(A, v)) {
+    bool upd = affected<VARIANT>(A, v), fresh = false;
+    if constexpr (Traits<VARIANT>::frontier) {
+      if (A.prev && !upd) {
+        uint32_t hit = 0;
+        for (uint32_t k = P.row_first[v] + lane; k < P.row_first[v + 1]; k += kWave) hit |= P.hit[k];
+        upd = fresh = __ballot(hit != 0) != 0;
+      }
+    }
+    if (!upd) {
       if (lane == 0) {
         copy_vertex<VARIANT>(A, v);
         f.affected = false;
@@ -280,6 +339,7 @@ __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, Rank
     s = group_sum<kWave>(s);
     if (lane == 0) {
       emax = fmax(emax, finish_vertex<VARIANT>(A, v, s, d, A.r[v], Traits<VARIANT>::prune ? A.cr[v] : 0.0, f));
+      keep_fresh<VARIANT>(A, v, fresh, f);
       cost.add(f, in_deg, d);
     }
   }

@@ -153,6 +153,14 @@ static int load_initial_ranks(prh_context *c, const prh_graph *g, const double *
   return PRH_SUCCESS;
 }
 
+// Edges up to which a row plan's frontier extension (direction chosen by the library) is part of the next iteration's
+// update, whose unaffected rows look at their in-neighbours' flags (RankArgs::prev), instead of a launch of its own for
+// which the update sums what either direction would cost. Per solve, launch of its own -> inside: RMAT, 16 edges a vertex,
+// DF: 5,000 vertices 794 -> 523 us, 64K 1019 -> 729; 20 edges: 200K 1720 -> 1262, 1M 5.74 -> 5.17 ms; DF-P at 1M with 1e-3
+// of the edges changed 4.25 -> 4.24. Grids, where ten changed edges leave nearly all rows unaffected to the end: 1.2M edges
+// 562 -> 324 us, 11.2M 1154 -> 937. Both sides meet at about 20M edges (40M, DF-P: 8.3 -> 8.7 ms).
+constexpr uint64_t kExtendInside = uint64_t(1) << 24;
+
 // The bands and items of a small graph's solve; false if the graph does not fit. (That the ids' 16-bit byte offsets hold
 // every vertex follows from the size of LDS.)
 static bool small_plan(const prh_graph *g, prh::SmallArgs &A) {
@@ -245,7 +253,8 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   // Extension direction (frontier variants): 0 push only, 1 chosen per iteration from the rank launch's costs,
   // 2 pull only. The pull form splits rows at in-degree 64 (a wave each) and 4 (8 lanes each).
   const int dir_mode = frontier ? c->tuning.extension_direction : 0;
-  const bool dir_auto = dir_mode == 1 && !binned;
+  const bool inside = dir_mode == 1 && !binned && !window && g->M <= kExtendInside;
+  const bool dir_auto = dir_mode == 1 && !binned && !small && !inside;
   if (dir_auto) PRH_CHECK(ensure(c, c->ext_stats, 2 * prh::kCostSums));  // the sums of two iterations in turn
   const prh::PullArgs pull{c->vaff.p, c->naff.p, g->l_in_off, g->l_in_src, layout_rows_above(g, 64),
                            layout_rows_above(g, 4), N};
@@ -257,7 +266,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     // The out-degree schedule serves the traversal levels and the row plan's frontier extension; the initial
     // extension runs from the batch list and the blocked plan extends inside its update.
     prh::ExtendArgs xo{};
-    if (dynamic && (method == PRH_DYNAMIC_TRAVERSAL || (frontier && !binned && !small))) {
+    if (dynamic && (method == PRH_DYNAMIC_TRAVERSAL || (frontier && !binned && !small && !inside))) {
       PRH_CHECK(out_schedule(c, gm, xo));
       if (account_prep) prep += gm->out_prep.take();
     }
@@ -305,6 +314,11 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       prh::RankArgs A{c->rank[(l + 1) & 1].p, c->rank[l & 1].p, c->contrib[(l + 1) & 1].p, c->contrib[l & 1].p,
                       c->naff.p, c->vaff.p, g->l_in_off, g->l_in_src, g->l_outdeg, C0, P, o->frontier_tolerance,
                       o->prune_tolerance, costs(l)};
+      if (inside) {  // the flags of two iterations in turn (the second buffer is the traversal levels')
+        uint8_t *const flags[2] = {c->naff.p, c->buff.p};
+        A.naff = flags[l & 1];
+        A.prev = l ? flags[(l - 1) & 1] : nullptr;
+      }
       if (c->ktiming) PRH_HIP(c, hipEventRecord(c->kev[2 * l], s));
       hipEvent_t mark = c->ktiming ? c->kev[2 * l + 1] : nullptr;
       if (binned)
@@ -314,7 +328,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
         if (mark) PRH_HIP(c, hipEventRecord(mark, s));
       } else if (sliced) PRH_HIP(c, prh::launch_sliced_update(A, g->sliced, ctl, s, mark));
       else PRH_HIP(c, prh::launch_rank_update(variant, A, plan, ctl, s, mark));
-      if (frontier && !binned) {  // the blocked plan extends inside the next iteration's update
+      if (frontier && !binned && !inside) {  // else the extension is inside the next iteration's update
         prh::ExtendArgs E = xo;
         E.vaff = c->vaff.p;
         E.naff = c->naff.p;

@@ -78,3 +78,29 @@ def test_small_graphs(ctx, oracle_mod, n, method):
         assert np.abs(res.ranks - ref).max() <= 1e-9
         again = solve(yg, method, o, batch=args[0], q=args[1])
         assert np.array_equal(again.ranks, res.ranks)
+
+
+@pytest.mark.parametrize("method", [3, 4], ids=["DF", "DFP"])
+@pytest.mark.parametrize("edges", [2, 300])
+def test_extension_inside_the_update(ctx, method, edges):
+    """The extension within the update (direction 1 at this size) sets the flags that push and pull set, in rows of every
+    class: the ranks are the same bit for bit."""
+    from pagerank_amd import Batch, apply_batch, solve
+    x = degree_graph(40003, 9)
+    q = solve(ctx.upload(x), 0).ranks
+    b = Batch.random(x, edges, 0.8, seed=5)
+    yg = ctx.upload(apply_batch(x, b))
+    old = ctx.get_tuning()
+    out = {}
+    try:
+        for d in (0, 1, 2):
+            print(f"[inside] method={method} edges={edges} direction={d}", flush=True)
+            t = ctx.get_tuning()
+            t.extension_direction = d
+            ctx.set_tuning(t)
+            out[d] = solve(yg, method, batch=b, q=q)
+    finally:
+        ctx.set_tuning(old)
+    for d in (1, 2):
+        assert out[d].iterations == out[0].iterations
+        assert np.array_equal(out[d].ranks, out[0].ranks), d
