@@ -116,15 +116,16 @@ __device__ __forceinline__ void overlay_expand(const BinnedPlan &P, const double
 template <int B, bool FROM_RANKS>
 __global__ __launch_bounds__(kBinBlock) void expand_kernel(BinnedPlan P, const double *cr, const double *r,
                                                            const uint32_t *deg, const uint8_t *naff, LoopCtl ctl) {
-  if (!iteration_begin(ctl)) return;
-  if (iter_index(ctl) == 0) naff = nullptr;  // the first iteration extends nothing (the marking did)
+  const uint4 it = P.ex_item[blockIdx.x < P.n_ex ? blockIdx.x : 0];  // block, first entry, end entry
+  const LoopState st = loop_state(ctl, it.y > it.z);
+  if (!iteration_begin(ctl, st)) return;
+  if (st.l == 0) naff = nullptr;  // the first iteration extends nothing (the marking did)
   if (blockIdx.x >= P.n_ex) {
     overlay_expand<FROM_RANKS>(P, cr, r, deg, naff, blockIdx.x - P.n_ex, gridDim.x - P.n_ex);
     report_begun(ctl);
     return;
   }
   __shared__ double c[B];
-  const uint4 it = P.ex_item[blockIdx.x];  // block, first entry, end entry
   const uint32_t base = it.x * uint32_t(B);
   const uint32_t n = min(uint32_t(B), P.N - base);
   // Pairs of entries: thread t takes pairs p = t + m * kBinBlock of the even-aligned range (16-byte stores, with the
@@ -253,7 +254,9 @@ __device__ __forceinline__ void add_slots(double *sum, uint8_t *ext, uint32_t d,
 // DF-P on 1.5M vertices (B = 2048, 93 SGPRs before) 46 against 67 us, weighted forward on 1M vertices 39 against 49 us.
 template <int B, int VARIANT>
 __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) void accumulate_kernel(RankArgs A, BinnedPlan P, LoopCtl ctl) {
-  if (!iteration_begin(ctl)) return;
+  const uint4 it = P.ac_item[blockIdx.x];  // bin, first slot, end slot, partial row (kWholeBin: none)
+  const LoopState st = loop_state(ctl, it.y > it.z);
+  if (!iteration_begin(ctl, st)) return;
   constexpr int kAccGroups = acc_groups<VARIANT>();
   constexpr bool EXT = Traits<VARIANT>::frontier;
   constexpr bool WEIGHTED = Traits<VARIANT>::weighted;
@@ -261,12 +264,6 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
   constexpr bool kDeadBit = B <= 8192;
   __shared__ double sum[B];
   __shared__ uint8_t ext[EXT ? B : 1];
-  const uint4 it = P.ac_item[blockIdx.x];  // bin, first slot, end slot, partial row (kWholeBin: none)
-  for (uint32_t i = threadIdx.x; i < uint32_t(B); i += kBinBlock) {
-    sum[i] = 0.0;
-    if constexpr (EXT) ext[i] = 0;
-  }
-  __syncthreads();
   const int w = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x & (kWave - 1);
   // Groups of 64 slots aligned to multiples of 64 (the slot array is padded to a multiple of 64), dealt to the
@@ -274,20 +271,26 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
   // X loads are issued, then the next batch's table and slot loads, so that the wait for X overlaps them. Loads of
   // groups past the item's end read the batch's first group again (always in bounds) and are not added.
   uint32_t g = __builtin_amdgcn_readfirstlane((it.y & ~63u) + uint32_t(w) * kWave);  // wave-uniform
-  if (g < it.z) {
-    uint4 t[kAccGroups];
-    uint32_t d[kAccGroups];
-    float wt[kAccGroups];  // weighted variants: the slots' weights (an item's last one past its end)
-    auto fetch = [&](uint32_t gb, uint32_t gv) {  // batch at gb; gv: a group start below it.z
+  uint4 t[kAccGroups];
+  uint32_t d[kAccGroups];
+  float wt[kAccGroups];  // weighted variants: the slots' weights (an item's last one past its end)
+  auto fetch = [&](uint32_t gb, uint32_t gv) {  // batch at gb; gv: a group start below it.z
 #pragma unroll
-      for (int u = 0; u < kAccGroups; ++u) {
-        const uint32_t gu = gb + u * kBinBlock < it.z ? gb + u * kBinBlock : gv;
-        t[u] = P.grp[gu >> 6];
-        d[u] = ld_nt(P.dst16 + gu + lane);
-        if constexpr (WEIGHTED) wt[u] = __builtin_nontemporal_load(P.ws + min(gu + lane, it.z - 1));
-      }
-    };
-    fetch(g, g);
+    for (int u = 0; u < kAccGroups; ++u) {
+      const uint32_t gu = gb + u * kBinBlock < it.z ? gb + u * kBinBlock : gv;
+      t[u] = P.grp[gu >> 6];
+      d[u] = ld_nt(P.dst16 + gu + lane);
+      if constexpr (WEIGHTED) wt[u] = __builtin_nontemporal_load(P.ws + min(gu + lane, it.z - 1));
+    }
+  };
+  // The first batch is on its way while the sums are cleared.
+  if (g < it.z) fetch(g, g);
+  for (uint32_t i = threadIdx.x; i < uint32_t(B); i += kBinBlock) {
+    sum[i] = 0.0;
+    if constexpr (EXT) ext[i] = 0;
+  }
+  __syncthreads();
+  if (g < it.z) {
     for (; g < it.z; g += kAccGroups * kBinBlock) {
       uint32_t dc[kAccGroups], k[kAccGroups];
       double x[kAccGroups];
@@ -348,9 +351,10 @@ __global__ __launch_bounds__(kBinBlock) __attribute__((amdgpu_num_sgpr(80))) voi
 //           sums in wave order (bins with many rows).
 template <int VARIANT>
 __global__ __launch_bounds__(kBinBlock) void finish_bins_kernel(RankArgs A, BinnedPlan P, LoopCtl ctl) {
-  if (!iteration_begin(ctl)) return;
-  __shared__ double part[kBinWaves][kWave];
   const uint4 m = P.multi[blockIdx.x];
+  const LoopState st = loop_state(ctl, m.z == 0);
+  if (!iteration_begin(ctl, st)) return;
+  __shared__ double part[kBinWaves][kWave];
   const bool split = (m.w >> 31) != 0;
   const uint32_t first = m.w & 0x7FFFFFFFu;
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);

@@ -103,20 +103,32 @@ __device__ __forceinline__ void tell_host(int *p, int v) {
 // Entry test for the first kernel of iteration l; all threads of a block agree.
 // done and err[l-1] were last written by earlier launches, whose completion made them visible: plain loads (both
 // issued together) suffice. A volatile read here would be a system-scope load at the start of every wave.
-__device__ __forceinline__ bool iteration_begin(const LoopCtl &c) {
-  const int done = *c.done;
-  const int l = iter_index(c);
-  const double e = l > 0 ? __longlong_as_double((long long)c.err[l - 1]) : c.tol;
-  if (done || l >= c.max_iter) return false;
-  if (e < c.tol) {
+// The test needs two loads; a workgroup's item can be loaded with them instead of after the test. `broken`, never true, is
+// a condition on the item: it keeps the compiler from moving the item's load behind the test. (An empty asm statement in its
+// place made the later uniform loads vector loads: RMAT-20, blocked, 3.60 -> 4.17 ms per solve.) Blocked plan, per solve,
+// test first -> together, and accumulate's first batch before its sums are cleared: RMAT-20 3.59 -> 3.46 ms, RMAT-24
+// 40.6 -> 40.4, weighted forward and backward on RMAT-20 9.79 -> 9.48.
+struct LoopState {
+  int done, l;
+  double e;
+};
+__device__ __forceinline__ LoopState loop_state(const LoopCtl &c, bool broken = false) {
+  const int done = *c.done, l = iter_index(c);
+  return {done | int(broken), l, l > 0 ? __longlong_as_double((long long)c.err[l - 1]) : c.tol};
+}
+
+__device__ __forceinline__ bool iteration_begin(const LoopCtl &c, const LoopState &s) {
+  if (s.done || s.l >= c.max_iter) return false;
+  if (s.e < c.tol) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-      *(volatile int *)c.done = l;
-      if (c.host) tell_host(c.host + 1, l);
+      *(volatile int *)c.done = s.l;
+      if (c.host) tell_host(c.host + 1, s.l);
     }
     return false;
   }
   return true;
 }
+__device__ __forceinline__ bool iteration_begin(const LoopCtl &c) { return iteration_begin(c, loop_state(c)); }
 
 // The first kernel of an iteration tells the host that it has run, at its end: a store before the kernel's loads would
 // keep the compiler from making the uniform ones scalar (RMAT-20, blocked: 3.79 -> 4.41 ms per solve).
