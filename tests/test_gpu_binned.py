@@ -115,3 +115,30 @@ def test_binned_repeats_to_rounding(ctx):
     b = _with_blocking(ctx, 1024, lambda: pagerankStaticHip(yg))
     assert abs(a.iterations - b.iterations) <= 1
     assert np.abs(a.ranks - b.ranks).max() <= 1e-12
+
+
+@pytest.mark.parametrize("method", [0, 4], ids=["static", "DFP"])
+@pytest.mark.parametrize("rows", [2, 3, 8, 9, 16, 17, 24, 33, 130])
+def test_partial_rows_of_a_split_bin(ctx, oracle_mod, rows, method):
+    """The heaviest bin is split into `rows` items of at most 16384 slots (M stays below 512 times that), whose partial
+    rows are added eight at a time, by a thread each up to 16 rows and by 16 waves above. Sums of at most 2,100 non-negative
+    terms in two orders differ by 2 * 2100 * 2^-53 of the sum, which the iteration amplifies by 1 / (1 - 0.85): 3.2e-12."""
+    from pagerank_amd import Batch, HostGraph, apply_batch, solve
+    n, B = 20000, 1024
+    edges = 16384 * rows - 8000
+    d = np.full(B, edges // B)
+    d[: edges % B] += 1
+    dst = np.repeat(np.arange(B), d - 1)
+    k = np.arange(len(dst)) - np.repeat(np.cumsum(d - 1) - (d - 1), d - 1)
+    x = HostGraph.from_edges(n, ((dst + 1 + k) % n).astype(np.uint32), dst.astype(np.uint32))
+    q, _, _ = oracle_mod.pagerank_cuda(oracle_mod.STATIC, x)
+    b = Batch.random(x, 50, 0.8, seed=3)
+    y = apply_batch(x, b)
+    args = dict(batch=b, q=q) if method else {}
+    print(f"[binned] rows={rows} method={method} M={y.M}", flush=True)
+    res = _with_blocking(ctx, B, lambda: solve(ctx.upload(y), method, **args))
+    ref, it, _ = oracle_mod.pagerank_cuda(method, y, *((b, q) if method else ()))
+    assert abs(res.iterations - it) <= 1
+    if res.iterations == it:
+        assert np.all(np.abs(res.ranks - ref) <= 3.2e-12 * ref)
+    assert np.abs(res.ranks - ref).max() <= RANK_TOL
