@@ -279,7 +279,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
     if (dynamic) PRH_CHECK(mark_affected(c, g, method, b, xo));
     PRH_HIP(c, hipEventRecord(c->ev[2], s));
     // Iterations.
-    PRH_HIP(c, prh::launch_fill_u64(err, 0ull, size_t(L) + 1, s));
+    if (!small) PRH_HIP(c, prh::launch_fill_u64(err, 0ull, size_t(L) + 1, s));
     if (dir_auto)
       PRH_HIP(c, prh::launch_fill_u64(reinterpret_cast<unsigned long long *>(c->ext_stats.p), 0ull,
                                       2 * prh::kCostSums, s));
@@ -341,9 +341,20 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       }
     }
     PRH_HIP(c, hipEventRecord(c->ev[3], s));
-    PRH_HIP(c, hipEventSynchronize(c->ev[3]));
     int n = 0;
     PRH_CHECK(end_loop(c, L, &n));
+    // Final ranks are in the buffer written by the last iteration (pagerankCuda.hxx:688, :826); back to the caller's
+    // vertex order (scatter through perm), as the reference scatters to span (:827). The device has told how many
+    // iterations it took, so these launches go out before the host waits for anything.
+    if (rep + 1 == o->repeat) {
+      const double *res = c->rank[n & 1].p;
+      double *to = host ? c->contrib[(n + 1) & 1].p : ranks;
+      PRH_HIP(c, prh::launch_scatter_f64(res, g->perm, N, to, s));
+      if (host) PRH_CHECK(copy_to_host(c, ranks, to, size_t(N) * 8));
+      else PRH_HIP(c, hipStreamSynchronize(s));
+    } else {
+      PRH_HIP(c, hipEventSynchronize(c->ev[3]));
+    }
     float t01 = 0, t12 = 0, t23 = 0;
     PRH_HIP(c, hipEventElapsedTime(&t01, c->ev[0], c->ev[1]));
     PRH_HIP(c, hipEventElapsedTime(&t12, c->ev[1], c->ev[2]));
@@ -361,17 +372,6 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       }
     }
   }
-  // Final ranks are in the buffer written by the last iteration (pagerankCuda.hxx:688, :826); back to the
-  // caller's vertex order (scatter through perm), as the reference scatters to span (:827).
-  const double *res = c->rank[iterations & 1].p;
-  if (host) {
-    double *tmp = c->contrib[(iterations + 1) & 1].p;
-    PRH_HIP(c, prh::launch_scatter_f64(res, g->perm, N, tmp, s));
-    PRH_CHECK(copy_to_host(c, ranks, tmp, size_t(N) * 8));
-  } else {
-    PRH_HIP(c, prh::launch_scatter_f64(res, g->perm, N, ranks, s));
-  }
-  PRH_HIP(c, hipStreamSynchronize(s));
   stats.iterations = iterations;
   stats.initialization_time = float(ti / o->repeat) + prep;
   stats.marking_time = float(tm / o->repeat);
