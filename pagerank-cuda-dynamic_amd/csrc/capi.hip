@@ -376,7 +376,10 @@ int prh_graph_create(prh_context *c, uint32_t N, uint64_t M, const uint32_t *in_
     }
   }
   if (st == PRH_SUCCESS)
-    for (uint32_t v = 0; v < N; ++v) g->dead_ends += outdeg[v] == 0;
+    for (uint32_t v = 0; v < N; ++v) {
+      g->dead_ends += outdeg[v] == 0;
+      g->max_outdeg = std::max(g->max_outdeg, outdeg[v]);
+    }
   if (st == PRH_SUCCESS) st = build_layout(c, g, in_off, outdeg, out_off != nullptr);
   if (st != PRH_SUCCESS) {
     prh_graph_destroy(g);

@@ -148,7 +148,8 @@ struct prh_graph {
   uint32_t *l_in_off = nullptr, *l_in_src = nullptr, *l_outdeg = nullptr, *l_out_off = nullptr, *l_out_dst = nullptr;
   std::vector<uint32_t> sorted_deg;  // host: in-degree of layout row i (descending when layout == 0)
   int layout = 0;                    // 0: rows by in-degree, descending; 1: the caller's vertex order
-  uint32_t dead_ends = 0;  // vertices with out-degree 0
+  uint32_t dead_ends = 0;   // vertices with out-degree 0
+  uint32_t max_outdeg = 0;  // largest out-degree uploaded (without an out-CSR any value: nothing bounds it by M)
   // In-place updates (prh_graph_update): once one has run, the caller-order arrays above are freed (the batched and
   // weighted solvers then refuse the graph); the layout's out-rows are kept ascending for the batch tidy.
   bool updated = false, out_sorted = false;

@@ -162,9 +162,12 @@ static int load_initial_ranks(prh_context *c, const prh_graph *g, const double *
 constexpr uint64_t kExtendInside = uint64_t(1) << 24;
 
 // The bands and items of a small graph's solve; false if the graph does not fit. (That the ids' 16-bit byte offsets hold
-// every vertex follows from the size of LDS.)
+// every vertex follows from the size of LDS. The out-degrees are kept in 16 bits too; M bounds them only where the graph
+// came with its out-CSR, whose rows they are checked against.)
 static bool small_plan(const prh_graph *g, prh::SmallArgs &A) {
-  if (g->layout != 0 || g->updated || g->M > 65535 || prh::small_lds(g->N, 0, g->M / 256) > prh::kSmallLds) return false;
+  if (g->layout != 0 || g->updated || g->M > 65535 || g->max_outdeg > 65535 ||
+      prh::small_lds(g->N, 0, g->M / 256) > prh::kSmallLds)
+    return false;
   A.N = g->N;
   A.band[0] = A.item[0] = A.rounds = 0;
   for (int k = 0; k < 7; ++k) {

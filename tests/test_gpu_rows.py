@@ -80,6 +80,31 @@ def test_small_graphs(ctx, oracle_mod, n, method):
         assert np.array_equal(again.ranks, res.ranks)
 
 
+@pytest.mark.parametrize("method", [0, 1], ids=["static", "ND"])
+@pytest.mark.parametrize("largest", [65535, 65536, 65539, 1 << 24, (1 << 32) - 1])
+def test_small_graph_with_large_out_degrees(ctx, method, largest):
+    """Without an out-CSR nothing bounds the out-degrees by the edges (an in-graph that holds part of a larger one).
+    Twenty iterations against numpy in 64 bits, with test_small_graphs' bound."""
+    from pagerank_amd import HostGraph, PagerankOptions, solve
+    x = small_graph(900, 11)
+    deg = x.outdeg.copy()
+    deg[::7] = largest
+    deg[3::7] = np.minimum(largest, 65534)
+    y = HostGraph(arrays=dict(out_off=x.out_off, out_edg=x.out_edg, in_off=x.in_off, in_edg=x.in_edg, in_eid=x.in_eid,
+                              outdeg=deg))
+    q = np.random.RandomState(2).rand(y.N)
+    q /= q.sum()
+    print(f"[small] out-degrees up to {largest} method={method}", flush=True)
+    res = solve(ctx.upload(y, with_out=False), method, PagerankOptions(tolerance=0.0, maxIterations=20),
+                q=q if method else None)
+    row = np.repeat(np.arange(y.N), np.diff(y.in_off.astype(np.int64)))
+    r = q if method else np.full(y.N, 1.0 / y.N)
+    for _ in range(20):
+        r = 0.15 / y.N + 0.85 * np.bincount(row, (r / deg)[y.in_edg], y.N)
+    assert res.iterations == 20
+    assert np.all(np.abs(res.ranks - r) <= 1.6e-12 * r)
+
+
 @pytest.mark.parametrize("method", [3, 4], ids=["DF", "DFP"])
 @pytest.mark.parametrize("edges", [2, 300])
 def test_extension_inside_the_update(ctx, method, edges):
