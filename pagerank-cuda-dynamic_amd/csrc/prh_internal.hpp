@@ -13,7 +13,8 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 
 // Control of an iteration loop on the device (see prh_device.hpp).
 struct LoopCtl {
-  unsigned long long *err;  // [max iterations] FP64 bits, zeroed before the loop: 0 or kChanged
+  unsigned long long *err;  // [max_iter] FP64 bits, zeroed before the loop: 0 or kChanged. err[l - 1] is loaded before l
+                            // is tested, so a loop that launches indices l >= max_iter needs a word for each of them
   int *done;                // 0 while running, else the number of iterations performed
   int l;                    // this launch's iteration index, or -1 - i: index done[1] + i (replayed graphs, where the
                             // same launch serves many iterations and a device word holds the run's first index)

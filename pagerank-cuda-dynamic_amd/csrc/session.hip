@@ -92,6 +92,9 @@ struct prh_stream {
 namespace {
 
 constexpr int kStreamChunk = 4;  // iterations per replay of the iteration graph (even: ping-pong buffers realign)
+// Words of the session's err: a replay runs all its indices, also past the iteration cap, and the entry test loads
+// err[l - 1] together with the words that tell it to stop (prh_device.hpp). The last replay starts below the cap.
+size_t err_words(const prh_options &o) { return size_t(o.max_iterations) + kStreamChunk; }
 constexpr int kClosureLevels = 8;  // traversal levels per replay of the closure graph (even: its buffers realign)
 
 int stream_alloc(prh_stream *S, void **p, size_t bytes) {
@@ -186,7 +189,7 @@ int stream_apply_body(prh_stream *S, int p) {
   }
   // Solver initialisation (pagerankCuda.hxx:811-821): ranks from the previous batch's result (or 1/N for Static),
   // contributions with the new out-degrees, loop state cleared, and the DF initial marking on the new graph.
-  PRH_HIP(c, prh::launch_fill_u64(S->err, 0ull, size_t(S->opt.max_iterations) + 1, s));
+  PRH_HIP(c, prh::launch_fill_u64(S->err, 0ull, err_words(S->opt), s));
   PRH_HIP(c, prh::launch_init_ranks(S->rank[0], S->rank[1], S->contrib[0], S->contrib[1], S->outdeg, N,
                                     S->method != PRH_STATIC, s));
   if (S->variant >= prh::kTraversal) {
@@ -344,7 +347,7 @@ int prh_stream_create(prh_context *c, const prh_graph *g, prh_method method, con
   step(stream_alloc(S, &S->ext_cnt, 2 * size_t(max_batch) + 1));
   step(stream_alloc(S, &S->ext_start, 2 * size_t(max_batch) + 1));
   step(stream_alloc(S, &S->ctl, 4));
-  step(stream_alloc(S, &S->err, size_t(o.max_iterations) + 1));
+  step(stream_alloc(S, &S->err, err_words(o)));
   if (st == PRH_SUCCESS && hipHostMalloc(reinterpret_cast<void **>(&S->h_batch), (4 * size_t(max_batch) + 2) * 4) !=
                                hipSuccess) {
     (void)hipGetLastError();

@@ -59,6 +59,33 @@ def test_stream_matches_sequential_calls(ctx, oracle_mod, method, blocking):
         ctx.set_tuning(old)
 
 
+@pytest.mark.parametrize("blocking", [0, 1024], ids=["rows", "blocked"])
+@pytest.mark.parametrize("method", [4, 3, 1], ids=["DFP", "DF", "ND"])
+@pytest.mark.parametrize("cap", [1, 2, 3, 4, 5, 6, 7, 9])
+def test_stream_iteration_cap(ctx, oracle_mod, method, blocking, cap):
+    """Caps of every remainder of the iterations per replay, reached unconverged (tolerance 0): exactly `cap` iterations a
+    batch, and the ranks of the same method called with the same cap on the host-applied graph."""
+    from pagerank_amd import HostGraph, PagerankOptions, Stream, Tuning, solve
+    x = HostGraph.rmat(11, 8, seed=3)
+    q, _, _ = oracle_mod.pagerank_cuda(oracle_mod.STATIC, x)
+    seq = _sequence(x, 3, max(1, int(1e-2 * x.M)), 40)
+    o = PagerankOptions(tolerance=0.0, maxIterations=cap)
+    old = ctx.get_tuning()
+    ctx.set_tuning(Tuning(**{**old.__dict__, "blocking": blocking}))
+    try:
+        st = Stream(ctx.upload(x), method, o, max_batch=4096, initial_ranks=q)
+        for i, (b, y) in enumerate(seq):
+            print(f"[stream cap] method={method} blocking={blocking} cap={cap} batch={i}", flush=True)
+            got = st.update(b)
+            ref = solve(ctx.upload(y), method, o, batch=b, q=q)
+            assert got.iterations == cap and ref.iterations == cap
+            assert np.abs(got.ranks - ref.ranks).max() <= RANK_TOL, i
+            q = ref.ranks
+        st.close()
+    finally:
+        ctx.set_tuning(old)
+
+
 def test_stream_traversal_sets_match_oracle(ctx, oracle_mod):
     """DT through the stream: after each batch the ranks equal the oracle's DT solve on the host-applied graph, whose
     marking is the traversal closure (bit-exact with the reference's BFS closure, tests/test_oracle.py)."""
