@@ -126,18 +126,27 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
     PRH_HIP(c, prh::launch_ppr_advance(A, chunk, s));
     return PRH_SUCCESS;
   };
-  hipGraphExec_t exec = nullptr;
-  int status = L > 0 && c->capture ? capture_graph(c, iterations_chunk, &exec) : PRH_SUCCESS;
+  // The loop below ends on what the device tells from inside a replay, so the replay may still run: the graph goes when the
+  // stream has ended, on every way out.
+  struct Replay {
+    prh_context *c;
+    hipGraphExec_t exec = nullptr;
+    ~Replay() {
+      if (!exec) return;
+      if (hipStreamSynchronize(c->stream) != hipSuccess) (void)hipGetLastError();
+      (void)hipGraphExecDestroy(exec);
+    }
+  } replay{c};
+  int status = L > 0 && c->capture ? capture_graph(c, iterations_chunk, &replay.exec) : PRH_SUCCESS;
   prh::PprState hs{};
   // A run is launched when the one before it has begun its last iteration, so that the device goes on without waiting.
   reset_progress(c);
   for (int launched = 0; status == PRH_SUCCESS && launched < L && !loop_stopped(c); launched += chunk) {
-    if (!exec) status = iterations_chunk();
-    else if (const hipError_t e = hipGraphLaunch(exec, s); e != hipSuccess)
+    if (!replay.exec) status = iterations_chunk();
+    else if (const hipError_t e = hipGraphLaunch(replay.exec, s); e != hipSuccess)
       status = fail(c, PRH_ERROR_DEVICE, "batched iterations: %s", hipGetErrorString(e));
     if (status == PRH_SUCCESS) status = wait_progress(c, std::min(L, launched + chunk));
   }
-  if (exec) (void)hipGraphExecDestroy(exec);
   PRH_CHECK(status);
   PRH_HIP(c, hipEventRecord(c->ev[2], s));
   PRH_HIP(c, prh::launch_ppr_ranks(A, c->ppr_out.p, s));

@@ -159,3 +159,26 @@ def test_ranks_larger_than_the_staging_area(ctx, oracle_mod):
     for j in (0, 31, 63):
         ref, it = oracle_mod.ppr(y, _teleport(n, seeds[j]))
         assert abs(int(res.iterations[j]) - it) <= 1 and np.abs(res.ranks[:, j] - ref).max() <= 1e-9
+
+
+@pytest.mark.parametrize("k", [3, 40])
+def test_iteration_cap_with_heavy_rows(monkeypatch, k):
+    """Caps before, at and after the end of a replay of eight iterations, reached unconverged, on rows cut into chunks:
+    the loop ends while the last replay's heavy rows are still to be finished. Captured and launched one by one, three
+    times over: the same bits."""
+    from pagerank_amd import Context, PagerankOptions, ppr_batched
+    from test_gpu_rows import degree_graph
+    y = degree_graph(40961, 13)
+    seeds = _seed_sets(y.N, k, 200, np.random.default_rng(k))
+    out = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("PRH_GRAPH_CAPTURE", mode)
+        with Context(0) as c:
+            yg = c.upload(y, with_out=False)
+            for cap in (0, 1, 7, 8, 9, 16):
+                for i in range(3 if mode == "1" else 1):
+                    print(f"[ppr cap] k={k} capture={mode} cap={cap} pass={i}", flush=True)
+                    res = ppr_batched(yg, seeds, PagerankOptions(tolerance=0.0, maxIterations=cap))
+                    assert np.all(res.iterations == cap)
+                    assert np.array_equal(res.ranks, out.setdefault(cap, res.ranks))
+            yg.close()
