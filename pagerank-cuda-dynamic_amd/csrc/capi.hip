@@ -31,7 +31,7 @@ int fail(prh_context *c, int status, const char *fmt, ...) {
   return status;
 }
 
-int dev_alloc(prh_context *c, void **p, size_t bytes) {
+int dev_alloc_spare(prh_context *c, void **p, size_t bytes) {
   if (bytes == 0) bytes = 16;
   if (c->limit && c->used + bytes > c->limit)
     return fail(c, PRH_ERROR_OUT_OF_MEMORY, "device memory limit: %zu bytes in use, %zu more requested, limit %zu",
@@ -43,6 +43,16 @@ int dev_alloc(prh_context *c, void **p, size_t bytes) {
   }
   c->used += bytes;
   return PRH_SUCCESS;
+}
+
+int dev_alloc(prh_context *c, void **p, size_t bytes) {
+  const int status = dev_alloc_spare(c, p, bytes);
+  if (status == PRH_SUCCESS || c->spare.empty()) return status;
+  // work that reads a spare map may still be enqueued
+  if (hipStreamSynchronize(c->stream) != hipSuccess) (void)hipGetLastError();
+  while (!c->spare.empty()) free_edge_of(c, *c->spare.back());
+  c->error.clear();
+  return dev_alloc_spare(c, p, bytes);
 }
 
 void dev_free(prh_context *c, void *p, size_t bytes) {

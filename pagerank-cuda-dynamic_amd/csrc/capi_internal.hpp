@@ -59,6 +59,8 @@ struct DevBuf {
 
 }  // namespace prhc
 
+struct BinnedCache;
+
 struct prh_context {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -95,7 +97,8 @@ struct prh_context {
   prhc::DevBuf<uint32_t> wt_chunks;       // heavy-row chunk tables of the weighted pull
   prhc::DevBuf<uint32_t> wt_sort, wt_sort_tmp;  // degree sort of its low rows
   prhc::DevBuf<double> wt_partial;        // their sums
-  uint64_t *pinned = nullptr;       // small host-pinned readback area (kPinnedBytes)
+  std::vector<BinnedCache *> spare;  // plans that hold an edge_of: given up when memory runs out (dev_alloc)
+  uint64_t *pinned = nullptr;        // small host-pinned readback area (kPinnedBytes)
   // Pinned words that a running iteration loop writes (LoopCtl::host): [0] iterations begun, [1] iterations performed
   // once it has stopped.
   int *progress = nullptr;
@@ -123,7 +126,8 @@ struct BinnedCache {
   uint32_t *base_off = nullptr, *base_src = nullptr, *slot_of = nullptr;
   uint64_t base_M = 0, base_cap = 0;  // base edges, and the capacity of base_src
   uint64_t slot_of_n = 0;             // entries of slot_of (the edges of the graph the plan was built from)
-  // Weighted solves: the caller's edge of every slot (the slot map composed with the layout's edge map), and its entries.
+  // Weighted solves: the caller's edge of every slot (the slot map composed with the layout's edge map), and its entries;
+  // optional, and listed in prh_context::spare while it is held.
   uint32_t *edge_of = nullptr;
   uint64_t edge_of_n = 0;
   unsigned long long *ov_key = nullptr;
@@ -216,7 +220,10 @@ int fail(prh_context *c, int status, const char *fmt, ...) __attribute__((format
     if (s_ != PRH_SUCCESS) return s_; \
   } while (0)
 
+// Device memory within the context's limit. Where there is none left, what the context holds only to save time (its spare
+// maps) is given up before the call fails; dev_alloc_spare, for such maps themselves, gives up nothing.
 int dev_alloc(prh_context *c, void **p, size_t bytes);
+int dev_alloc_spare(prh_context *c, void **p, size_t bytes);
 void dev_free(prh_context *c, void *p, size_t bytes);
 
 template <class T>

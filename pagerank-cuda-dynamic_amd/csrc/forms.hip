@@ -358,11 +358,12 @@ int from_layout(prh_context *c, const double *src, const uint32_t *map, size_t n
 }
 
 // The weights in the slot order of a blocked plan (wt_wl), through the map from slots to the caller's edges: kept with
-// the plan, or composed for each weight where there is no room for it.
+// the plan as long as there is room for it, else composed for each weight.
 int slot_weights(prh_context *c, BinnedCache &bc, const float *w, const uint32_t *eid, uint64_t M) {
   if (!bc.edge_of && M) {
-    if (dev_alloc(c, reinterpret_cast<void **>(&bc.edge_of), M * 4) == PRH_SUCCESS) {
+    if (dev_alloc_spare(c, reinterpret_cast<void **>(&bc.edge_of), M * 4) == PRH_SUCCESS) {
       bc.edge_of_n = M;
+      c->spare.push_back(&bc);
       PRH_HIP(c, prh::launch_permute_u32(eid, bc.plan.slot, M, bc.edge_of, c->stream));
     } else {
       bc.edge_of = nullptr;

@@ -233,6 +233,8 @@ void free_binned(prh_context *c, BinnedCache &bc) {
 }
 
 void free_edge_of(prh_context *c, BinnedCache &bc) {
+  if (!bc.edge_of) return;
+  c->spare.erase(std::remove(c->spare.begin(), c->spare.end(), &bc), c->spare.end());
   dev_free(c, bc.edge_of, bc.edge_of_n * 4);
   bc.edge_of = nullptr;
   bc.edge_of_n = 0;

@@ -178,3 +178,31 @@ def test_row_classes_and_gradient_tiles(ctx, oracle_mod, flip, blocking):
     size = (0.85 * r / W)[u] * (np.abs(lam[v]) + (np.abs(lam - g) / 0.85)[u])
     assert np.all(np.abs(gw - gw_o) <= 1e-11 * size)
     assert np.all(np.abs(gs - gs_o) <= 1e-15 * np.abs(lam))
+
+
+def test_slot_maps_make_room():
+    """The slot-to-edge maps of the blocked weighted solves (4 bytes an edge, one for each direction) only save time: with
+    no memory left below the limit, another graph takes their place, and the solves go on without them."""
+    from pagerank_amd import Context, HostGraph, Tuning, weighted_adjoint, weighted_pagerank
+    y, w, c, s = _case(14)
+    with Context(0) as ctx:
+        ctx.set_tuning(Tuning(blocking=1024))
+        yg = ctx.upload(y)
+
+        def step():
+            fw = weighted_pagerank(yg, w, s)
+            return (fw.ranks,) + weighted_adjoint(yg, w, fw.ranks, 2 * c * fw.ranks)[:3]
+
+        first = step()
+        used = ctx.memory_used()
+        print(f"[maps] N={y.N} M={y.M} used={used}", flush=True)
+        ctx.set_memory_limit(used)
+        z = HostGraph.rmat(11, 8, seed=1)
+        zg = ctx.upload(z)  # less than the 8 bytes an edge of the two maps
+        assert ctx.memory_used() < used - 4 * y.M
+        for _ in range(2):  # composed per call, then kept again where there is room
+            for a, b in zip(step(), first):
+                assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max()
+            assert ctx.memory_used() <= used
+        zg.close()
+        yg.close()
