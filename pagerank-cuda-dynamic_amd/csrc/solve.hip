@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "capi_internal.hpp"
@@ -97,20 +98,28 @@ void reset_progress(prh_context *c) {
   __atomic_store_n(c->progress + 1, 0, __ATOMIC_RELEASE);
 }
 
+// Polls for a few microseconds (iterations of small graphs last no longer), then offers its core to other threads between
+// polls, and from a millisecond on sleeps between them: iterations that long leave the host time, as some are enqueued
+// ahead. Polling throughout -> this, blocked solves of 1M vertices: four threads on one core 246 -> 292 a second, on two
+// cores 323 -> 334; one thread 246 and 246 (64K vertices 1438 and 1432). Batched PPR, runs of 29 ms: the calling thread is
+// busy for 13 of 116 ms.
 int wait_progress(prh_context *c, int begun) {
   using clock = std::chrono::steady_clock;
-  const auto wait = std::chrono::milliseconds(100);
-  clock::time_point next;
-  for (unsigned i = 1; !loop_stopped(c) && __atomic_load_n(c->progress, __ATOMIC_ACQUIRE) < begun; ++i) {
-    if (i % 1024) {
-      __builtin_ia32_pause();
-      continue;
-    }
+  using std::chrono::microseconds;
+  const auto waiting = [&]() {
+    return !loop_stopped(c) && __atomic_load_n(c->progress, __ATOMIC_ACQUIRE) < begun;
+  };
+  for (int i = 0; i < 256; ++i)
+    if (!waiting()) return PRH_SUCCESS;
+  const clock::time_point begin = clock::now();
+  clock::time_point query = begin + microseconds(100000);
+  while (waiting()) {
+    const clock::time_point now = clock::now();
+    if (now - begin > microseconds(1000)) std::this_thread::sleep_for(microseconds(50));
+    else if (now - begin > microseconds(20)) std::this_thread::yield();
     // Long iterations, or launches that failed: ask the stream now and then (a query adds a marker to it).
-    const auto now = clock::now();
-    if (i == 1024) next = now + wait;
-    if (now < next) continue;
-    next = now + wait;
+    if (now < query) continue;
+    query = now + microseconds(100000);
     const hipError_t e = hipStreamQuery(c->stream);
     if (e == hipSuccess) break;
     if (e != hipErrorNotReady) return fail(c, PRH_ERROR_DEVICE, "iterations: %s", hipGetErrorString(e));

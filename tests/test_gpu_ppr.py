@@ -182,3 +182,27 @@ def test_iteration_cap_with_heavy_rows(monkeypatch, k):
                     assert np.all(res.iterations == cap)
                     assert np.array_equal(res.ranks, out.setdefault(cap, res.ranks))
             yg.close()
+
+
+def test_waiting_leaves_the_core(ctx):
+    """The host waits 16 ms and more for each run of iterations (512 of at least 32 us): it polls for the first millisecond
+    and sleeps after it, so the calling thread takes less than half of the call's time (the rest of it, the capture and
+    the way back of 34 MB, is some ten milliseconds)."""
+    import time
+
+    from pagerank_amd import HostGraph, PagerankOptions, Tuning, ppr_batched
+    y = HostGraph.rmat(16, 16, seed=4)
+    seeds = _seed_sets(y.N, 64, 20, np.random.default_rng(5))
+    yg = ctx.upload(y, with_out=False)
+    old = ctx.get_tuning()
+    try:
+        ctx.set_tuning(Tuning(**{**old.__dict__, "check_interval": 512}))
+        o = PagerankOptions(tolerance=0.0, maxIterations=2048)
+        ppr_batched(yg, seeds, o)
+        wall, cpu = time.perf_counter(), time.thread_time()
+        ppr_batched(yg, seeds, o)
+        wall, cpu = time.perf_counter() - wall, time.thread_time() - cpu
+    finally:
+        ctx.set_tuning(old)
+    print(f"[wait] {wall * 1e3:.1f} ms, {cpu * 1e3:.1f} ms of the calling thread's", flush=True)
+    assert cpu < 0.5 * wall
