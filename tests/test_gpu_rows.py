@@ -129,3 +129,89 @@ def test_extension_inside_the_update(ctx, method, edges):
     for d in (1, 2):
         assert out[d].iterations == out[0].iterations
         assert np.array_equal(out[d].ranks, out[0].ranks), d
+
+
+@pytest.mark.parametrize("method", [3, 4], ids=["DF", "DFP"])
+@pytest.mark.parametrize("edges", [40, 20000])
+def test_extension_directions_above_the_inside_limit(ctx, method, edges):
+    """Above 2^24 edges the extension is a launch of its own, pushed, pulled, or the cheaper by the sums that the rank
+    launches leave (direction 1); rows cut into chunks, which the second launch finishes, add to those sums too. All three
+    set the same flags: the ranks are the same bit for bit."""
+    from pagerank_amd import Batch, HostGraph, apply_batch, solve
+    x = HostGraph.rmat(20, 18, seed=6)
+    b = Batch.random(x, edges, 0.8, seed=2)
+    y = apply_batch(x, b)
+    assert y.M > 1 << 24 and np.diff(y.in_off.astype(np.int64)).max() > 16384
+    q = solve(ctx.upload(x), 0).ranks
+    yg = ctx.upload(y)
+    old = ctx.get_tuning()
+    out = {}
+    try:
+        for d in (0, 1, 2):
+            print(f"[outside] M={y.M} method={method} edges={edges} direction={d}", flush=True)
+            t = ctx.get_tuning()
+            t.extension_direction = d
+            ctx.set_tuning(t)
+            out[d] = solve(yg, method, batch=b, q=q)
+    finally:
+        ctx.set_tuning(old)
+    for d in (1, 2):
+        assert out[d].iterations == out[0].iterations
+        assert np.array_equal(out[d].ranks, out[0].ranks), d
+
+
+@pytest.mark.parametrize("direction", [0, 2])
+def test_hub_chunks_of_the_push_across_tunings(ctx, oracle_mod, direction):
+    """A source of 6000 out-edges among the batch's: the push takes it in chunks of the cached out-degree schedule, before
+    and after a tuning change that rebuilds the rank plan (the pull for comparison)."""
+    from pagerank_amd import Batch, HostGraph, apply_batch, solve
+    n = 9000
+    rng = np.random.default_rng(4)
+    src = np.concatenate([np.zeros(6000, np.uint32), rng.integers(0, n, 30000).astype(np.uint32)])
+    dst = np.concatenate([np.arange(1, 6001, dtype=np.uint32), rng.integers(0, n, 30000).astype(np.uint32)])
+    x = HostGraph.from_edges(n, src, dst, self_loops=True)
+    b = Batch.tidy(x, [[0, 1]], [[0, 7000], [5, 8000]])
+    y = apply_batch(x, b)
+    print(f"[hub push] N={y.N} M={y.M} direction={direction}", flush=True)
+    yg = ctx.upload(y)
+    q, _, _ = oracle_mod.pagerank_cuda(oracle_mod.STATIC, x)
+    ref, it, _ = oracle_mod.pagerank_cuda(3, y, b, q)
+    old = ctx.get_tuning()
+    try:
+        for switch in (64, 128):
+            t = ctx.get_tuning()
+            t.extension_direction, t.switch_degree = direction, switch
+            ctx.set_tuning(t)
+            res = solve(yg, 3, batch=b, q=q)
+            assert abs(res.iterations - it) <= 1
+            assert np.abs(res.ranks - ref).max() <= 1e-9
+    finally:
+        ctx.set_tuning(old)
+
+
+@pytest.mark.parametrize("method", [0, 3], ids=["static", "DF"])
+def test_rows_without_in_edges_beyond_one_workgroup(ctx, oracle_mod, method):
+    """More vertices than one workgroup's LDS holds, most of them without in-edges, one row in chunks of 64 edges. (Not
+    DF-P: its closed form takes every vertex to have a self-loop, and without one the oracle too diverges to NaN.)"""
+    from pagerank_amd import Batch, HostGraph, Tuning, apply_batch, solve
+    n = 9000
+    u = np.arange(n, dtype=np.uint32)
+    src = np.concatenate([u[1:], [0], u[:100]])
+    dst = np.concatenate([np.zeros(n - 1, np.uint32), [1], (u[:100] * 7 + 3) % 50])
+    x = HostGraph.from_edges(n, src, dst, self_loops=False)
+    b = Batch.tidy(x, np.zeros((0, 2)), [[3, 60], [200, 61]])
+    y = apply_batch(x, b)
+    q, _, _ = oracle_mod.pagerank_cuda(oracle_mod.STATIC, x)
+    args = (b, q) if method else (None, None)
+    old = ctx.get_tuning()
+    print(f"[no-in-edges] N={y.N} M={y.M} method={method}", flush=True)
+    try:
+        ctx.set_tuning(Tuning(64, 64, old.low_width, old.check_interval, 0))
+        res = solve(ctx.upload(y), method, batch=args[0], q=args[1])
+    finally:
+        ctx.set_tuning(old)
+    ref, it, _ = oracle_mod.pagerank_cuda(method, y, *args)
+    assert abs(res.iterations - it) <= 1
+    assert np.abs(res.ranks - ref).max() <= 1e-9
+    if not method:
+        assert np.all(res.ranks[np.diff(y.in_off.astype(np.int64)) == 0] == (1 - 0.85) / n)
