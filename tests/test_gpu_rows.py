@@ -215,3 +215,30 @@ def test_rows_without_in_edges_beyond_one_workgroup(ctx, oracle_mod, method):
     assert np.abs(res.ranks - ref).max() <= 1e-9
     if not method:
         assert np.all(res.ranks[np.diff(y.in_off.astype(np.int64)) == 0] == (1 - 0.85) / n)
+
+
+@pytest.mark.parametrize("method", [3, 4], ids=["DF", "DFP"])
+def test_push_of_every_out_degree(ctx, method):
+    """Sources of every class and remainder of the push (lane groups, waves, chunks; eight loads in flight a lane) in the
+    frontier: pushed and pulled, the same flags, hence the same bits."""
+    from pagerank_amd import Batch, HostGraph, apply_batch, solve
+    t = degree_graph(40003, 17)
+    dst = np.repeat(np.arange(t.N, dtype=np.uint32), np.diff(t.out_off.astype(np.int64)))
+    x = HostGraph.from_edges(t.N, t.out_edg.astype(np.uint32), dst)  # transposed: DEGREES are out-degrees
+    q = solve(ctx.upload(x), 0).ranks
+    k = np.arange(len(DEGREES))
+    b = Batch.tidy(x, np.zeros((0, 2)), np.stack([k, 30000 + k], axis=1))
+    yg = ctx.upload(apply_batch(x, b))
+    old = ctx.get_tuning()
+    out = {}
+    try:
+        for d in (0, 2):
+            print(f"[push] method={method} direction={d}", flush=True)
+            tuning = ctx.get_tuning()
+            tuning.extension_direction = d
+            ctx.set_tuning(tuning)
+            out[d] = solve(yg, method, batch=b, q=q)
+    finally:
+        ctx.set_tuning(old)
+    assert out[0].iterations == out[2].iterations > 1
+    assert np.array_equal(out[0].ranks, out[2].ranks)
