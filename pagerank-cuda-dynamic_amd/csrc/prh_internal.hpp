@@ -107,6 +107,9 @@ struct RankArgs {
   // The launch then does that iteration's extension itself (a row not affected becomes so if an in-neighbour has the
   // flag); naff is another buffer.
   const uint8_t *prev = nullptr;
+  // Frontier variants on the row plan: the in-CSR is read with the non-temporal hint, so that it does not displace what the
+  // pushed extension reads after this launch (see stream_in_csr).
+  bool stream = false;
 };
 
 struct ExtendArgs {

@@ -38,11 +38,18 @@ struct RowOperands {
   bool upd;       // the row is updated (always, except unaffected rows of the dynamic variants)
 };
 
-template <int VARIANT>
+// A load of the in-CSR. STREAM: non-temporal, past the caches (RankArgs::stream).
+template <bool STREAM>
+__device__ __forceinline__ uint32_t csr_load(const uint32_t *p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
+template <int VARIANT, bool STREAM>
 __device__ __forceinline__ RowOperands row_operands(const RankArgs &A, uint32_t v) {
   RowOperands o;
-  o.b = A.off[v];
-  o.e = A.off[v + 1];
+  o.b = csr_load<STREAM>(A.off + v);
+  o.e = csr_load<STREAM>(A.off + v + 1);
   o.d = A.deg[v];
   o.rv = A.r[v];
   o.crv = Traits<VARIANT>::dynamic ? A.cr[v] : 0.0;
@@ -57,15 +64,15 @@ __device__ __forceinline__ RowOperands row_operands(const RankArgs &A, uint32_t 
 // without it sits these two loads out: repeating a load instead costs the address unit as much as a new one). Source ids
 // and offsets are plain loads: neighbouring rows share their lines, which the non-temporal hint made each fetch again
 // (300K vertices 2306 -> 1907 us per solve without it, 1M 6.64 -> 5.30 ms, 7M 44.4 -> 44.3 ms).
-template <int STEP, int U>
+template <int STEP, int U, bool STREAM>
 __device__ __forceinline__ void gather_batch(const uint32_t *src, const double *cr, uint32_t e, uint32_t left,
                                              double (&s)[4]) {
   const bool last = (U - 1) * STEP < left;
   uint32_t u[U];
   double x[U];
 #pragma unroll
-  for (int k = 0; k + 1 < U; ++k) u[k] = src[e + k * STEP];
-  u[U - 1] = last ? src[e + (U - 1) * STEP] : 0u;
+  for (int k = 0; k + 1 < U; ++k) u[k] = csr_load<STREAM>(src + e + k * STEP);
+  u[U - 1] = last ? csr_load<STREAM>(src + e + (U - 1) * STEP) : 0u;
 #pragma unroll
   for (int k = 0; k + 1 < U; ++k) x[k] = cr[u[k]];
   x[U - 1] = last ? cr[u[U - 1]] : 0.0;
@@ -73,10 +80,10 @@ __device__ __forceinline__ void gather_batch(const uint32_t *src, const double *
   for (int k = 0; k < U; ++k) s[k & 3] += x[k];
 }
 
-// Sum of cr[src[e]] for e = b + i, b + i + STEP, ... < end, where i < STEP is the thread's place among the STEP threads
+// Sum of cr[csr_load<STREAM>(src + e)] for e = b + i, b + i + STEP, ... < end, where i < STEP is the thread's place among the STEP threads
 // of the row (a wave or a workgroup) and b, end are the same for all of them: batches of eight gathers a thread, the
 // last batch of exactly as many as are left.
-template <int STEP>
+template <int STEP, bool STREAM = false>
 __device__ __forceinline__ double gather_sum(const uint32_t *src, const double *cr, uint32_t b, uint32_t end,
                                              uint32_t i) {
   double s[4] = {0.0, 0.0, 0.0, 0.0};
@@ -84,19 +91,19 @@ __device__ __forceinline__ double gather_sum(const uint32_t *src, const double *
   src += b;
   end -= b;
   uint32_t e = i;
-  for (; n > 8; n -= 8, e += 8 * STEP) gather_batch<STEP, 8>(src, cr, e, end - e, s);
+  for (; n > 8; n -= 8, e += 8 * STEP) gather_batch<STEP, 8, STREAM>(src, cr, e, end - e, s);
   // A thread of the last batch may have no edge in a one-edge batch; in longer ones its first edge always exists.
   switch (n) {
     case 1:
-      if (e < end) s[0] += cr[src[e]];
+      if (e < end) s[0] += cr[csr_load<STREAM>(src + e)];
       break;
-    case 2: gather_batch<STEP, 2>(src, cr, e, end - e, s); break;
-    case 3: gather_batch<STEP, 3>(src, cr, e, end - e, s); break;
-    case 4: gather_batch<STEP, 4>(src, cr, e, end - e, s); break;
-    case 5: gather_batch<STEP, 5>(src, cr, e, end - e, s); break;
-    case 6: gather_batch<STEP, 6>(src, cr, e, end - e, s); break;
-    case 7: gather_batch<STEP, 7>(src, cr, e, end - e, s); break;
-    case 8: gather_batch<STEP, 8>(src, cr, e, end - e, s); break;
+    case 2: gather_batch<STEP, 2, STREAM>(src, cr, e, end - e, s); break;
+    case 3: gather_batch<STEP, 3, STREAM>(src, cr, e, end - e, s); break;
+    case 4: gather_batch<STEP, 4, STREAM>(src, cr, e, end - e, s); break;
+    case 5: gather_batch<STEP, 5, STREAM>(src, cr, e, end - e, s); break;
+    case 6: gather_batch<STEP, 6, STREAM>(src, cr, e, end - e, s); break;
+    case 7: gather_batch<STEP, 7, STREAM>(src, cr, e, end - e, s); break;
+    case 8: gather_batch<STEP, 8, STREAM>(src, cr, e, end - e, s); break;
     default: break;
   }
   return (s[0] + s[1]) + (s[2] + s[3]);
@@ -105,18 +112,18 @@ __device__ __forceinline__ double gather_sum(const uint32_t *src, const double *
 // The same for a group of W lanes, whose rows differ within the wave: lane j takes edges b + j, b + j + W, ... A band's
 // rows have W < in-degree <= 2 W, so the first two edges go together (two round trips; one by one they took four), and
 // what rows of other degrees have left goes by fours.
-template <int W>
+template <int W, bool STREAM = false>
 __device__ __forceinline__ double group_gather_sum(const uint32_t *src, const double *cr, uint32_t b, uint32_t end,
                                                    uint32_t j) {
   src += b;
   end -= b;
   if (j >= end) return 0.0;
   double s[4] = {0.0, 0.0, 0.0, 0.0};
-  gather_batch<W, 2>(src, cr, j, end - j, s);
+  gather_batch<W, 2, STREAM>(src, cr, j, end - j, s);
   for (uint32_t e = j + 2 * W; e < end; e += 4 * W) {
     uint32_t u[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) u[k] = e + k * W < end ? src[e + k * W] : 0u;
+    for (int k = 0; k < 4; ++k) u[k] = e + k * W < end ? csr_load<STREAM>(src + e + k * W) : 0u;
 #pragma unroll
     for (int k = 0; k < 4; ++k) s[k] += e + k * W < end ? cr[u[k]] : 0.0;
   }
@@ -124,10 +131,11 @@ __device__ __forceinline__ double group_gather_sum(const uint32_t *src, const do
 }
 
 // Sum of a workgroup-strided gather, valid in thread 0. Every thread must call it.
+template <bool STREAM = false>
 __device__ __forceinline__ double block_gather_sum(const uint32_t *src, const double *cr, uint32_t b, uint32_t e,
                                                    double *lds) {
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  const double acc = group_sum<kWave>(gather_sum<kBlock>(src, cr, b, e, threadIdx.x));
+  const double acc = group_sum<kWave>(gather_sum<kBlock, STREAM>(src, cr, b, e, threadIdx.x));
   if (lane == 0) lds[w] = acc;
   __syncthreads();
   const double t = (lds[0] + lds[1]) + (lds[2] + lds[3]);
@@ -161,7 +169,7 @@ __device__ __forceinline__ void keep_fresh(const RankArgs &A, uint32_t v, bool f
 
 // One workgroup per chunk item: its partial sum goes to the item's slot; rows are finished by
 // finish_chunked_kernel after this launch (the kernel boundary makes every chunk's partial visible).
-template <int VARIANT>
+template <int VARIANT, bool STREAM>
 __device__ __forceinline__ void chunked_rows(const RankArgs &A, const RankPlan &P, const RankSection &S, uint32_t blk,
                                              double *lds) {
   const uint32_t ib = S.begin + blk * S.per_block, ie = min(S.end, ib + S.per_block);
@@ -171,7 +179,7 @@ __device__ __forceinline__ void chunked_rows(const RankArgs &A, const RankPlan &
     const bool upd = affected<VARIANT>(A, v);
     if (!upd && !test) continue;
     const uint32_t b = P.item_beg[it], e = P.item_end[it];
-    const double t = block_gather_sum(A.src, A.cr, b, e, lds);
+    const double t = block_gather_sum<STREAM>(A.src, A.cr, b, e, lds);
     const bool hit = test && !upd && __syncthreads_or(any_frontier<kBlock>(A.prev, A.src, b, e, threadIdx.x)) != 0;
     if (threadIdx.x == 0) {
       P.partial[it] = t;
@@ -181,19 +189,19 @@ __device__ __forceinline__ void chunked_rows(const RankArgs &A, const RankPlan &
 }
 
 // One workgroup per row of `per_block` rows: the rows too long for one wave's chain of batches (kBlockRowDegree).
-template <int VARIANT>
+template <int VARIANT, bool STREAM>
 __device__ __forceinline__ void block_rows(const RankArgs &A, const RankSection &S, uint32_t blk, double *lds,
                                            double &emax, CostAcc &cost) {
   const uint32_t rb = S.begin + blk * S.per_block, re = min(S.end, rb + S.per_block);
   for (uint32_t v = rb; v < re; ++v) {  // block-uniform
-    RowOperands o = row_operands<VARIANT>(A, v);
+    RowOperands o = row_operands<VARIANT, STREAM>(A, v);
     RowFlags f;
     bool fresh = false;
     if constexpr (Traits<VARIANT>::frontier) {
       if (A.prev && !o.upd)
         o.upd = fresh = __syncthreads_or(any_frontier<kBlock>(A.prev, A.src, o.b, o.e, threadIdx.x)) != 0;
     }
-    const double t = o.upd ? block_gather_sum(A.src, A.cr, o.b, o.e, lds) : 0.0;
+    const double t = o.upd ? block_gather_sum<STREAM>(A.src, A.cr, o.b, o.e, lds) : 0.0;
     if (threadIdx.x == 0) {
       if (o.upd) {
         emax = fmax(emax, finish_vertex<VARIANT>(A, v, t, o.d, o.rv, o.crv, f));
@@ -207,13 +215,13 @@ __device__ __forceinline__ void block_rows(const RankArgs &A, const RankSection 
   }
 }
 
-template <int VARIANT>
+template <int VARIANT, bool STREAM>
 __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &S, uint32_t blk, double &emax,
                                           CostAcc &cost) {
   const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   const uint32_t rb = S.begin + blk * S.per_block, re = min(S.end, rb + S.per_block);
   for (uint32_t v = rb + w; v < re; v += kWavesPerBlock) {  // wave-uniform
-    RowOperands o = row_operands<VARIANT>(A, v);
+    RowOperands o = row_operands<VARIANT, STREAM>(A, v);
     RowFlags f;
     bool fresh = false;
     if constexpr (Traits<VARIANT>::frontier) {
@@ -228,7 +236,7 @@ __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &
       }
       continue;
     }
-    const double acc = group_sum<kWave>(gather_sum<kWave>(A.src, A.cr, o.b, o.e, lane));
+    const double acc = group_sum<kWave>(gather_sum<kWave, STREAM>(A.src, A.cr, o.b, o.e, lane));
     if (lane == 0) {
       emax = fmax(emax, finish_vertex<VARIANT>(A, v, acc, o.d, o.rv, o.crv, f));
       keep_fresh<VARIANT>(A, v, fresh, f);
@@ -237,7 +245,7 @@ __device__ __forceinline__ void wave_rows(const RankArgs &A, const RankSection &
   }
 }
 
-template <int VARIANT, int W>
+template <int VARIANT, int W, bool STREAM>
 __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection &S, uint32_t blk, double &emax,
                                            CostAcc &cost) {
   constexpr int G = kWave / W;  // rows per wave per round
@@ -250,7 +258,7 @@ __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection 
     RowOperands o{};
     double acc = 0.0;
     bool fresh = false;
-    if (valid) o = row_operands<VARIANT>(A, v);
+    if (valid) o = row_operands<VARIANT, STREAM>(A, v);
     if constexpr (Traits<VARIANT>::frontier) {
       if (A.prev) {
         const unsigned long long hits =
@@ -259,7 +267,7 @@ __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection 
         o.upd = o.upd || fresh;
       }
     }
-    if (valid && o.upd) acc = group_gather_sum<W>(A.src, A.cr, o.b, o.e, j);
+    if (valid && o.upd) acc = group_gather_sum<W, STREAM>(A.src, A.cr, o.b, o.e, j);
     acc = group_sum<W>(acc);  // all lanes active again here
     if (valid && j == 0) {
       RowFlags f;
@@ -275,7 +283,7 @@ __device__ __forceinline__ void group_rows(const RankArgs &A, const RankSection 
   }
 }
 
-template <int VARIANT>
+template <int VARIANT, bool STREAM>
 __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPlan P, LoopCtl ctl) {
   if (!iteration_begin(ctl)) return;
   __shared__ double lds_sum[kWavesPerBlock];
@@ -286,19 +294,19 @@ __global__ __launch_bounds__(kBlock) void rank_update_kernel(RankArgs A, RankPla
   double emax = 0.0;
   CostAcc cost;
   if (S.kind == kChunkedRows) {
-    chunked_rows<VARIANT>(A, P, S, blk, lds_sum);
+    chunked_rows<VARIANT, STREAM>(A, P, S, blk, lds_sum);
   } else if (S.kind == kBlockRows) {
-    block_rows<VARIANT>(A, S, blk, lds_sum, emax, cost);
+    block_rows<VARIANT, STREAM>(A, S, blk, lds_sum, emax, cost);
   } else if (S.kind == kWaveRows) {
-    wave_rows<VARIANT>(A, S, blk, emax, cost);
+    wave_rows<VARIANT, STREAM>(A, S, blk, emax, cost);
   } else {
     switch (S.width) {
-      case 1: group_rows<VARIANT, 1>(A, S, blk, emax, cost); break;
-      case 2: group_rows<VARIANT, 2>(A, S, blk, emax, cost); break;
-      case 4: group_rows<VARIANT, 4>(A, S, blk, emax, cost); break;
-      case 8: group_rows<VARIANT, 8>(A, S, blk, emax, cost); break;
-      case 16: group_rows<VARIANT, 16>(A, S, blk, emax, cost); break;
-      default: group_rows<VARIANT, 32>(A, S, blk, emax, cost); break;
+      case 1: group_rows<VARIANT, 1, STREAM>(A, S, blk, emax, cost); break;
+      case 2: group_rows<VARIANT, 2, STREAM>(A, S, blk, emax, cost); break;
+      case 4: group_rows<VARIANT, 4, STREAM>(A, S, blk, emax, cost); break;
+      case 8: group_rows<VARIANT, 8, STREAM>(A, S, blk, emax, cost); break;
+      case 16: group_rows<VARIANT, 16, STREAM>(A, S, blk, emax, cost); break;
+      default: group_rows<VARIANT, 32, STREAM>(A, S, blk, emax, cost); break;
     }
   }
   __shared__ double lds_cost[2 * kWavesPerBlock];
@@ -350,7 +358,12 @@ __global__ __launch_bounds__(kBlock) void finish_chunked_kernel(RankArgs A, Rank
 
 template <int VARIANT>
 hipError_t launch_variant(const RankArgs &A, const RankPlan &P, const LoopCtl &ctl, hipStream_t s, hipEvent_t mark) {
-  rank_update_kernel<VARIANT><<<P.blocks, kBlock, 0, s>>>(A, P, ctl);
+  if constexpr (Traits<VARIANT>::frontier) {
+    if (A.stream) rank_update_kernel<VARIANT, true><<<P.blocks, kBlock, 0, s>>>(A, P, ctl);
+    else rank_update_kernel<VARIANT, false><<<P.blocks, kBlock, 0, s>>>(A, P, ctl);
+  } else {
+    rank_update_kernel<VARIANT, false><<<P.blocks, kBlock, 0, s>>>(A, P, ctl);
+  }
   if (mark) {
     const hipError_t e = hipEventRecord(mark, s);
     if (e != hipSuccess) return e;

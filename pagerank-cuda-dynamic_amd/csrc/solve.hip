@@ -170,6 +170,16 @@ static int load_initial_ranks(prh_context *c, const prh_graph *g, const double *
 // 562 -> 324 us, 11.2M 1154 -> 937. Both sides meet at about 20M edges (40M, DF-P: 8.3 -> 8.7 ms).
 constexpr uint64_t kExtendInside = uint64_t(1) << 24;
 
+// Whether a frontier solve that pushes its extension (direction 0) reads the in-CSR past the Infinity Cache (256 MB): where
+// an iteration's other arrays (the out-CSR and its schedule, ranks and contributions, degrees, flags) fit there without the
+// in-CSR but not with it. Per DF solve through the cache -> past it, 1e-2 of the edges changed: 4M vertices, 16M edges
+// 25.1 -> 22.2 ms, RMAT-21 23.8 -> 22.4; where all of it fits (RMAT-20) 10.5 -> 11.8, where not even the rest does
+// (RMAT-22) 48.6 -> 49.5. The pull and the solves without a frontier gain nothing from it (RMAT-21: 14.6 -> 16.7, pulled).
+static bool stream_in_csr(const prh_graph *g) {
+  const uint64_t cache = uint64_t(256) << 20, N = g->N, csr = 4 * (g->M + N), rest = csr + 42 * N;
+  return rest <= cache && csr + rest > cache;
+}
+
 // The bands and items of a small graph's solve; false if the graph does not fit. (That the ids' 16-bit byte offsets hold
 // every vertex follows from the size of LDS. The out-degrees are kept in 16 bits too; M bounds them only where the graph
 // came with its out-CSR, whose rows they are checked against.)
@@ -266,6 +276,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
   // 2 pull only. The pull form splits rows at in-degree 64 (a wave each) and 4 (8 lanes each).
   const int dir_mode = frontier ? c->tuning.extension_direction : 0;
   const bool inside = dir_mode == 1 && !binned && !window && g->M <= kExtendInside;
+  const bool stream = frontier && dir_mode == 0 && stream_in_csr(g);
   const bool dir_auto = dir_mode == 1 && !binned && !small && !inside;
   if (dir_auto) PRH_CHECK(ensure(c, c->ext_stats, 2 * prh::kCostSums));  // the sums of two iterations in turn
   const prh::PullArgs pull{c->vaff.p, c->naff.p, g->l_in_off, g->l_in_src, layout_rows_above(g, 64),
@@ -326,6 +337,7 @@ int solve_impl(prh_context *c, const prh_graph *g, int method, const prh_options
       prh::RankArgs A{c->rank[(l + 1) & 1].p, c->rank[l & 1].p, c->contrib[(l + 1) & 1].p, c->contrib[l & 1].p,
                       c->naff.p, c->vaff.p, g->l_in_off, g->l_in_src, g->l_outdeg, C0, P, o->frontier_tolerance,
                       o->prune_tolerance, costs(l)};
+      A.stream = stream;
       if (inside) {  // the flags of two iterations in turn (the second buffer is the traversal levels')
         uint8_t *const flags[2] = {c->naff.p, c->buff.p};
         A.naff = flags[l & 1];

@@ -242,3 +242,29 @@ def test_push_of_every_out_degree(ctx, method):
         ctx.set_tuning(old)
     assert out[0].iterations == out[2].iterations > 1
     assert np.array_equal(out[0].ranks, out[2].ranks)
+
+
+@pytest.mark.parametrize("method", [3, 4], ids=["DF", "DFP"])
+def test_pushed_solves_beyond_the_infinity_cache(ctx, method):
+    """A graph whose in-CSR the pushed solves read with non-temporal loads (5M vertices, rows of every class): the same bits
+    as pulled, where the loads are plain ones."""
+    from pagerank_amd import Batch, apply_batch, solve
+    x = degree_graph(5_000_003, 21)
+    rest = 4 * (x.M + x.N) + 42 * x.N
+    assert rest <= 1 << 28 < 4 * (x.M + x.N) + rest  # the rule of the dispatch
+    q = solve(ctx.upload(x), 0).ranks
+    b = Batch.random(x, 3000, 0.8, seed=5)
+    yg = ctx.upload(apply_batch(x, b))
+    old = ctx.get_tuning()
+    out = {}
+    try:
+        for d in (0, 2):
+            print(f"[stream csr] method={method} direction={d}", flush=True)
+            tuning = ctx.get_tuning()
+            tuning.extension_direction = d
+            ctx.set_tuning(tuning)
+            out[d] = solve(yg, method, batch=b, q=q)
+    finally:
+        ctx.set_tuning(old)
+    assert out[0].iterations == out[2].iterations > 1
+    assert np.array_equal(out[0].ranks, out[2].ranks)
