@@ -379,7 +379,7 @@ struct PprArgs {
   const uint32_t *off, *src, *deg;  // layout in-CSR and out-degrees
   const uint32_t *perm;             // layout row -> vertex
   const int32_t *seed_row;          // [N]: row of v in seed_mass, or -1
-  const double *seed_mass;          // [rows][cols]: s_j[v]
+  const double *seed_mass;          // [rows][cols]: s_j[v] (counts until the start contributions are made)
   const uint32_t *order;            // rows by in-degree: [up to kPprGroup | up to the chunk size | heavier]
   uint32_t n_low, n_high, n_heavy;
   const uint32_t *chunk_beg, *chunk_end;  // edge ranges of the heavy rows' chunks, row by row

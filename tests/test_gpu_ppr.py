@@ -206,3 +206,26 @@ def test_waiting_leaves_the_core(ctx):
         ctx.set_tuning(old)
     print(f"[wait] {wall * 1e3:.1f} ms, {cpu * 1e3:.1f} ms of the calling thread's", flush=True)
     assert cpu < 0.5 * wall
+
+
+def test_repeated_seeds(ctx, oracle_mod):
+    """Seed sets that repeat few vertices many times, in runs, shuffled and among seeds of their own: the shares are the
+    counts over the size, whatever the order, and the results repeat bit for bit."""
+    from pagerank_amd import HostGraph, ppr_batched
+    y = HostGraph.rmat(11, 16, seed=6)
+    rng = np.random.default_rng(8)
+    runs = np.repeat(np.arange(10, dtype=np.uint32), 3001)
+    seeds = [runs, rng.permutation(runs), np.full(50021, 7, np.uint32),
+             rng.permutation(np.concatenate([np.arange(y.N, dtype=np.uint32), np.full(777, 3, np.uint32)])),
+             np.array([5], np.uint32), np.arange(63, dtype=np.uint32), np.repeat(np.arange(65, dtype=np.uint32), 2)]
+    print(f"[ppr repeats] N={y.N} M={y.M}", flush=True)
+    yg = ctx.upload(y, with_out=False)
+    res = ppr_batched(yg, seeds)
+    assert np.array_equal(res.ranks[:, 0], res.ranks[:, 1])
+    again = ppr_batched(yg, seeds)
+    assert np.array_equal(again.ranks, res.ranks)
+    for j, sd in enumerate(seeds):
+        s = np.bincount(sd, minlength=y.N) / len(sd)
+        ref, it = oracle_mod.ppr(y, s)
+        assert abs(int(res.iterations[j]) - it) <= 1
+        assert np.abs(res.ranks[:, j] - ref).max() <= 1e-9
