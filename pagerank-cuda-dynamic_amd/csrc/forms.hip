@@ -237,14 +237,14 @@ int weighted_common(prh_context *c, const prh_graph *g, const float *w, const pr
   PRH_CHECK(stage(c, w, size_t(M), device, c->wt_wout, w_out));
   PRH_CHECK(ensure(c, c->wt_W, N));
   PRH_CHECK(ensure(c, c->wt_Wl, N));
-  PRH_CHECK(ensure(c, c->sched_out, N));
+  PRH_CHECK(ensure(c, c->wt_wl, std::max<uint64_t>(1, M)));
   PRH_CHECK(ensure(c, c->tiles, size_t(3) * prh::partition_tiles(N)));
   PRH_CHECK(ensure(c, c->counts, 8));
-  PRH_HIP(c, prh::launch_partition(g->out_off, N, prh::kSumLane, prh::kSumWave, c->sched_out.p, c->tiles.p, c->counts.p,
-                                   hs));
-  PRH_HIP(c, prh::launch_out_weight_sum(g->out_off, *w_out, N, c->sched_out.p, c->counts.p, c->wt_W.p, hs));
+  // The rows by out-degree stand where the weights in layout order come later (M >= N: every row has an edge).
+  uint32_t *order = reinterpret_cast<uint32_t *>(c->wt_wl.p);
+  PRH_HIP(c, prh::launch_partition(g->out_off, N, prh::kSumLane, prh::kSumWave, order, c->tiles.p, c->counts.p, hs));
+  PRH_HIP(c, prh::launch_out_weight_sum(g->out_off, *w_out, N, order, c->counts.p, c->wt_W.p, hs));
   PRH_HIP(c, prh::launch_gather_f64(c->wt_W.p, g->perm, N, c->wt_Wl.p, hs));
-  PRH_CHECK(ensure(c, c->wt_wl, std::max<uint64_t>(1, M)));
   for (int i = 0; i < 2; ++i) {
     PRH_CHECK(ensure(c, c->wt_x[i], N));
     PRH_CHECK(ensure(c, c->wt_z[i], N));
