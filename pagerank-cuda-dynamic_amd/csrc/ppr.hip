@@ -382,7 +382,6 @@ hipError_t launch_tiles(const PprArgs &A, int step, double *out, hipStream_t s) 
     case 8: return launch_pass<8, FINAL>(A, step, out, s);
     case 16: return launch_pass<16, FINAL>(A, step, out, s);
     case 32: return launch_pass<32, FINAL>(A, step, out, s);
-    case 64: return launch_pass<64, FINAL>(A, step, out, s);
     default: return hipErrorInvalidValue;
   }
 }

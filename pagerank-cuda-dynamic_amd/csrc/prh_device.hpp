@@ -56,17 +56,6 @@ __device__ __forceinline__ double group_sum(double x) {
   return x;
 }
 
-template <int W>
-__device__ __forceinline__ double group_max(double x) {
-  if constexpr (W >= 2) x = fmax(x, dpp_move<kDppQuadSwap1>(x));
-  if constexpr (W >= 4) x = fmax(x, dpp_move<kDppQuadSwap2>(x));
-  if constexpr (W >= 8) x = fmax(x, dpp_move<kDppRowHalfMirror>(x));
-  if constexpr (W >= 16) x = fmax(x, dpp_move<kDppRowMirror>(x));
-  if constexpr (W >= 32) x = fmax(x, swizzle_xor16(x));
-  if constexpr (W >= 64) x = fmax(read_lane(x, 0), read_lane(x, 32));
-  return x;
-}
-
 __device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)); }
 
 // Number of set bits of a 64-bit wave mask below this lane.
