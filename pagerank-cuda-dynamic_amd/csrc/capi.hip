@@ -385,11 +385,15 @@ int prh_graph_create(prh_context *c, uint32_t N, uint64_t M, const uint32_t *in_
                   bits & 8 ? " in-id-range" : "", bits & 16 ? " out-id-range" : "", bits & 32 ? " out-offsets" : "");
     }
   }
-  if (st == PRH_SUCCESS)
+  if (st == PRH_SUCCESS) {
+    uint32_t dead = 0, most = 0;
     for (uint32_t v = 0; v < N; ++v) {
-      g->dead_ends += outdeg[v] == 0;
-      g->max_outdeg = std::max(g->max_outdeg, outdeg[v]);
+      dead += outdeg[v] == 0;
+      most = std::max(most, outdeg[v]);
     }
+    g->dead_ends = dead;
+    g->max_outdeg = most;
+  }
   if (st == PRH_SUCCESS) st = build_layout(c, g, in_off, outdeg, out_off != nullptr);
   if (st != PRH_SUCCESS) {
     prh_graph_destroy(g);
