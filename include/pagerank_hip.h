@@ -78,7 +78,9 @@ typedef struct prh_stats {
 } prh_stats;
 
 /* Launch tuning (no counterpart in the reference, whose values are fixed: switch degree 64, 256-thread blocks).
- * Results do not depend on these beyond floating-point summation order. */
+ * Results do not depend on these beyond floating-point summation order. On a graph that fits one workgroup's LDS (about
+ * 2,500 vertices of 16 edges, 3,300 of few; not updated in place) the row plan runs a solve's iterations in one launch
+ * and uses none of switch_degree, huge_degree, low_width, check_interval, block_edges and extension_direction. */
 typedef struct prh_tuning {
   uint32_t switch_degree; /* in-degree <= this: several vertices per wave; above: one wave (long rows: one workgroup)
                              per vertex [64] */
@@ -130,7 +132,9 @@ void prh_default_tuning(prh_tuning *tuning);
 int prh_context_create(int device, prh_context **context);
 void prh_context_destroy(prh_context *context);
 const char *prh_context_last_error(const prh_context *context);
-/* Upper bound on device bytes this context may allocate (graphs + workspace); 0 = unlimited. */
+/* Upper bound on device bytes this context may allocate (graphs + workspace); 0 = unlimited. The weighted solves keep a
+ * map of 4 bytes an edge with each blocked plan they use, which is counted as used; it is given up when an allocation of
+ * the context finds no room. */
 int prh_context_set_memory_limit(prh_context *context, size_t bytes);
 size_t prh_context_memory_used(const prh_context *context);
 int prh_context_set_tuning(prh_context *context, const prh_tuning *tuning);

@@ -248,7 +248,7 @@ __device__ __forceinline__ void add_slots(double *sum, uint8_t *ext, uint32_t d,
 // Weighted variants multiply each slot's value by its edge's weight (P.ws, slot order), loaded with the slot: loaded at the
 // addition it was a round trip of its own (RMAT-20, B = 2048: 42.5 -> 38.3 us forward, 40.5 -> 35.8 us adjoint; three
 // groups in flight take 14.4 ms per forward and backward against 13.3 with two).
-// At most 80 SGPRs: with more, one workgroup of sixteen waves runs per CU instead of two (a wave's SGPRs come in sixteens
+// At most 80 SGPRs (B = 16384 takes up to 92, where the sums in LDS leave room for one workgroup anyway): with more, one workgroup of sixteen waves runs per CU instead of two (a wave's SGPRs come in sixteens
 // out of 800 per SIMD, sixteen of them the system's own: eight waves of 96 do not fit). Per iteration with and without:
 // DF-P on 1.5M vertices (B = 2048, 93 SGPRs before) 46 against 67 us, weighted forward on 1M vertices 39 against 49 us.
 template <int B, int VARIANT>

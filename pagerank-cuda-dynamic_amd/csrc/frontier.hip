@@ -4,16 +4,16 @@
 //                 (pagerankAffectedFrontierPartialCukU, pagerankCuda.hxx:272-281).
 //   extend:       vaff[w] = 1 for every out-neighbour w of a vertex u with naff[u]
 //                 (pagerankAffectedExtend{Thread,Block}CukU + pagerankMarkNeighborsCudU, :55-63, :313-366),
-//                 split by out-degree: 8 lanes per low-out-degree vertex, one wave per high-out-degree vertex.
-//                 With `fresh` set it is one breadth-first level: only newly marked vertices enter `fresh`
-//                 and `changed` records whether any vertex was newly marked (the DT closure, :438-456).
+//                 split by out-degree: 8 lanes per low-out-degree vertex, one wave per high-out-degree vertex or
+//                 chunk of one. With `fresh` set it is one breadth-first level: only newly marked vertices enter
+//                 `fresh` and `changed` records whether any vertex was newly marked (the DT closure, :438-456).
 //   extend_batch  the same marking for the initial extension, whose flagged vertices are exactly the batch's
 //                 sources: driven by the batch list instead of a scan of every vertex, with each source's edges
 //                 cut into chunks of kBatchChunk spread over all the waves (a hub's edges are not left to one).
-//   direction /   the same extension in pull form (the direction-optimizing idea of Beamer et al., SC 2012):
-//   extend_pull   every unaffected row w takes vaff[w] = 1 when an in-neighbour is in the frontier. The rank
-//                 launch leaves per-workgroup costs of both forms (in-edges of unaffected rows, out-edges of
-//                 frontier rows); `direction` totals them and the cheaper form runs. Both give the same flags.
+//   extend_either the extension after a rank launch, pushed as above or in pull form (the direction-optimizing idea
+//                 of Beamer et al., SC 2012): every unaffected row w takes vaff[w] = 1 when an in-neighbour is in
+//                 the frontier. The rank launch leaves sums of what both forms would cost (in-edges of unaffected
+//                 rows, out-edges of frontier rows), and the cheaper form runs. Both give the same flags.
 // Concurrent writers only ever store 1, so the flags are the same for any interleaving.
 #include "prh_device.hpp"
 #include "prh_internal.hpp"

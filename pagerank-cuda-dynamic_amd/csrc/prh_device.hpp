@@ -90,10 +90,11 @@ __device__ __forceinline__ void tell_host(int *p, int v) {
 }
 
 // Entry test for the first kernel of iteration l; all threads of a block agree.
-// done and err[l-1] were last written by earlier launches, whose completion made them visible: plain loads (both
-// issued together) suffice. A volatile read here would be a system-scope load at the start of every wave.
+// done and err[l-1] were last written by earlier launches, whose completion made them visible: plain loads suffice. A
+// volatile read here would be a system-scope load at the start of every wave.
 // The test needs two loads; a workgroup's item can be loaded with them instead of after the test. `broken`, never true, is
-// a condition on the item: it keeps the compiler from moving the item's load behind the test. (An empty asm statement in its
+// a condition on the item: it keeps the compiler from moving the item's load behind the test. (The kernels that pass none
+// wait for done before they load err[l-1].) (An empty asm statement in its
 // place made the later uniform loads vector loads: RMAT-20, blocked, 3.60 -> 4.17 ms per solve.) Blocked plan, per solve,
 // test first -> together, and accumulate's first batch before its sums are cleared: RMAT-20 3.59 -> 3.46 ms, RMAT-24
 // 40.6 -> 40.4, weighted forward and backward on RMAT-20 9.79 -> 9.48.

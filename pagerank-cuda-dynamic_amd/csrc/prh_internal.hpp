@@ -536,7 +536,6 @@ hipError_t launch_copy_u8(uint8_t *dst, const uint8_t *src, size_t n, hipStream_
 // ---- frontier.hip ----
 hipError_t launch_mark_partial(uint8_t *naff, uint8_t *vaff, const uint32_t *delu, const uint32_t *delv,
                                size_t ND, const uint32_t *insu, size_t NI, hipStream_t s);
-// Extension; when err/done are non-null the kernel honours the iteration control of iteration l.
 // Initial extension from the batch list: vaff[w] = 1 for every out-neighbour w of every batch source (deletion
 // sources delu, insertion sources insu), each source once: naff (1 for the sources, from mark_partial; its
 // allocation a multiple of 4 bytes) is set to 2 for a source when an entry claims it. cnt and start hold ND + NI + 1
@@ -550,6 +549,7 @@ hipError_t launch_extend_batch_keys(uint8_t *vaff, uint8_t *naff, const unsigned
                                     const unsigned long long *ik, const uint32_t *ni, uint32_t cap,
                                     const uint32_t *off, const uint32_t *dst, uint32_t *cnt, uint32_t *start,
                                     void *tmp, size_t &tmp_bytes, hipStream_t s);
+// One push of the flagged vertices' out-edges (a traversal level).
 hipError_t launch_extend(const ExtendArgs &A, hipStream_t s);
 // The extension after iteration ctl.l's rank launch: mode 0 push, 2 pull, 1 the cheaper by the costs that launch added to
 // `stats` (kCostSums doubles); next_stats, the next iteration's, is cleared.
