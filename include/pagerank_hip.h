@@ -128,7 +128,7 @@ void prh_default_tuning(prh_tuning *tuning);
 /* Context: device, stream and reusable device workspace. Replaces the per-call cudaSetDeviceFlags and
  * cudaMalloc/cudaFree of pagerankInvokeCuda (pagerankCuda.hxx:777-796, :829-847). The environment variable
  * PRH_GRAPH_CAPTURE=0 at creation makes the context issue the launches it would replay from captured HIP graphs
- * (batched PPR, the streaming session) one by one. */
+ * (batched PPR, the streaming session) one by one; so does any context while another thread is inside a call. */
 int prh_context_create(int device, prh_context **context);
 void prh_context_destroy(prh_context *context);
 const char *prh_context_last_error(const prh_context *context);

@@ -340,6 +340,7 @@ using namespace prhc;
 extern "C" {
 
 int prh_graph_csr(prh_context *c, const prh_graph *g, int which, uint32_t *offsets, uint32_t *ids) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (!g || g->ctx != c || !offsets || (g->M && !ids) || (which != 0 && which != 1))
     return fail(c, PRH_ERROR_INVALID_ARGUMENT, "null or foreign graph, null array or bad CSR selector");
@@ -357,6 +358,7 @@ int prh_graph_csr(prh_context *c, const prh_graph *g, int which, uint32_t *offse
 
 int prh_graph_update(prh_context *c, prh_graph *g, const uint32_t *del_u, const uint32_t *del_v, size_t nd,
                      const uint32_t *ins_u, const uint32_t *ins_v, size_t ni, float *update_ms) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (update_ms) *update_ms = 0.0f;
   if (!g || g->ctx != c) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "null or foreign graph");

@@ -142,6 +142,7 @@ extern "C" {
 
 int prh_autotune(prh_context *c, const prh_graph *g, const char *cache_path, int iterations, prh_tuning *chosen,
                  double *ms_per_iteration, int *from_cache) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (!g || g->ctx != c || iterations < 1) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "bad graph or iterations");
   if (from_cache) *from_cache = 0;

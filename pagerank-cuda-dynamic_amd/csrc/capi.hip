@@ -210,6 +210,7 @@ void prh_default_tuning(prh_tuning *t) {
 }
 
 int prh_context_create(int device, prh_context **out) {
+  const Call call;
   if (!out) return PRH_ERROR_INVALID_ARGUMENT;
   *out = nullptr;
   int count = 0;
@@ -243,6 +244,7 @@ int prh_context_create(int device, prh_context **out) {
 }
 
 void prh_context_destroy(prh_context *c) {
+  const Call call;
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (int i = 0; i < 2; ++i) {
@@ -342,6 +344,7 @@ void *prh_context_stream(prh_context *c) { return c ? reinterpret_cast<void *>(c
 
 int prh_graph_create(prh_context *c, uint32_t N, uint64_t M, const uint32_t *in_off, const uint32_t *in_src,
                      const uint32_t *outdeg, const uint32_t *out_off, const uint32_t *out_dst, prh_graph **out) {
+  const Call call;
   if (!c || !out) return PRH_ERROR_INVALID_ARGUMENT;
   *out = nullptr;
   if (M >= (uint64_t(1) << 32)) return fail(c, PRH_ERROR_INVALID_GRAPH, "M = %llu does not fit uint32 offsets", (unsigned long long)M);
@@ -404,6 +407,7 @@ int prh_graph_create(prh_context *c, uint32_t N, uint64_t M, const uint32_t *in_
 }
 
 void prh_graph_destroy(prh_graph *g) {
+  const Call call;
   if (!g) return;
   prh_context *c = g->ctx;
   if (c && c->stream) (void)hipStreamSynchronize(c->stream);
@@ -445,6 +449,7 @@ uint64_t prh_graph_size(const prh_graph *g) { return g ? g->M : 0; }
 int prh_solve(prh_context *c, const prh_graph *g, prh_method method, int partition, const prh_options *o,
               const uint32_t *du, const uint32_t *dv, size_t nd, const uint32_t *iu, size_t ni, const double *q,
               double *ranks, prh_stats *st) {
+  const Call call;
   (void)partition;
   return solve_impl(c, g, method, o, du, dv, nd, iu, ni, q, ranks, st, true, true);
 }
@@ -452,11 +457,13 @@ int prh_solve(prh_context *c, const prh_graph *g, prh_method method, int partiti
 int prh_solve_device(prh_context *c, const prh_graph *g, prh_method method, int partition, const prh_options *o,
                      const uint32_t *du, const uint32_t *dv, size_t nd, const uint32_t *iu, size_t ni,
                      const double *q, double *ranks, prh_stats *st) {
+  const Call call;
   (void)partition;
   return solve_impl(c, g, method, o, du, dv, nd, iu, ni, q, ranks, st, false, true);
 }
 
 int prh_partition(prh_context *c, uint32_t N, const uint32_t *off, uint32_t d, uint32_t *order, uint32_t *np) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (N == 0) {
     if (np) *np = 0;
@@ -480,6 +487,7 @@ int prh_partition(prh_context *c, uint32_t N, const uint32_t *off, uint32_t d, u
 
 int prh_mark_affected(prh_context *c, const prh_graph *g, prh_method method, const uint32_t *du, const uint32_t *dv,
                       size_t nd, const uint32_t *iu, size_t ni, uint8_t *affected) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (!g || !affected || method < PRH_DYNAMIC_TRAVERSAL || method > PRH_PRUNE_DYNAMIC_FRONTIER)
     return fail(c, PRH_ERROR_INVALID_ARGUMENT, "null argument or non-dynamic method");

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/pagerank_hip.h"
+#include "gate.hpp"
 #include "prh_internal.hpp"
 
 namespace prhc {
@@ -287,9 +288,14 @@ inline uint32_t layout_rows_above(const prh_graph *g, uint32_t x) {
   return g->layout == 0 ? rows_above(g->sorted_deg, x) : 0u;
 }
 
-// Capture `body` (launches on the context stream only) into an executable graph.
+// Capture `body` (launches on the context stream only) into an executable graph. *exec stays null, and the caller issues
+// the launches one by one, while another thread is inside the engine (gate.hpp).
 template <class F>
 int capture_graph(prh_context *c, F body, hipGraphExec_t *exec) {
+  if (!gate().begin_capture()) return PRH_SUCCESS;
+  struct End {
+    ~End() { gate().end_capture(); }
+  } end;
   hipGraph_t graph = nullptr;
   PRH_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   const int st = body();
@@ -303,6 +309,9 @@ int capture_graph(prh_context *c, F body, hipGraphExec_t *exec) {
   if (ie != hipSuccess) return fail(c, PRH_ERROR_DEVICE, "hipGraphInstantiate: %s", hipGetErrorString(ie));
   return PRH_SUCCESS;
 }
+
+// Whether a captured graph is there and may be replayed.
+inline bool replayable(hipGraphExec_t exec) { return exec && gate().alone(); }
 
 // Batch arrays staged in the context (host or device source), checked against N and mapped to layout ids.
 struct DevBatch {

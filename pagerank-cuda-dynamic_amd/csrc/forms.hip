@@ -142,7 +142,7 @@ int ppr_impl(prh_context *c, const prh_graph *g, int k, const uint32_t *so, cons
   // A run is launched when the one before it has begun its last iteration, so that the device goes on without waiting.
   reset_progress(c);
   for (int launched = 0; status == PRH_SUCCESS && launched < L && !loop_stopped(c); launched += chunk) {
-    if (!replay.exec) status = iterations_chunk();
+    if (!replayable(replay.exec)) status = iterations_chunk();
     else if (const hipError_t e = hipGraphLaunch(replay.exec, s); e != hipSuccess)
       status = fail(c, PRH_ERROR_DEVICE, "batched iterations: %s", hipGetErrorString(e));
     if (status == PRH_SUCCESS) status = wait_progress(c, std::min(L, launched + chunk));
@@ -543,6 +543,7 @@ extern "C" {
 
 int prh_weighted_pagerank(prh_context *c, const prh_graph *g, const float *w, const double *s, const prh_options *o,
                           double *ranks, prh_stats *st, int device_pointers) {
+  const Call call;
   if (c && g && g->N == 0) {
     if (st) *st = prh_stats{};
     return PRH_SUCCESS;
@@ -553,6 +554,7 @@ int prh_weighted_pagerank(prh_context *c, const prh_graph *g, const float *w, co
 int prh_weighted_adjoint(prh_context *c, const prh_graph *g, const float *w, const double *r, const double *gr,
                          const prh_options *o, double *lam, double *grad_w, double *grad_s, prh_stats *st,
                          int device_pointers) {
+  const Call call;
   if (c && g && g->N == 0) {
     if (st) *st = prh_stats{};
     return PRH_SUCCESS;
@@ -562,6 +564,7 @@ int prh_weighted_adjoint(prh_context *c, const prh_graph *g, const float *w, con
 
 int prh_ppr_batched(prh_context *c, const prh_graph *g, int k, const uint32_t *so, const uint32_t *seeds,
                     const prh_options *o, double *ranks, int *iterations, prh_stats *st) {
+  const Call call;
   if (c && g && g->N == 0) {
     if (st) *st = prh_stats{};
     if (iterations)

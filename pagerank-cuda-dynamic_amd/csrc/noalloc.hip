@@ -74,6 +74,7 @@ extern "C" {
 
 int prh_partition_noalloc(prh_context *c, uint32_t n, const uint32_t *offsets, uint32_t switch_degree,
                           uint32_t *order, uint32_t *partition_point) {
+  const Call call;
   if (!c) return PRH_ERROR_INVALID_ARGUMENT;
   if (!partition_point || (n && (!offsets || !order))) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "null argument");
   if (n > kNoAllocMaxVertices)

@@ -274,6 +274,7 @@ extern "C" {
 
 int prh_stream_create(prh_context *c, const prh_graph *g, prh_method method, const prh_options *options,
                       uint32_t max_batch, uint64_t max_edges, const double *initial_ranks, prh_stream **out) {
+  const Call call;
   if (!c || !out) return PRH_ERROR_INVALID_ARGUMENT;
   *out = nullptr;
   if (!g || !options || g->ctx != c) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "null graph/options or foreign graph");
@@ -506,6 +507,7 @@ int prh_stream_create(prh_context *c, const prh_graph *g, prh_method method, con
 
 int prh_stream_update(prh_stream *S, const uint32_t *del_u, const uint32_t *del_v, size_t nd, const uint32_t *ins_u,
                       const uint32_t *ins_v, size_t ni, double *ranks, prh_stats *stats) {
+  const Call call;
   if (!S) return PRH_ERROR_INVALID_ARGUMENT;
   prh_context *c = S->ctx;
   if (S->broken) return fail(c, PRH_ERROR_INVALID_ARGUMENT, "stream is unusable after an earlier failed update");
@@ -534,12 +536,10 @@ int prh_stream_update(prh_stream *S, const uint32_t *del_u, const uint32_t *del_
   PRH_HIP(c, hipEventRecord(c->ev[0], s));
   PRH_HIP(c, hipMemcpyAsync(S->d_batch, h, (4 * size_t(cap) + 2) * 4, hipMemcpyHostToDevice, s));
   const int p = S->cur, q = 1 - p;
-  if (c->capture) {
-    if (!S->apply[p]) PRH_CHECK(capture_graph(c, [&]() { return stream_apply_body(S, p); }, &S->apply[p]));
-    PRH_HIP(c, hipGraphLaunch(S->apply[p], s));
-  } else {
-    PRH_CHECK(stream_apply_body(S, p));
-  }
+  if (c->capture && !S->apply[p])
+    PRH_CHECK(capture_graph(c, [&]() { return stream_apply_body(S, p); }, &S->apply[p]));
+  if (replayable(S->apply[p])) PRH_HIP(c, hipGraphLaunch(S->apply[p], s));
+  else PRH_CHECK(stream_apply_body(S, p));
   PRH_HIP(c, hipEventRecord(c->ev[1], s));
   PRH_HIP(c, hipMemcpyAsync(c->pinned, S->ctl + 3, 4, hipMemcpyDeviceToHost, s));
   PRH_HIP(c, hipMemcpyAsync(c->pinned + 1, S->in_off[q] + S->N, 4, hipMemcpyDeviceToHost, s));
@@ -558,7 +558,7 @@ int prh_stream_update(prh_stream *S, const uint32_t *del_u, const uint32_t *del_
       PRH_CHECK(capture_graph(c, [&]() { return stream_closure_body(S, q); }, &S->closure[q]));
     int stop = 0;
     for (uint64_t lv = 0; !stop && lv <= uint64_t(S->N) + kClosureLevels; lv += kClosureLevels) {
-      if (c->capture) PRH_HIP(c, hipGraphLaunch(S->closure[q], s));
+      if (replayable(S->closure[q])) PRH_HIP(c, hipGraphLaunch(S->closure[q], s));
       else PRH_CHECK(stream_closure_body(S, q));
       PRH_HIP(c, hipMemcpyAsync(c->pinned, S->lvl + 1, 4, hipMemcpyDeviceToHost, s));
       PRH_HIP(c, hipStreamSynchronize(s));
@@ -572,7 +572,7 @@ int prh_stream_update(prh_stream *S, const uint32_t *del_u, const uint32_t *del_
   // to the next without waiting for the host.
   reset_progress(c);
   for (int launched = 0; launched < S->opt.max_iterations && !loop_stopped(c); launched += kStreamChunk) {
-    if (c->capture) PRH_HIP(c, hipGraphLaunch(S->iter[q], s));
+    if (replayable(S->iter[q])) PRH_HIP(c, hipGraphLaunch(S->iter[q], s));
     else PRH_CHECK(stream_iter_body(S, q));
     PRH_CHECK(wait_progress(c, launched + kStreamChunk - 1));
   }
@@ -601,6 +601,7 @@ int prh_stream_update(prh_stream *S, const uint32_t *del_u, const uint32_t *del_
 }
 
 int prh_stream_ranks(prh_stream *S, double *ranks) {
+  const Call call;
   if (!S || !ranks) return S ? fail(S->ctx, PRH_ERROR_INVALID_ARGUMENT, "null ranks") : PRH_ERROR_INVALID_ARGUMENT;
   prh_context *c = S->ctx;
   PRH_CHECK(ensure(c, c->contrib[0], S->N));
@@ -613,6 +614,7 @@ int prh_stream_ranks(prh_stream *S, double *ranks) {
 uint64_t prh_stream_size(const prh_stream *S) { return S ? S->M : 0; }
 
 int prh_stream_csr(prh_stream *S, int which, uint32_t *offsets, uint32_t *ids) {
+  const Call call;
   if (!S) return PRH_ERROR_INVALID_ARGUMENT;
   prh_context *c = S->ctx;
   if (!offsets || (S->M && !ids) || (which != 0 && which != 1))
@@ -625,6 +627,7 @@ int prh_stream_csr(prh_stream *S, int which, uint32_t *offsets, uint32_t *ids) {
 }
 
 void prh_stream_destroy(prh_stream *S) {
+  const Call call;
   if (!S) return;
   (void)hipSetDevice(S->ctx->device);
   (void)hipStreamSynchronize(S->ctx->stream);
